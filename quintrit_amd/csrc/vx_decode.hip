@@ -1071,10 +1071,6 @@ struct AttnArgs {
     uint32_t n_heads, gqa, max_ctx;
     uint32_t rope_normal;  // 1: pairs (2i, 2i + 1) (RopeMode::Normal), 0: (i, i + head_dim / 2) (NEOX)
     float scale;
-    // prefill: n_tok tokens at positions ctl->pos + 1 - n_tok .. ctl->pos, their rotated f16 queries in
-    // qbuf[token][n_heads * head_dim] and their k, v already in the cache; out is [token][n_heads * head_dim]
-    const uint16_t* qbuf;
-    uint32_t n_tok;
     // decode in two kernels: the scores [n_heads][max_ctx], then per chunk its f16 accumulators cy [n_heads][4][HD]
     // (one per word), its (max, sum) pairs cms [n_heads][slices][4][2] and a ticket per (head, slice) (0 between steps)
     float* scores;
@@ -1083,14 +1079,9 @@ struct AttnArgs {
     uint32_t* ticket;
 };
 
-constexpr uint32_t kAttnMaxCtx = 8192;  // KV positions held in LDS (scores, running maxima)
-constexpr uint32_t kVDepth = 8;         // groups of 8 positions of V in flight per lane in the accumulator chain
+constexpr uint32_t kAttnMaxCtx = 8192;  // KV positions of a context at most
 // Positions per row of the transposed V cache: max_ctx rounded up to 8 (one 16-byte load is 8 positions).
 inline uint32_t vstride_of(uint32_t max_ctx) { return (max_ctx + 7u) / 8u * 8u; }
-// The attention kernel's shape for a head dimension: coordinates per lane, waves (4 chunks of attn_waves / 4), threads.
-__host__ __device__ constexpr uint32_t attn_cpl(uint32_t hd) { return hd >= 256u ? hd / 128u : 1u; }
-__host__ __device__ constexpr uint32_t attn_waves(uint32_t hd) { return hd >= 128u ? 8u : 4u; }
-__host__ __device__ constexpr uint32_t attn_threads(uint32_t hd) { return 64u * attn_waves(hd); }
 
 // f16 value of an f32 (round to nearest even, after the f32 rounding of x), kept in an f32
 __device__ __forceinline__ float r16(float x) { return static_cast<float>(static_cast<_Float16>(keep_f32(x))); }
@@ -1112,375 +1103,466 @@ __device__ __forceinline__ void r16_all(float (&y)[N]) {
     if constexpr (N % 2 == 1) y[N - 1] = r16(y[N - 1]);
 }
 
-// One workgroup per query head (and token, PREFILL). First the inputs of the position: q of this head and k, v of its KV
-// head, RoPE over all head_dim coordinates (ops.rs:199-221, NEOX or Normal pairing: x0' = fma(x0, c, -(x1 s)),
-// x1' = fma(x0, s, x1 c)) and the f16 rounding of the cache (kv_cache.rs:24-182); the first query head of each KV head
-// appends k and v to the cache, and every workgroup uses its own copy of them for the position itself (the other
-// positions come from earlier steps). PREFILL: the query comes rotated from qbuf and the position's k and v from the
-// cache (pf_rope_kernel wrote them), nothing is appended.
-// Then the reference's attend_head (attention.rs:483-542) over the positions 0..pos. Below a padded KV length of 512 one
-// online softmax covers all positions; from 512 on, 4 chunks of ceil(n_kv / 4) positions run one each and are combined
-// in order. The online softmax of a chunk (attend_range, attention.rs:436-468) is rebuilt without its serial
-// dependences except the FP16 accumulator itself:
-//   scores        every position in parallel (four lanes each): ggml_vec_dot_f16(q, k) * scale
-//   running max   a scan per chunk; the reference's max moves only on score > max, the scan combines the same way
-//   factors       every position in parallel: a new maximum gives ms = expf(m_old - score), vs = 1; otherwise ms = 1,
-//                 vs = expf(score - max); stored as -ms or vs (the sign marks the case)
-//   accumulator   per coordinate, in position order: y = f16(y * ms), y = f16(fma(v, vs, y)), s = fma(s, ms, vs)
-// The accumulator chains: each chunk has attn_waves(HD) / 4 waves, a lane attn_cpl(HD) coordinates (independent
-// chains). V is cached in tiles of 8 positions, [kv_head][position / 8][coordinate][position % 8]: one 16-byte load is
-// eight consecutive positions of one coordinate, and a wave's load of 64 coordinates reads 1 KiB of contiguous memory;
-// kVDepth such loads per coordinate are in flight ahead of the chain.
-template <int HD, bool PREFILL>
-__global__ __launch_bounds__(attn_threads(HD)) void attention_kernel(AttnArgs a) {
-    constexpr uint32_t kCpl = attn_cpl(HD);           // coordinates (chains) per lane
-    constexpr uint32_t kWpc = attn_waves(HD) / 4u;    // waves per chunk
-    constexpr uint32_t kLanes = HD / (kWpc * kCpl);   // lanes of a wave with coordinates (64, or 32 at head_dim 32)
-    constexpr uint32_t kThreads = attn_threads(HD);
-    constexpr uint32_t kHalf = HD / 2;        // RoPE pairs
-    constexpr int kBlk = HD / 32;             // 32-value blocks of a row
-    __shared__ __align__(16) float sc[kAttnMaxCtx];
-    __shared__ float pm[kAttnMaxCtx];
-    __shared__ __align__(16) uint16_t qs[HD];
-    __shared__ __align__(16) uint16_t kp[HD];  // k and v of the position itself
-    __shared__ __align__(16) uint16_t vp[HD];
-    __shared__ float cm[4], cs[4];
-    __shared__ uint16_t cv[4][HD];
-    const uint32_t h = blockIdx.x, tid = threadIdx.x, lane = tid & 63u;
+// ---- prefill attention -----------------------------------------------------------------------------------------------------
+//
+// The reference's attend_head (attention.rs:483-542) for many tokens at once: below a padded KV length of 512 one online
+// softmax covers the positions 0..pos of a token, from 512 on 4 chunks of ceil(n_kv / 4) positions run one each and are
+// combined in order. A chunk's online softmax (attend_range, attention.rs:436-468) is rebuilt without its serial
+// dependences except the FP16 accumulator itself: the scores of all positions, the running maximum as a scan (it moves
+// only on score > max, so NaN never moves it), the factors (a new maximum gives ms = expf(m_old - score), vs = 1;
+// otherwise ms = 1, vs = expf(score - max); held as -ms or vs, the sign marks the case), then per coordinate, in
+// position order, y = f16(y ms), y = f16(fma(v, vs, y)), and s = fma(s, ms, vs).
+//
+// Work split: a workgroup takes one query head, one chunk and TOK tokens at consecutive positions from a multiple of
+// TOK on (they share the padded length, so the chunk's bounds), and walks the chunk in ranges of POS positions per wave.
+// In a range wave w first computes the scores and factors of its POS positions for all tokens, and then runs the
+// accumulators of its own tokens over the whole range, a lane holding some coordinates of each: the V words of 8
+// positions are loaded once for all of them, the factors are read from LDS (one address per wave). TOK = 16 with 4
+// waves of 16 positions measured 10.6 ms of a 1500-token prompt (30 layers of 20 heads of 128; 32 tokens with 8 waves
+// of 16 or 32 positions 12.1 and 13.1 ms) and 24.0 ms of a 3900-token one (10 layers of 12 heads of 256; 27.6, 27.3).
+// One workgroup per (head, token) with every phase on the vector unit took 30.8 and 45.4 ms.
+//
+// Scores on the matrix cores. ggml_vec_dot_f16 (ops.rs:960-1015) sums 32 chains: accumulator j (0..3), lane l (0..7)
+// takes the values 32 i + 8 j + l of every 32-value block i, one fused multiply-add each in increasing i; then
+// (a0 + a2) + (a1 + a3), red[l] + red[l + 4], (t0 + t1) + (t2 + t3). v_mfma_f32_16x16x1 (K = 1, four 16 x 16 blocks)
+// adds one product to every element with a single rounding, so it is that fused multiply-add (bit for bit, Inf and NaN
+// included: compared with fmaf over 0.26 M chains of random normal and random-bit operands): A is the chain's value of
+// 16 positions, B of 16 tokens, block j the accumulator. It does twice the multiply-adds of the vector unit per cycle
+// and leaves that free for the accumulators. D's lane l holds token l % 16 and positions 4 (l / 16) + e in registers
+// 4 j + e, so the running maximum and the exponentials are computed in registers (the quarters of a wave exchange the
+// maxima of their 4 positions) and only the factors go to LDS.
+//
+// What bounds it: the vector unit (65 % busy), 1.5 instructions per coordinate and position for the accumulators (a
+// fused multiply-add and half a packed conversion; at head_dim 128 3.3 of the 6.6 per score and wave), the sums of the
+// chains and the exponentials.
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+struct PfAttnArgs {
+    const Ctl* ctl;
+    const uint16_t* kc;    // this layer: [kv_head][max_ctx][head_dim] f16
+    const uint16_t* vc;    // this layer: [kv_head][vstride / 8][head_dim][8] f16
+    const uint16_t* qbuf;  // [n_tok][n_heads * head_dim] rotated f16 queries of positions ctl->pos + 1 - n_tok ..
+    float* out;            // [n_tok][n_heads * head_dim]
+    uint16_t* cy;          // [n_tok][n_heads][4][head_dim] f16 accumulators of the chunks of a split context
+    float* cms;            // [n_tok][n_heads][4][2] their maxima and sums
+    uint32_t vstride, n_heads, gqa, max_ctx, n_tok;
+    float scale;
+};
+
+// The padded KV length of a context of seq positions, and its chunks (attention.rs:483-510).
+struct KvSplit {
+    uint32_t n_kv, chunk, n_chunks;
+};
+__device__ __forceinline__ KvSplit kv_split(uint32_t seq, uint32_t max_ctx) {
+    KvSplit k;
+    k.n_kv = min((seq + 255u) / 256u * 256u, max_ctx);
+    const bool split = k.n_kv >= 512u;
+    k.chunk = split ? (k.n_kv + 3u) / 4u : k.n_kv;
+    k.n_chunks = split ? 4u : 1u;
+    return k;
+}
+
+// x of lanes l % 16, + 16, + 32 and + 48 in every lane.
+__device__ __forceinline__ void all_quarters(float x, float (&q)[4]) {
+    const auto r = __builtin_amdgcn_permlane32_swap(f32_bits(x), f32_bits(x), false, false);  // quarters 0, 1 and 2, 3
+    const auto lo = __builtin_amdgcn_permlane16_swap(r[0], r[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(r[1], r[1], false, false);
+    q[0] = bits_f32(lo[0]);
+    q[1] = bits_f32(lo[1]);
+    q[2] = bits_f32(hi[0]);
+    q[3] = bits_f32(hi[1]);
+}
+
+// expf of a value that is not positive (or NaN): glibc's, without the range checks that such a value cannot need.
+template <typename Tab>
+__device__ __forceinline__ float expf_nonpos(float x, Tab tab) {
+    const float y = glibc_expf_core(x, tab);
+    return x < -0x1.9fe368p6f ? 0.0f : y;  // underflow (and -inf)
+}
+
+// TOK tokens (16 or 32) per workgroup of W waves, POS positions (16 or 32) per wave and range; SL workgroups share the
+// coordinates of a head, each computing the scores and factors for itself.
+template <int HD, int TOK, int POS, int W, int SL>
+__global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel(PfAttnArgs a) {
+    constexpr uint32_t kCpl = HD >= 64 ? HD / (64u * SL) : 1u;  // coordinates per lane
+    constexpr uint32_t kOwn = TOK / W;                          // tokens per wave
+    constexpr uint32_t kTh = TOK / 16u, kPh = POS / 16u;        // 16-token and 16-position halves of a wave's scores
+    constexpr uint32_t kRange = W * POS;
+    constexpr uint32_t kRing = SL > 1 || kCpl == 1u ? 8u : 4u;  // V groups of 8 positions in flight
+    constexpr int kBlk = HD / 32;
+    constexpr uint32_t kQRow = HD + 8u;                         // halves per token row in LDS
+    static_assert(kRange % (8u * kRing) == 0 && (kOwn == 2u || kOwn == 4u), "whole rings in a range, 2 or 4 tokens per wave");
+    __shared__ __align__(16) float fac[TOK][kRange + 4u];       // (the rows start on different banks)
+    __shared__ __align__(16) uint16_t qs[TOK][kQRow];
+    __shared__ float wmax[W][TOK];
+    // byte [g][t]: token t has a new maximum among the first (bit 0), the last (bit 1) 4 positions of group g
+    __shared__ __align__(4) uint8_t newmax[kRange / 8u][TOK];
+    __shared__ uint64_t etab[32];
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t kvh = h / a.gqa;
-    const uint32_t tok = PREFILL ? blockIdx.y : 0u;
-    const uint32_t pos = PREFILL ? a.ctl->pos + 1u - a.n_tok + tok : a.ctl->pos;
-    const uint32_t seq = pos + 1;
+    const uint32_t h = blockIdx.x / SL, kvh = h / a.gqa, c = blockIdx.z;
+    const uint32_t last = a.ctl->pos, first = last + 1u - a.n_tok;  // the pass' positions
+    // later tokens first: they have the most positions
+    const uint32_t tp = (first / TOK + (gridDim.y - 1u - blockIdx.y)) * TOK;
+    if (tp > last) return;
+    const KvSplit kv = kv_split(tp + 1u, a.max_ctx);
+    if (c >= kv.n_chunks) return;
+    const uint32_t st = c * kv.chunk;
+    const uint32_t t_last = min(tp + TOK - 1u, last);                        // the tile's last token
+    const uint32_t en_max = min(min(st + kv.chunk, kv.n_kv), t_last + 1u);   // positions of the longest one
+    if (st >= en_max) return;
     const uint16_t* kb = a.kc + static_cast<size_t>(kvh) * a.max_ctx * HD;
-    uint16_t* vt = a.vc + static_cast<size_t>(kvh) * HD * a.vstride;  // this KV head's tiles: [vstride / 8][HD][8]
-    auto vt_at = [&](uint32_t p, uint32_t dd) -> size_t {
-        return (static_cast<size_t>(p >> 3) * HD + dd) * 8u + (p & 7u);
-    };
+    const uint16_t* vt = a.vc + static_cast<size_t>(kvh) * HD * a.vstride;
+    const size_t qd = static_cast<size_t>(a.n_heads) * HD;
 
-    uint32_t n_kv = (seq + 255u) / 256u * 256u;
-    if (n_kv > a.max_ctx) n_kv = a.max_ctx;
-    const bool split = n_kv >= 512u;
-    const uint32_t chunk = split ? (n_kv + 3u) / 4u : seq;
-    const uint32_t n_chunks = split ? 4u : 1u;
-    // This wave's chunk; the lane's coordinates are d0 + 64 m (m < kCpl) when it has any.
-    const uint32_t c = wave / kWpc;
-    const uint32_t d0 = (wave % kWpc) * 64u * kCpl + lane;
-    const bool has_d = lane < kLanes;
-    uint32_t st = 0, en = 0;
-    if (c < n_chunks) {
-        st = c * chunk;
-        en = min(min(st + chunk, n_kv), seq);
+    for (uint32_t i = tid; i < TOK * HD / 8u; i += 64u * W) {
+        const uint32_t t = i / (HD / 8u), d = i % (HD / 8u) * 8u;
+        const uint32_t p = min(max(tp + t, first), last);  // a token outside the pass repeats one of it (never stored)
+        *reinterpret_cast<uint4*>(&qs[t][d]) = *reinterpret_cast<const uint4*>(a.qbuf + (p - first) * qd + h * HD + d);
     }
-
-    if (PREFILL) {
-        if (tid < HD) {
-            qs[tid] = a.qbuf[(static_cast<size_t>(tok) * a.n_heads + h) * HD + tid];
-            kp[tid] = kb[static_cast<size_t>(pos) * HD + tid];
-            vp[tid] = vt[vt_at(pos, tid)];
-        }
-    } else {
-        const float* cache = a.rope + static_cast<size_t>(pos) * HD;
-        if (tid < HD) {  // q (tid < HD / 2) or k: the rotation of pair i
-            const bool isq = tid < kHalf;
-            const uint32_t i = tid & (kHalf - 1u);
-            const uint32_t i0 = a.rope_normal ? 2u * i : i, i1 = a.rope_normal ? 2u * i + 1u : i + kHalf;
-            const ProjOut& o = isq ? a.q : a.k;
-            const uint32_t base = (isq ? h : kvh) * HD;
-            bool zero;
-            const float post = proj_post(o, &zero);
-            const float x0 = proj_at(o, base + i0, post, zero), x1 = proj_at(o, base + i1, post, zero);
-            const float cc = cache[2 * i], ss = cache[2 * i + 1];
-            const float x1s = x1 * ss, x1c = x1 * cc;
-            const float y0 = __builtin_fmaf(x0, cc, -x1s);
-            const float y1 = __builtin_fmaf(x0, ss, x1c);
-            uint16_t* dst = isq ? qs : kp;
-            dst[i0] = f32_f16(y0);
-            dst[i1] = f32_f16(y1);
-        } else if (tid < 2u * HD) {
-            const uint32_t dd = tid - HD;
-            bool zero;
-            const float post = proj_post(a.v, &zero);
-            vp[dd] = f32_f16(proj_at(a.v, kvh * HD + dd, post, zero));
-        }
-    }
+    if (tid < 32u) etab[tid] = expf_tab(tid);
+    const auto tab = [&](uint32_t k) { return etab[k]; };
     __syncthreads();
-    if (!PREFILL && h % a.gqa == 0 && tid < HD) {
-        a.kc[(static_cast<size_t>(kvh) * a.max_ctx + pos) * HD + tid] = kp[tid];
-        vt[vt_at(pos, tid)] = vp[tid];
+
+    // Scores: this lane's tokens (columns cl and cl + 16) and quarter (the positions 4 qt .. + 3 of each 16).
+    const uint32_t cl = lane & 15u, qt = lane >> 4;
+    uint32_t en[kTh];     // the tokens' positions [st, en)
+    float carry[kTh];     // their running maxima
+#pragma unroll
+    for (uint32_t th = 0; th < kTh; ++th) {
+        const uint32_t p = tp + 16u * th + cl;
+        en[th] = p >= first && p <= last ? min(en_max, p + 1u) : st;
+        carry[th] = -__builtin_inff();
     }
 
-    // The chain's V: group g holds positions 8 g .. 8 g + 7 (every tile read is below vstride: groups run to the chunk's
-    // end rounded up to 8). Its first kVDepth groups are requested once the scores are done, so that they arrive during
-    // the scan and the exponentials without adding to the scores' registers. The value of the position itself, not yet
-    // visible in the cache to every workgroup, is patched from vp when its group is used.
-    const bool chain = c < n_chunks && st < en;
-    const uint32_t g_first = st / 8u, g_end = chain ? (en + 7u) / 8u : g_first + 1u;
-    const uint32_t dl = has_d ? d0 : 0u;  // a lane without coordinates reads coordinate 0 and never uses it
-    u32x4 ring[kVDepth][kCpl];
-    auto load_group = [&](uint32_t g, u32x4 (&r)[kCpl]) {
-        const uint32_t gg = min(g, g_end - 1u);
+    // Accumulators: the wave's tokens t0 .., the lane's coordinates dl + 64 m of each.
+    const uint32_t t0 = wave * kOwn;
+    uint32_t own_en[kOwn], own_max = 0, own_min = ~0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kOwn; ++k) {
+        const uint32_t p = tp + t0 + k;
+        own_en[k] = p >= first && p <= last ? min(en_max, p + 1u) : st;
+        own_max = max(own_max, own_en[k]);
+        own_min = min(own_min, own_en[k]);
+    }
+    const bool has_d = HD >= 64 || lane < HD;
+    const uint32_t dl = (has_d ? lane : 0u) + blockIdx.x % SL * 64u * kCpl;  // without coordinates: 0, unstored
+    float y[kOwn * kCpl];
+#pragma unroll
+    for (uint32_t k = 0; k < kOwn * kCpl; ++k) y[k] = 0.0f;
+    float ssum = 0.0f;  // of token t0 + lane % kOwn
+
+    const uint32_t g_last = (en_max - 1u) / 8u;  // the last V tile with a position of the chunk
+    auto load_v = [&](uint32_t g, u32x4 (&w)[kCpl]) __attribute__((always_inline)) {
+        const uint32_t gg = min(g, g_last);
 #pragma unroll
         for (uint32_t m = 0; m < kCpl; ++m)
-            r[m] = *reinterpret_cast<const u32x4*>(vt + (static_cast<size_t>(gg) * HD + dl + 64u * m) * 8u);
+            w[m] = *reinterpret_cast<const u32x4*>(vt + (static_cast<size_t>(gg) * HD + dl + 64u * m) * 8u);
     };
 
-    // Scores, four lanes per position (ggml_vec_dot_f16, ops.rs:960-1015): lane j of a group holds accumulator j
-    // (values 32 i + 8 j .. + 7 of every 32-value block i) with q in registers as f32; (a0 + a2) + (a1 + a3) across the
-    // group, then red[k] + red[k + 4] and (t0 + t1) + (t2 + t3) in lane 0. The next position's k is loaded while the
-    // current one is summed.
-    {
-        const uint32_t j = tid & 3u, g = tid >> 2;
-        constexpr uint32_t kGroups = kThreads / 4u;
-        // q is read from LDS at each use (the 4-lane groups of a wave all read the same addresses: broadcasts), two
-        // f16 per register; each product widens both operands exactly, as f16_f32 does. Held in registers as f32 for
-        // the whole loop, it took 4 kBlk of them, which left room for one workgroup per CU instead of two.
-        auto load_k = [&](uint32_t p, uint4 (&kr)[kBlk]) {
-            if (p == pos) {
+    for (uint32_t sb = st / 32u * 32u; sb < en_max; sb += kRange) {
+        const uint32_t p0 = sb + POS * wave;  // this wave's positions
+        float sc[kTh][kPh][4];  // [16 tokens][16 positions][position 4 qt + e]
+        if (p0 < en_max) {
+            // K rows: lane (position l % 16 of 16, j = l / 16) holds its coordinates 32 i + 8 j .. + 7 (a position past
+            // the chunk repeats its last one; its factor is set to +0 below)
+            uint4 kr[kPh][kBlk];
 #pragma unroll
-                for (int i = 0; i < kBlk; ++i) kr[i] = *reinterpret_cast<const uint4*>(kp + 32 * i + 8 * j);
-            } else {
-                const uint16_t* row = kb + static_cast<size_t>(p) * HD + 8 * j;
+            for (uint32_t ph = 0; ph < kPh; ++ph) {
+                const uint16_t* row = kb + static_cast<size_t>(min(p0 + 16u * ph + cl, en_max - 1u)) * HD + 8u * qt;
 #pragma unroll
-                for (int i = 0; i < kBlk; ++i) kr[i] = *reinterpret_cast<const uint4*>(row + 32 * i);
+                for (int i = 0; i < kBlk; ++i) kr[ph][i] = *reinterpret_cast<const uint4*>(row + 32 * i);
             }
-        };
-        auto score = [&](uint32_t p, const uint4 (&kr)[kBlk]) {
-            uint32_t qo = 8u * j;
-            asm volatile("" : "+v"(qo));  // keeps q's reads in the loop (the compiler would hoist them into registers)
-            float acc[8];
+            auto dw = [](const uint4& v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); };
 #pragma unroll
-            for (int l = 0; l < 8; ++l) acc[l] = 0.0f;
+            for (uint32_t tile = 0; tile < kTh * kPh; ++tile) {
+                const uint32_t th = tile / kPh, ph = tile % kPh;
+                // k's conversions are made again for the second token half (kept, they would not fit the registers)
 #pragma unroll
-            for (int i = 0; i < kBlk; ++i) {
-                const uint32_t kw[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-                const uint4 qv = *reinterpret_cast<const uint4*>(qs + 32 * i + qo);
-                const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
+                for (int i = 0; i < kBlk; ++i)
+                    asm volatile("" : "+v"(kr[ph][i].x), "+v"(kr[ph][i].y), "+v"(kr[ph][i].z), "+v"(kr[ph][i].w));
+                float t01[4];
 #pragma unroll
-                for (int l = 0; l < 8; ++l)
-                    acc[l] = __builtin_fmaf(f16_f32(static_cast<uint16_t>(qw[l >> 1] >> ((l & 1) * 16))),
-                                            f16_f32(static_cast<uint16_t>(kw[l >> 1] >> ((l & 1) * 16))), acc[l]);
-            }
+                for (int dp = 0; dp < 2; ++dp) {          // chain lanes l = 2 dp, 2 dp + 1 and their partners l + 4
+                    float tt[2][4];
 #pragma unroll
-            for (int l = 0; l < 8; ++l) {
-                acc[l] = acc[l] + bits_f32(dpp32<kDppXor2>(f32_bits(acc[l])));  // lane j ^ 2 of the quad (DPP)
-                acc[l] = acc[l] + bits_f32(dpp32<kDppXor1>(f32_bits(acc[l])));  // lane j ^ 1
-            }
-            if (j == 0) {
-                const float t0 = acc[0] + acc[4], t1 = acc[1] + acc[5], t2 = acc[2] + acc[6], t3 = acc[3] + acc[7];
-                sc[p] = ((t0 + t1) + (t2 + t3)) * a.scale;
-            }
-        };
-        uint4 ka[kBlk], kn[kBlk];
-        uint32_t p = g;
-        if (p < seq) load_k(p, ka);
-        for (; p < seq; p += 2u * kGroups) {  // unrolled by two so that the buffers keep their registers
-            if (p + kGroups < seq) load_k(p + kGroups, kn);
-            score(p, ka);
-            if (p + kGroups >= seq) break;
-            if (p + 2u * kGroups < seq) load_k(p + 2u * kGroups, ka);
-            score(p + kGroups, kn);
-        }
-    }
+                    for (int up = 0; up < 2; ++up) {      // l = 2 dp + lo + 4 up: half lo of dword dp + 2 up
+                        // read here and not earlier: q's values of one step only are held in registers
+                        uint32_t qo = (16u * th + cl) * kQRow + 8u * qt + 2u * (dp + 2 * up);
+                        asm volatile("" : "+v"(qo));
+                        uint32_t qw[kBlk];
 #pragma unroll
-    for (uint32_t k = 0; k < kVDepth; ++k) load_group(g_first + k, ring[k]);
-    uint16_t vself[kCpl];
+                        for (int i = 0; i < kBlk; ++i) qw[i] = *reinterpret_cast<const uint32_t*>(&qs[0][0] + qo + 32 * i);
 #pragma unroll
-    for (uint32_t m = 0; m < kCpl; ++m) vself[m] = vp[dl + 64u * m];
-    __syncthreads();
-
-    if (wave < n_chunks) {  // the running maximum of chunk `wave`
-        const uint32_t s0 = wave * chunk, s1 = min(min(s0 + chunk, n_kv), seq);
-        float carry = -__builtin_inff();
-        for (uint32_t base = s0; base < s1; base += 64u) {
-            const uint32_t p = base + lane;
-            float v = p < s1 ? sc[p] : -__builtin_inff();
+                        for (int lo = 0; lo < 2; ++lo) {
+                            v16f acc = {};
 #pragma unroll
-            for (int sh = 1; sh < 64; sh <<= 1) {
-                const float o = __shfl_up(v, sh);
-                if (lane >= static_cast<uint32_t>(sh)) v = v > o ? v : o;
-            }
-            v = v > carry ? v : carry;
-            if (p < s1) pm[p] = v;
-            carry = __shfl(v, 63);
-        }
-    }
-    __syncthreads();
-
-    for (uint32_t p = tid; p < seq; p += kThreads) {
-        const uint32_t s0 = split ? p / chunk * chunk : 0u;
-        const float prev = p == s0 ? -__builtin_inff() : pm[p - 1];
-        const float s = sc[p];
-        sc[p] = s > prev ? -glibc_expf(prev - s) : glibc_expf(s - prev);
-    }
-    __syncthreads();
-
-    // The accumulator chains of this lane's coordinates over positions st .. en - 1, eight positions per group; a group
-    // with no new maximum (ms = 1 throughout) takes the shorter step.
-    float y[kCpl], ssum = 0.0f;
+                            for (int i = 0; i < kBlk; ++i)
+                                acc = __builtin_amdgcn_mfma_f32_16x16x1f32(
+                                    f16_f32(static_cast<uint16_t>(dw(kr[ph][i], dp + 2 * up) >> (16 * lo))),
+                                    f16_f32(static_cast<uint16_t>(qw[i] >> (16 * lo))), acc, 0, 0, 0);
 #pragma unroll
-    for (uint32_t m = 0; m < kCpl; ++m) y[m] = 0.0f;
-    if (chain) {
-        // the factors of the next group are read from LDS while the current group is summed, into the other of two
-        // slots (slot k & 1 of group slot k: kVDepth is even, so the pattern repeats on every pass of the loop)
-        static_assert(kVDepth % 2 == 0, "two factor slots alternate over the ring");
-        float4 fq[2][2];
-        fq[0][0] = *reinterpret_cast<const float4*>(sc + 8u * g_first);
-        fq[0][1] = *reinterpret_cast<const float4*>(sc + 8u * g_first + 4u);
-        for (uint32_t g0 = g_first; g0 < g_end; g0 += kVDepth) {
-            static_for<kVDepth>([&](auto kc) {  // the ring's slot as a constant: no rotation of its registers
-                constexpr uint32_t k = decltype(kc)::value;
-                const uint32_t gg = g0 + k;
-                {
-                    const uint32_t pn = 8u * min(gg + 1u, g_end - 1u);
-                    fq[(k + 1u) & 1u][0] = *reinterpret_cast<const float4*>(sc + pn);
-                    fq[(k + 1u) & 1u][1] = *reinterpret_cast<const float4*>(sc + pn + 4u);
-                }
-                if (gg < g_end) {  // wave-uniform
-                    // the group's V words, used in place; the slot is refilled (kVDepth groups ahead) once they are
-                    // consumed, so that the refill lands in the same registers (no register rotation)
-                    u32x4(&w)[kCpl] = ring[k];
-                    const uint32_t p0 = 8u * gg;
-                    const float4 fa = fq[k & 1u][0], fb = fq[k & 1u][1];
-                    if (pos >= p0 && pos < p0 + 8u) {  // the position itself, from this workgroup's copy
-                        const uint32_t e = pos - p0, sh = (e & 1u) * 16u, keep = ~(0xffffu << sh);
-#pragma unroll
-                        for (uint32_t m = 0; m < kCpl; ++m) {
-                            const uint32_t ins = static_cast<uint32_t>(vself[m]) << sh;
-                            const uint32_t q = e >> 1;
-                            w[m].x = q == 0 ? ((w[m].x & keep) | ins) : w[m].x;
-                            w[m].y = q == 1 ? ((w[m].y & keep) | ins) : w[m].y;
-                            w[m].z = q == 2 ? ((w[m].z & keep) | ins) : w[m].z;
-                            w[m].w = q == 3 ? ((w[m].w & keep) | ins) : w[m].w;
+                            for (int e = 0; e < 4; ++e) {
+                                const float r = (acc[e] + acc[8 + e]) + (acc[4 + e] + acc[12 + e]);
+                                tt[lo][e] = up == 0 ? r : tt[lo][e] + r;
+                            }
+                            __builtin_amdgcn_sched_barrier(0);  // one chain lane at a time: their sums would not fit
                         }
                     }
-                    float f[8] = {fa.x, fa.y, fa.z, fa.w, fb.x, fb.y, fb.z, fb.w};
-                    // A group that starts inside the chunk is summed whole: at its positions from en on (the chunk's
-                    // last group) the factor becomes +0 (vs = 0, no new maximum) and V -0, so that a step there adds
-                    // -0 and leaves y and the sum as they are.
-                    const bool whole = p0 >= st;
-                    if (whole && p0 + 8u > en) {
-                        const uint32_t n = en - p0;
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) f[e] = static_cast<uint32_t>(e) < n ? f[e] : 0.0f;
+                    for (int e = 0; e < 4; ++e) {
+                        const float s = tt[0][e] + tt[1][e];
+                        if (dp == 0) t01[e] = s;
+                        else sc[th][ph][e] = (t01[e] + s) * a.scale;
+                    }
+                }
+            }
+        }
+        // the maxima of every quarter's 4 positions, and the wave's
+        float qm[kTh][kPh][4];
 #pragma unroll
-                        for (uint32_t m = 0; m < kCpl; ++m) {
-                            uint32_t ww[4] = {w[m].x, w[m].y, w[m].z, w[m].w};
+        for (uint32_t th = 0; th < kTh; ++th) {
+            float tmax = -__builtin_inff();
+#pragma unroll
+            for (uint32_t ph = 0; ph < kPh; ++ph) {
+                float m = -__builtin_inff();
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e) {
+                    const uint32_t p = p0 + 16u * ph + 4u * qt + e;
+                    sc[th][ph][e] = p >= st && p < en[th] ? sc[th][ph][e] : -__builtin_inff();
+                    m = sc[th][ph][e] > m ? sc[th][ph][e] : m;
+                }
+                all_quarters(m, qm[th][ph]);
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) tmax = qm[th][ph][q] > tmax ? qm[th][ph][q] : tmax;
+            }
+            if (qt == 0) wmax[wave][16u * th + cl] = tmax;
+        }
+        __syncthreads();  // every wave is also done with the previous range's factors
+#pragma unroll
+        for (uint32_t th = 0; th < kTh; ++th) {
+            float m = carry[th];
+#pragma unroll
+            for (uint32_t w = 0; w < W; ++w) {
+                const float v = wmax[w][16u * th + cl];
+                carry[th] = v > carry[th] ? v : carry[th];
+                if (w < wave) m = v > m ? v : m;
+            }
+            if (p0 >= en_max) continue;
+#pragma unroll
+            for (uint32_t ph = 0; ph < kPh; ++ph) {
+                float prev = m;
+#pragma unroll
+                for (uint32_t q = 0; q < 3; ++q) prev = q < qt && qm[th][ph][q] > prev ? qm[th][ph][q] : prev;
+                float f[4];
+                uint32_t sign = 0;
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e) {
+                    const uint32_t p = p0 + 16u * ph + 4u * qt + e;
+                    const float s = sc[th][ph][e];
+                    const bool up = s > prev;
+                    const float x = expf_nonpos(up ? prev - s : s - prev, tab);
+                    f[e] = p >= st && p < en[th] ? (up ? -x : x) : 0.0f;
+                    sign |= f32_bits(f[e]);
+                    prev = up ? s : prev;
+                }
+                const uint32_t o = POS * wave + 16u * ph + 4u * qt;
+                *reinterpret_cast<float4*>(&fac[16u * th + cl][o]) = make_float4(f[0], f[1], f[2], f[3]);
+                float sq[4];
+                all_quarters(bits_f32(sign), sq);
+                if ((qt & 1u) == 0u) {
+                    const uint32_t s0 = qt == 0 ? f32_bits(sq[0]) : f32_bits(sq[2]), s1 = qt == 0 ? f32_bits(sq[1]) : f32_bits(sq[3]);
+                    newmax[o / 8u][16u * th + cl] = static_cast<uint8_t>(s0 >> 31 | s1 >> 31 << 1);
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) m = qm[th][ph][q] > m ? qm[th][ph][q] : m;
+            }
+        }
+        __syncthreads();
+
+        // the accumulators of the wave's tokens over the range, a ring of groups of 8 positions at a time
+        const uint32_t p_end = min(sb + kRange, own_max);
+        u32x4 v[kRing][kCpl];
+        if (sb < p_end) {
+#pragma unroll
+            for (uint32_t g = 0; g < kRing; ++g) load_v(sb / 8u + g, v[g]);
+        }
+        for (uint32_t pt = sb; pt < p_end; pt += 8u * kRing) {
+            static_for<kRing>([&](auto gc) {
+                constexpr uint32_t g = decltype(gc)::value;
+                const uint32_t pg = pt + 8u * g, fo = pg - sb;
+                u32x4(&w)[kCpl] = v[g];
+                auto value = [&](const u32x4& ww, int e) {
+                    const uint32_t word = e < 2 ? ww.x : (e < 4 ? ww.y : (e < 6 ? ww.z : ww.w));
+                    return f16_f32(static_cast<uint16_t>(word >> ((e & 1) * 16)));
+                };
+                const uint8_t* nmp = &newmax[fo / 8u][t0];  // a byte per token of the wave
+                const uint32_t nm = __builtin_amdgcn_readfirstlane(
+                    kOwn == 4u ? *reinterpret_cast<const uint32_t*>(nmp) : *reinterpret_cast<const uint16_t*>(nmp));
+                const float* fown = &fac[t0 + lane % kOwn][fo];
+                const float4 sa = *reinterpret_cast<const float4*>(fown), sz = *reinterpret_cast<const float4*>(fown + 4);
+                const float fs[8] = {sa.x, sa.y, sa.z, sa.w, sz.x, sz.y, sz.z, sz.w};
+                float fv[kOwn][8];
+#pragma unroll
+                for (uint32_t k = 0; k < kOwn; ++k) {
+                    const float4 fa = *reinterpret_cast<const float4*>(&fac[t0 + k][fo]);
+                    const float4 fb = *reinterpret_cast<const float4*>(&fac[t0 + k][fo + 4u]);
+                    fv[k][0] = fa.x, fv[k][1] = fa.y, fv[k][2] = fa.z, fv[k][3] = fa.w;
+                    fv[k][4] = fb.x, fv[k][5] = fb.y, fv[k][6] = fb.z, fv[k][7] = fb.w;
+                }
+                if (nm == 0u && pg >= st && pg + 8u <= own_min) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+#pragma unroll
+                        for (uint32_t k = 0; k < kOwn; ++k)
+#pragma unroll
+                            for (uint32_t m = 0; m < kCpl; ++m)
+                                y[k * kCpl + m] = __builtin_fmaf(value(w[m], e), fv[k][e], y[k * kCpl + m]);
+                        r16_all(y);
+                        ssum = ssum + fs[e];
+                    }
+                } else if (pg < p_end) {
+                    // a group with a new maximum of one of the tokens, or an edge of the chunk
+#pragma unroll
+                    for (uint32_t k = 0; k < kOwn; ++k) {
+                        if (pg >= own_en[k] || pg + 8u <= st) continue;  // wave-uniform
+                        // Positions outside [st, en): the factor is +0 there, and V is set to -0, so that a step
+                        // adds -0 and leaves y as it is (-0 + y = y for every y).
+                        u32x4 ww[kCpl];
+#pragma unroll
+                        for (uint32_t m = 0; m < kCpl; ++m) ww[m] = w[m];
+                        if (pg < st || pg + 8u > own_en[k]) {
+                            uint32_t keep[4];
 #pragma unroll
                             for (uint32_t q = 0; q < 4; ++q) {
-                                const uint32_t keep = (2u * q < n ? 0xffffu : 0u) | (2u * q + 1u < n ? 0xffff0000u : 0u);
-                                ww[q] = (ww[q] & keep) | (0x80008000u & ~keep);
+                                const uint32_t pa = pg + 2u * q, pb = pa + 1u;
+                                keep[q] = (pa >= st && pa < own_en[k] ? 0xffffu : 0u) | (pb >= st && pb < own_en[k] ? 0xffff0000u : 0u);
                             }
-                            w[m] = u32x4{ww[0], ww[1], ww[2], ww[3]};
-                        }
-                    }
-                    uint32_t neg = 0;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) neg |= f32_bits(f[e]) >> 31;
-                    neg = __builtin_amdgcn_readfirstlane(neg);
-                    if (whole && neg == 0) {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
 #pragma unroll
                             for (uint32_t m = 0; m < kCpl; ++m) {
-                                const uint32_t wv[4] = {w[m].x, w[m].y, w[m].z, w[m].w};
-                                const float v = f16_f32(static_cast<uint16_t>(wv[e >> 1] >> ((e & 1) * 16)));
-                                y[m] = __builtin_fmaf(v, f[e], y[m]);
+                                ww[m].x = (ww[m].x & keep[0]) | (0x80008000u & ~keep[0]);
+                                ww[m].y = (ww[m].y & keep[1]) | (0x80008000u & ~keep[1]);
+                                ww[m].z = (ww[m].z & keep[2]) | (0x80008000u & ~keep[2]);
+                                ww[m].w = (ww[m].w & keep[3]) | (0x80008000u & ~keep[3]);
                             }
-                            r16_all(y);
-                            ssum = ssum + f[e];
                         }
-                    } else if (whole) {
-                        // a group with a new maximum: the full step at every position (ms = 1 where there is none,
-                        // which leaves y as it is), straight-line
+                        float yk[kCpl];
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const bool nm = __builtin_signbit(f[e]);
-                            const float ev = __builtin_fabsf(f[e]);
-                            const float ms = nm ? ev : 1.0f, vs = nm ? 1.0f : ev;
+                        for (uint32_t m = 0; m < kCpl; ++m) yk[m] = y[k * kCpl + m];
 #pragma unroll
-                            for (uint32_t m = 0; m < kCpl; ++m) y[m] = y[m] * ms;
-                            r16_all(y);
+                        for (int hf = 0; hf < 2; ++hf) {
+                            const float* f = &fv[k][4 * hf];
+                            if ((nm >> (8u * k + hf) & 1u) == 0u) {
 #pragma unroll
-                            for (uint32_t m = 0; m < kCpl; ++m) {
-                                const uint32_t wv[4] = {w[m].x, w[m].y, w[m].z, w[m].w};
-                                const float v = f16_f32(static_cast<uint16_t>(wv[e >> 1] >> ((e & 1) * 16)));
-                                y[m] = __builtin_fmaf(v, vs, y[m]);
-                            }
-                            r16_all(y);
-                            ssum = __builtin_fmaf(ssum, ms, vs);
-                        }
-                    } else {  // the chunk starts inside this group (positions before it skipped)
-                        const uint32_t e0 = p0 < st ? st - p0 : 0u, e1 = min(8u, en - p0);
+                                for (int e = 0; e < 4; ++e) {
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            if (static_cast<uint32_t>(e) >= e0 && static_cast<uint32_t>(e) < e1) {
-                                const bool nm = __builtin_signbit(f[e]);
-                                const float ev = __builtin_fabsf(f[e]);
-                                const float ms = nm ? ev : 1.0f, vs = nm ? 1.0f : ev;
-#pragma unroll
-                                for (uint32_t m = 0; m < kCpl; ++m) y[m] = y[m] * ms;
-                                r16_all(y);
-#pragma unroll
-                                for (uint32_t m = 0; m < kCpl; ++m) {
-                                    const uint32_t wv[4] = {w[m].x, w[m].y, w[m].z, w[m].w};
-                                    const float v = f16_f32(static_cast<uint16_t>(wv[e >> 1] >> ((e & 1) * 16)));
-                                    y[m] = __builtin_fmaf(v, vs, y[m]);
+                                    for (uint32_t m = 0; m < kCpl; ++m) yk[m] = __builtin_fmaf(value(ww[m], 4 * hf + e), f[e], yk[m]);
+                                    r16_all(yk);
                                 }
-                                r16_all(y);
-                                ssum = __builtin_fmaf(ssum, ms, vs);
+                            } else {  // the full step at every position (ms = 1 where there is no new maximum)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const bool up = __builtin_signbit(f[e]);
+                                    const float ev = __builtin_fabsf(f[e]);
+                                    const float ms = up ? ev : 1.0f, vs = up ? 1.0f : ev;
+#pragma unroll
+                                    for (uint32_t m = 0; m < kCpl; ++m) yk[m] = yk[m] * ms;
+                                    r16_all(yk);
+#pragma unroll
+                                    for (uint32_t m = 0; m < kCpl; ++m) yk[m] = __builtin_fmaf(value(ww[m], 4 * hf + e), vs, yk[m]);
+                                    r16_all(yk);
+                                }
                             }
                         }
+#pragma unroll
+                        for (uint32_t m = 0; m < kCpl; ++m) y[k * kCpl + m] = yk[m];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const bool up = __builtin_signbit(fs[e]);
+                        const float ev = __builtin_fabsf(fs[e]);
+                        ssum = __builtin_fmaf(ssum, up ? ev : 1.0f, up ? 1.0f : ev);
                     }
                 }
-                // every slot is refilled, used or not (the index stays inside the cache), so that the number of
-                // loads issued after a slot's refill, and with it the wait for the slot, is the same on every path
-                load_group(gg + kVDepth, ring[k]);
+                load_v(pg / 8u + kRing, w);
             });
         }
     }
-    float* out = a.out + (static_cast<size_t>(tok) * a.n_heads + h) * HD;
-    if (!split) {
-        if (c == 0 && has_d) {
-            const float s_inv = ssum == 0.0f ? 0.0f : 1.0f / ssum;
+
 #pragma unroll
-            for (uint32_t m = 0; m < kCpl; ++m) out[d0 + 64u * m] = y[m] * s_inv;
-        }
-        return;
-    }
-    if (c < 4) {
-        if (has_d) {
+    for (uint32_t k = 0; k < kOwn; ++k) {
+        if (own_en[k] <= st) continue;  // the token is not of the pass, or has no position in the chunk
+        const size_t ti = tp + t0 + k - first;
+        const float s = bits_f32(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(f32_bits(ssum)), static_cast<int>(k))));
+        if (kv.n_chunks == 1u) {
+            const float s_inv = s == 0.0f ? 0.0f : 1.0f / s;
 #pragma unroll
-            for (uint32_t m = 0; m < kCpl; ++m) cv[c][d0 + 64u * m] = f32_f16(y[m]);
-        }
-        if (wave % kWpc == 0 && lane == 0) {
-            cm[c] = st < en ? pm[en - 1] : -__builtin_inff();
-            cs[c] = ssum;
+            for (uint32_t m = 0; m < kCpl; ++m)
+                if (has_d) a.out[ti * qd + h * HD + dl + 64u * m] = y[k * kCpl + m] * s_inv;
+        } else {
+            const size_t slot = (ti * a.n_heads + h) * 4u + c;
+#pragma unroll
+            for (uint32_t m = 0; m < kCpl; ++m)
+                if (has_d) a.cy[slot * HD + dl + 64u * m] = f32_f16(y[k * kCpl + m]);
+            if (lane == 0 && blockIdx.x % SL == 0) a.cms[2u * slot + 1u] = s;
         }
     }
+    if (kv.n_chunks > 1u && wave == 0 && blockIdx.x % SL == 0 && qt < kTh) {
+        const uint32_t e = kTh == 1u || qt == 0 ? en[0] : en[kTh - 1u];
+        if (e > st)
+            a.cms[2u * (((tp + lane - first) * static_cast<size_t>(a.n_heads) + h) * 4u + c)] = kTh == 1u || qt == 0 ? carry[0] : carry[kTh - 1u];
+    }
+}
+
+// The chunks of every token with a split context, combined in order (attention.rs:526-541). A thread computes the
+// chunks' weights once for 8 coordinates (for one, they cost more than everything else).
+template <int HD>
+__global__ __launch_bounds__(256) void pf_attn_combine_kernel(PfAttnArgs a) {
+    __shared__ uint64_t etab[32];
+    if (threadIdx.x < 32u) etab[threadIdx.x] = expf_tab(threadIdx.x);
     __syncthreads();
-    if (c != 0 || !has_d) return;
+    const auto tab = [&](uint32_t k) { return etab[k]; };
+    const uint32_t t = blockIdx.y, i = (blockIdx.x * 256u + threadIdx.x) * 8u;
+    const uint32_t seq = a.ctl->pos + 2u - a.n_tok + t, h = i / HD;
+    const KvSplit kv = kv_split(seq, a.max_ctx);
+    if (kv.n_chunks == 1u || h >= a.n_heads) return;
+    const size_t slot = (static_cast<size_t>(t) * a.n_heads + h) * 4u;
+    float mk[4], sk[4];
+    uint4 yk[4];
 #pragma unroll
-    for (uint32_t m = 0; m < kCpl; ++m) {
-        const uint32_t d = d0 + 64u * m;
-        float mf = -__builtin_inff(), sf = 0.0f, acc = 0.0f;
-        for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t ks = k * chunk, ke = min(min(ks + chunk, n_kv), seq);
-            if (ks >= ke) continue;
-            const float sk = cs[k];
-            if (sk == 0.0f) continue;
-            const float mk = cm[k];
-            const float mn = __builtin_fmaxf(mf, mk);
-            const float so = glibc_expf(mf - mn);
-            const float sn = glibc_expf(mk - mn);
-            const float vn = f16_f32(cv[k][d]) * sn;
-            acc = __builtin_fmaf(acc, so, vn);
-            const float ssn = sk * sn;
-            sf = __builtin_fmaf(sf, so, ssn);
-            mf = mn;
-        }
-        out[d] = sf != 0.0f ? acc * (1.0f / sf) : acc;
+    for (uint32_t k = 0; k < 4; ++k) {
+        const bool have = k * kv.chunk < min(min((k + 1u) * kv.chunk, kv.n_kv), seq);
+        mk[k] = have ? a.cms[2u * (slot + k)] : 0.0f;
+        sk[k] = have ? a.cms[2u * (slot + k) + 1u] : 0.0f;
+        yk[k] = have ? *reinterpret_cast<const uint4*>(a.cy + (slot + k) * HD + i % HD) : make_uint4(0u, 0u, 0u, 0u);
     }
+    float mf = -__builtin_inff(), sf = 0.0f, acc[8];
+#pragma unroll
+    for (uint32_t e = 0; e < 8; ++e) acc[e] = 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        if (sk[k] == 0.0f) continue;  // no positions, or a sum of zero
+        const float mn = __builtin_fmaxf(mf, mk[k]);
+        const float so = glibc_expf_with(mf - mn, tab);
+        const float sn = glibc_expf_with(mk[k] - mn, tab);
+        const uint32_t w[4] = {yk[k].x, yk[k].y, yk[k].z, yk[k].w};
+#pragma unroll
+        for (uint32_t e = 0; e < 8; ++e) {
+            const float vn = f16_f32(static_cast<uint16_t>(w[e / 2u] >> (16u * (e & 1u)))) * sn;
+            acc[e] = __builtin_fmaf(acc[e], so, vn);
+        }
+        const float ssn = sk[k] * sn;
+        sf = __builtin_fmaf(sf, so, ssn);
+        mf = mn;
+    }
+    const float inv = 1.0f / sf;
+    float o[8];
+#pragma unroll
+    for (uint32_t e = 0; e < 8; ++e) o[e] = sf != 0.0f ? acc[e] * inv : acc[e];
+    float4* out = reinterpret_cast<float4*>(a.out + static_cast<size_t>(t) * a.n_heads * HD + i);
+    out[0] = make_float4(o[0], o[1], o[2], o[3]);
+    out[1] = make_float4(o[4], o[5], o[6], o[7]);
 }
 
 // ---- decode attention: scores, then the accumulator chains ---------------------------------------------------------------
@@ -2522,18 +2604,6 @@ int launch_dgemv(const DStageArgs& a, hipStream_t s) {
     return VX_OK;
 }
 
-template <bool PREFILL>
-static int launch_attention_mode(const AttnArgs& a, uint32_t head_dim, hipStream_t s) {
-    const dim3 grid(a.n_heads, PREFILL ? a.n_tok : 1u);
-    if (head_dim == 256) hipLaunchKernelGGL((attention_kernel<256, PREFILL>), grid, dim3(attn_threads(256)), 0, s, a);
-    else if (head_dim == 128) hipLaunchKernelGGL((attention_kernel<128, PREFILL>), grid, dim3(attn_threads(128)), 0, s, a);
-    else if (head_dim == 64) hipLaunchKernelGGL((attention_kernel<64, PREFILL>), grid, dim3(attn_threads(64)), 0, s, a);
-    else if (head_dim == 32) hipLaunchKernelGGL((attention_kernel<32, PREFILL>), grid, dim3(attn_threads(32)), 0, s, a);
-    else VX_FAIL(VX_ERR_INTERNAL, "no attention kernel for head_dim %u", head_dim);
-    VX_HIP(hipGetLastError());
-    return VX_OK;
-}
-
 // The decode step's attention: the score kernel over every 64-position range of max_ctx (ranges past the position
 // return at once), then the chain kernel over (head, 64 coordinates) x 4 chunks (chunks past the split return).
 int launch_attention(const AttnArgs& a, uint32_t head_dim, hipStream_t s) {
@@ -2572,8 +2642,36 @@ int launch_attention_short(const AttnArgs& a, uint32_t head_dim, hipStream_t s) 
     return VX_OK;
 }
 
-int launch_attention_prefill(const AttnArgs& a, uint32_t head_dim, hipStream_t s) {
-    return launch_attention_mode<true>(a, head_dim, s);
+template <int HD, int TOK, int POS, int W, int SL>
+static void launch_pf_attn_as(const PfAttnArgs& a, bool split, hipStream_t s) {
+    // one tile more than the tokens fill: they need not start at a multiple of TOK
+    const dim3 grid(a.n_heads * SL, (a.n_tok + TOK - 1u) / TOK + 1u, split ? 4u : 1u);
+    hipLaunchKernelGGL((pf_attn_kernel<HD, TOK, POS, W, SL>), grid, dim3(64 * W), 0, s, a);
+}
+
+// A workgroup takes 16 tokens and all coordinates of a head where that gives two workgroups per CU or more. Below that
+// the chains of the few workgroups set the time, and the head's coordinates go to HD / 64 workgroups of twice the waves
+// (each computing every score): 64 tokens of 12 heads of 256 12.2 us instead of 21.7 (48 whole-head workgroups), 256 of
+// them 42.6 instead of 53.2 (192); 256 tokens of 20 heads of 128 29.7 instead of 38.5 (320); with 300 tokens (912 and
+// 1520 workgroups, the split context) the two forms take the same time.
+template <int HD>
+static void launch_pf_attn(const PfAttnArgs& a, int num_cus, bool split, hipStream_t s) {
+    const uint32_t wgs = a.n_heads * ((a.n_tok + 15u) / 16u) * (split ? 4u : 1u);
+    if (wgs < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 16, 16, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
+    else launch_pf_attn_as<HD, 16, 16, 4, 1>(a, split, s);
+    if (split)
+        hipLaunchKernelGGL(pf_attn_combine_kernel<HD>, dim3((a.n_heads * HD + 2047u) / 2048u, a.n_tok), dim3(256), 0, s, a);
+}
+
+// The attention of a prefill pass; split: some position of the pass has a padded length of 512 or more.
+int launch_attention_prefill(const PfAttnArgs& a, uint32_t head_dim, int num_cus, bool split, hipStream_t s) {
+    if (head_dim == 256) launch_pf_attn<256>(a, num_cus, split, s);
+    else if (head_dim == 128) launch_pf_attn<128>(a, num_cus, split, s);
+    else if (head_dim == 64) launch_pf_attn<64>(a, num_cus, split, s);
+    else if (head_dim == 32) launch_pf_attn<32>(a, num_cus, split, s);
+    else VX_FAIL(VX_ERR_INTERNAL, "no attention kernel for head_dim %u", head_dim);
+    VX_HIP(hipGetLastError());
+    return VX_OK;
 }
 
 int launch_head(const HeadArgs& a, bool f16, uint32_t grid, hipStream_t s) {
@@ -2648,12 +2746,14 @@ struct vx_decoder {
     uint32_t pf_ld[vx::kProjKinds];
     uint16_t* pf_q;                   // [pf_cap][n_heads * head_dim] rotated f16 queries
     float* pf_att;                    // [pf_cap][n_heads * head_dim] attention outputs
+    uint16_t* pf_cy;                  // [pf_cap][n_heads][4][head_dim] chunk accumulators of split contexts (PfAttnArgs)
+    float* pf_cms;                    // [pf_cap][n_heads][4][2] their maxima and sums
     float* pf_act;                    // [pf_cap][ffn] gated activations
     uint8_t* pf_staged;               // the GEMM's staged activations
     uint8_t* pf_part;                 // the GEMM's K-slice partial sums
     struct PfGraph {
         uint32_t n;
-        bool head;
+        bool head, split;
         hipGraph_t graph;
         hipGraphExec_t exec;
     };
@@ -2702,7 +2802,8 @@ static void drop_graph(vx_decoder* d) {
 }
 
 static void free_prefill(vx_decoder* d) {
-    void* bufs[] = {d->pf_x, d->pf_codes, d->pf_as, d->pf_q, d->pf_att, d->pf_act, d->pf_staged, d->pf_part};
+    void* bufs[] = {d->pf_x,   d->pf_codes, d->pf_as,     d->pf_q,   d->pf_att,
+                    d->pf_cy,  d->pf_cms,   d->pf_act,    d->pf_staged, d->pf_part};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (int32_t*& y : d->pf_y) {
@@ -2714,6 +2815,8 @@ static void free_prefill(vx_decoder* d) {
     d->pf_as = nullptr;
     d->pf_q = nullptr;
     d->pf_att = nullptr;
+    d->pf_cy = nullptr;
+    d->pf_cms = nullptr;
     d->pf_act = nullptr;
     d->pf_staged = nullptr;
     d->pf_part = nullptr;
@@ -3198,6 +3301,10 @@ static int ensure_prefill(vx_decoder* d) {
     }
     grab(&d->pf_q, static_cast<size_t>(cap) * d->qd * 2);
     grab(&d->pf_att, static_cast<size_t>(cap) * d->qd * 4);
+    if (c.max_ctx >= 2 * kShortCtx) {
+        grab(&d->pf_cy, static_cast<size_t>(cap) * d->qd * 4 * 2);
+        grab(&d->pf_cms, static_cast<size_t>(cap) * c.n_heads * 4 * 2 * 4);
+    }
     grab(&d->pf_act, static_cast<size_t>(cap) * c.ffn * 4);
     grab(&d->pf_staged, stage_bytes);
     grab(&d->pf_part, part_bytes);
@@ -3222,7 +3329,8 @@ static ProjOut pf_proj_out(const vx_decoder* d, size_t layer, int kind, const fl
 
 // Enqueues one prefill pass over n tokens (the last at the loop state's position) on `st`; with `head`, the final norm,
 // head and greedy argmax of the last token follow and advance the loop state as a decode step does.
-static int record_prefill(const vx_decoder* d, uint32_t n, bool head, hipStream_t st) {
+// split: some position of the pass is at kShortCtx or beyond, where the attention runs in chunks.
+static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split, hipStream_t st) {
     const vx_decoder_config_t& c = d->cfg;
     const size_t L = c.n_layers, H = c.hidden, F = c.ffn;
     const bool sub = has_sub_norms(d);
@@ -3309,20 +3417,21 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, hipStream_
         const uint32_t n_elem = c.n_heads * c.head_dim / 2u + c.n_kv_heads * c.head_dim / 2u + c.n_kv_heads * c.head_dim;
         hipLaunchKernelGGL(pf_rope_kernel, dim3(n, (n_elem + 255u) / 256u), dim3(256), 0, st, ra);
         VX_HIP(hipGetLastError());
-        AttnArgs at{};
+        PfAttnArgs at{};
         at.ctl = d->d_ctl;
         at.kc = d->d_kc + l * layer_kv;
         at.vc = d->d_vc + l * layer_v;
         at.vstride = vstride_of(c.max_ctx);
         at.out = d->pf_att;
+        at.cy = d->pf_cy;
+        at.cms = d->pf_cms;
         at.n_heads = c.n_heads;
         at.gqa = c.n_heads / c.n_kv_heads;
         at.max_ctx = c.max_ctx;
-        at.rope_normal = ra.rope_normal;
         at.scale = 1.0f / sqrtf(static_cast<float>(c.head_dim));
         at.qbuf = d->pf_q;
         at.n_tok = n;
-        VX_TRY(launch_attention_prefill(at, c.head_dim, st));
+        VX_TRY(launch_attention_prefill(at, c.head_dim, d->num_cus, split, st));
         // the o input: attention output (sub-norm or none)
         in = stage_input(d, kInPlain, d->qd, d->pf_att, nullptr, sub ? nw[VX_NORM_ATTN_SUB] : nullptr);
         VX_TRY(stage(in, static_cast<uint32_t>(d->qd), 0, as_o));
@@ -3388,9 +3497,9 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, hipStream_
 }
 
 // The graph of a prefill pass over n tokens (recorded on first use; a few are kept).
-static int prefill_graph(vx_decoder* d, uint32_t n, bool head, hipGraphExec_t* out) {
+static int prefill_graph(vx_decoder* d, uint32_t n, bool head, bool split, hipGraphExec_t* out) {
     for (const auto& g : d->pf_graphs)
-        if (g.n == n && g.head == head) {
+        if (g.n == n && g.head == head && g.split == split) {
             *out = g.exec;
             return VX_OK;
         }
@@ -3401,7 +3510,7 @@ static int prefill_graph(vx_decoder* d, uint32_t n, bool head, hipGraphExec_t* o
         d->pf_graphs.erase(d->pf_graphs.begin());
     }
     VX_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-    const int st = record_prefill(d, n, head, d->stream);
+    const int st = record_prefill(d, n, head, split, d->stream);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(d->stream, &graph);
     if (st != VX_OK) {
@@ -3415,7 +3524,7 @@ static int prefill_graph(vx_decoder* d, uint32_t n, bool head, hipGraphExec_t* o
         (void)hipGraphDestroy(graph);
         VX_HIP(ei);
     }
-    d->pf_graphs.push_back({n, head, graph, exec});
+    d->pf_graphs.push_back({n, head, split, graph, exec});
     *out = exec;
     return VX_OK;
 }
@@ -3429,7 +3538,9 @@ static int run_prefill(vx_decoder* d, uint32_t pos0, uint32_t n, uint32_t n_prom
         const uint32_t m = std::min(d->pf_cap, n - done);
         const bool last = done + m == n;
         hipGraphExec_t exec = nullptr;
-        VX_TRY(prefill_graph(d, m, last, &exec));
+        // the split starts at a padded length of 512 (kv_split), so at position 256, unless max_ctx caps it below
+        const bool split = d->cfg.max_ctx >= 2 * kShortCtx && pos0 + done + m > kShortCtx;
+        VX_TRY(prefill_graph(d, m, last, split, &exec));
         hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(64), 0, d->stream, d->d_ctl, pos0 + done + m - 1, 0u, n_prompt, n_out);
         VX_HIP(hipGetLastError());
         VX_HIP(hipGraphLaunch(exec, d->stream));

@@ -46,22 +46,15 @@ VX_HD inline float bits_f32(uint32_t u) { return __builtin_bit_cast(float, u); }
 VX_HD inline double bits_f64(uint64_t u) { return __builtin_bit_cast(double, u); }
 VX_HD inline uint64_t f64_bits(double d) { return __builtin_bit_cast(uint64_t, d); }
 
-// The function with the table read through tab(i) (a device caller may keep the table in LDS).
+// The function without its range checks: for |x| < 88, for NaN (which it returns), and for -0x1.9fe368p6 <= x <= -88.
+// The table is read through tab(i) (a device caller may keep it in LDS).
 template <typename Tab>
-VX_HD inline float glibc_expf_with(float x, Tab tab) {
+VX_HD inline float glibc_expf_core(float x, Tab tab) {
     const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
     const double kShift = 0x1.8p+52;
     const double kC0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
     const double kC1 = 0x1.ebfce50fac4f3p-3 / 32.0 / 32.0;
     const double kC2 = 0x1.62e42ff0c52d6p-1 / 32.0;
-    const uint32_t abstop = (f32_bits(x) >> 20) & 0x7ffu;
-    if (abstop >= ((f32_bits(88.0f) >> 20) & 0x7ffu)) {
-        // |x| >= 88 or x is NaN
-        if (f32_bits(x) == f32_bits(-__builtin_inff())) return 0.0f;
-        if (abstop >= ((f32_bits(__builtin_inff()) >> 20) & 0x7ffu)) return x + x;
-        if (x > 0x1.62e42ep6f) return __builtin_inff();  // overflow
-        if (x < -0x1.9fe368p6f) return 0.0f;             // underflow
-    }
     const double xd = static_cast<double>(x);
     double kd = __builtin_fma(kInvLn2N, xd, kShift);  // k = round(x * 32 / ln2), ties to even
     const uint64_t ki = f64_bits(kd);
@@ -76,6 +69,19 @@ VX_HD inline float glibc_expf_with(float x, Tab tab) {
     y = __builtin_fma(z, r2, y);
     y = y * s;
     return static_cast<float>(y);
+}
+
+template <typename Tab>
+VX_HD inline float glibc_expf_with(float x, Tab tab) {
+    const uint32_t abstop = (f32_bits(x) >> 20) & 0x7ffu;
+    if (abstop >= ((f32_bits(88.0f) >> 20) & 0x7ffu)) {
+        // |x| >= 88 or x is NaN
+        if (f32_bits(x) == f32_bits(-__builtin_inff())) return 0.0f;
+        if (abstop >= ((f32_bits(__builtin_inff()) >> 20) & 0x7ffu)) return x + x;
+        if (x > 0x1.62e42ep6f) return __builtin_inff();  // overflow
+        if (x < -0x1.9fe368p6f) return 0.0f;             // underflow
+    }
+    return glibc_expf_core(x, tab);
 }
 
 VX_HD inline float glibc_expf(float x) { return glibc_expf_with(x, expf_tab); }
