@@ -34,7 +34,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <initializer_list>
 #include <type_traits>
 #include <vector>
 
@@ -64,16 +63,6 @@ __device__ __forceinline__ uint16_t f32_f16(float f) {
     return __builtin_bit_cast(uint16_t, static_cast<_Float16>(keep_f32(f)));
 }
 __device__ __forceinline__ float f16_f32(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
-
-// f(std::integral_constant<uint32_t, k>) for k = 0 .. N - 1: a loop body with its index as a compile-time constant, so that
-// arrays indexed by it stay in fixed registers (a counted loop may be kept rolled, with the registers rotated).
-template <uint32_t N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<uint32_t, N - 1>{});
-    }
-}
 
 // ---- wave reductions (DPP within rows of 16 lanes, then the four row results) ------------------------------------------------
 
@@ -2400,8 +2389,10 @@ struct PfStageArgs {
     StageInput in;          // the input of token 0; rows of x_in / x_out are x_stride floats apart, of a.part a_stride
     uint32_t x_stride, a_stride, n_tok;
     const uint32_t* prompt;  // kInEmbed: the token at each position
-    int8_t* codes;          // [n_tok][codes_stride]
+    int8_t* codes;          // [n_tok][codes_stride]; unused where staged is set
     uint32_t codes_stride;
+    uint4* staged;          // the codes as the GEMM's B fragments (gemm_fragment), or null
+    uint32_t n_ksteps, n_tg;  // staged: K steps of the input, token groups of 32
     float* as_out;          // [n_tok]
 };
 
@@ -2437,7 +2428,7 @@ __global__ __launch_bounds__(kNT) void pf_stage_kernel(PfStageArgs a) {
     float m = 0.0f;
     for (int w = 0; w < kNT / 64; ++w) m = fmax_nn(m, s.red_f[w]);
     const float sc = m > 0.0f ? 127.0f / m : 0.0f;
-    int8_t* row = a.codes + static_cast<size_t>(t) * a.codes_stride;
+    int8_t* row = a.staged != nullptr ? reinterpret_cast<int8_t*>(s.ys) : a.codes + static_cast<size_t>(t) * a.codes_stride;
 #pragma unroll
     for (int k = 0; k < P4; ++k) {
         const uint32_t i = elem4(tid, k);
@@ -2449,6 +2440,14 @@ __global__ __launch_bounds__(kNT) void pf_stage_kernel(PfStageArgs a) {
                 w4 |= (static_cast<uint32_t>(x) & 0xffu) << (8 * e);
             }
             *reinterpret_cast<uint32_t*>(row + i) = w4;
+        }
+    }
+    if (a.staged != nullptr) {  // the same in every workgroup
+        __syncthreads();
+        for (uint32_t i = tid; i < a.n_ksteps * 10u; i += kNT) {
+            const uint32_t ks = i / 10u, kb = i % 10u >> 1, hs = i & 1u;
+            a.staged[(static_cast<size_t>(ks * 5u + kb) * a.n_tg + (t >> 5)) * 64u + (t & 31u) + 32u * hs] =
+                gemm_fragment(row, in.n, ks, kb, hs);
         }
     }
     if (tid == 0) a.as_out[t] = sc;
@@ -3273,20 +3272,11 @@ static int ensure_prefill(vx_decoder* d) {
     size_t stage_bytes = 0, part_bytes = 0;
     for (size_t cols : {static_cast<size_t>(c.hidden), d->qd, static_cast<size_t>(c.ffn)})
         stage_bytes = std::max(stage_bytes, gemm_stage_bytes(cols, cap));
-    for (int k = 0; k < kProjKinds; ++k) {
-        const Geometry& g = d->proj[k]->g;  // every layer's projection k has this shape
-        for (uint32_t m = 1; m <= cap; ++m) part_bytes = std::max(part_bytes, gemm_part_bytes(g, m, d->num_cus));
-    }
-    {  // q, k and v, and gate and up, in one launch each (record_prefill)
-        GemmSub qkv[3], gu[2];
-        for (int k = 0; k < 3; ++k) qkv[k] = GemmSub{nullptr, &d->proj[VX_PROJ_Q + k]->g, nullptr, 0};
-        for (int k = 0; k < 2; ++k) gu[k] = GemmSub{nullptr, &d->proj[VX_PROJ_GATE + k]->g, nullptr, 0};
-        for (uint32_t m = 1; m <= cap; ++m) {
-            if (gemm_group_small_path(qkv, 3, m, d->num_cus))
-                part_bytes = std::max(part_bytes, gemm_group_part_bytes(qkv, 3, m, d->num_cus));
-            if (gemm_group_small_path(gu, 2, m, d->num_cus))
-                part_bytes = std::max(part_bytes, gemm_group_part_bytes(gu, 2, m, d->num_cus));
-        }
+    for (const auto& kinds : kStageKinds) {  // every layer's projections have these shapes
+        GemmSub subs[kMaxStageJobs];
+        int k = 0;
+        for (; k < kMaxStageJobs && kinds[k] >= 0; ++k) subs[k] = GemmSub{nullptr, &d->proj[kinds[k]]->g, nullptr, 0};
+        for (uint32_t m = 1; m <= cap; ++m) part_bytes = std::max(part_bytes, gemm_group_part_bytes(subs, k, m, d->num_cus));
     }
     hipError_t e = hipSuccess;
     auto grab = [&](auto** p, size_t bytes) {
@@ -3340,8 +3330,15 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
     float* as_o = d->pf_as + cap;
     float* as_ffn = d->pf_as + 2 * cap;
     float* as_down = d->pf_as + 3 * cap;
+    // more than kGemmSmallM tokens are staged by the kernel that quantizes them
+    const bool staged = n > kGemmSmallM;
     auto stage = [&](const StageInput& in, uint32_t x_stride, uint32_t a_stride, float* as_out) -> int {
         PfStageArgs a{};
+        if (staged) {
+            a.staged = reinterpret_cast<uint4*>(d->pf_staged);
+            a.n_ksteps = static_cast<uint32_t>(gemm_ksteps(in.n));
+            a.n_tg = (n + 31u) / 32u;
+        }
         a.in = in;
         a.x_stride = x_stride;
         a.a_stride = a_stride;
@@ -3352,19 +3349,16 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
         a.as_out = as_out;
         return launch_pf_stage(a, st);
     };
-    // GEMMs on the small path read the codes themselves; the others read them staged once per input
-    auto small = [&](int kind) { return gemm_small_path(d->proj[kind]->g, n, d->num_cus); };
-    auto gemm_stage = [&](size_t cols, std::initializer_list<int> kinds) -> int {
-        bool need = false;
-        for (int k : kinds) need = need || !small(k);
-        return need ? launch_gemm_stage(d->pf_codes, n, d->pf_codes_ld, cols, d->pf_staged, st) : VX_OK;
-    };
-    auto gemm = [&](size_t layer, int kind) -> int {
-        const vx_matrix* m = d->proj[layer * kProjKinds + kind];
-        if (small(kind))
-            return launch_gemm(m->d_w, m->g, d->num_cus, d->pf_codes, n, d->pf_codes_ld, d->pf_y[kind], d->pf_ld[kind],
-                               d->pf_part, st);
-        return launch_gemm_staged(m->d_w, m->g, d->num_cus, d->pf_staged, n, d->pf_y[kind], d->pf_ld[kind], d->pf_part, st);
+    // the projections of a stage (kStageKinds), which share their input, in one launch
+    auto gemm = [&](size_t layer, int stage) -> int {
+        GemmSub subs[kMaxStageJobs];
+        int k = 0;
+        for (; k < kMaxStageJobs && kStageKinds[stage][k] >= 0; ++k) {
+            const int kind = kStageKinds[stage][k];
+            const vx_matrix* m = d->proj[layer * kProjKinds + kind];
+            subs[k] = GemmSub{m->d_w, &m->g, d->pf_y[kind], d->pf_ld[kind]};
+        }
+        return launch_gemm_group(subs, k, d->num_cus, staged ? nullptr : d->pf_codes, n, d->pf_codes_ld, d->pf_staged, d->pf_part, st);
     };
     for (size_t l = 0; l < L; ++l) {
         const float* const* nw = d->norms.data() + l * kNormKinds;
@@ -3379,18 +3373,7 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
             in.a = pf_proj_out(d, l - 1, VX_PROJ_DOWN, as_down);
         }
         VX_TRY(stage(in, static_cast<uint32_t>(H), d->pf_ld[VX_PROJ_DOWN], as_qkv));
-        // q, k and v in one small-path launch where each takes that path
-        GemmSub qkv[3];
-        for (int k = 0; k < 3; ++k) {
-            const vx_matrix* m = d->proj[l * kProjKinds + VX_PROJ_Q + k];
-            qkv[k] = GemmSub{m->d_w, &m->g, d->pf_y[VX_PROJ_Q + k], d->pf_ld[VX_PROJ_Q + k]};
-        }
-        if (gemm_group_small_path(qkv, 3, n, d->num_cus)) {
-            VX_TRY(launch_gemm_group(qkv, 3, d->num_cus, d->pf_codes, n, d->pf_codes_ld, d->pf_part, st));
-        } else {
-            VX_TRY(gemm_stage(H, {VX_PROJ_Q, VX_PROJ_K, VX_PROJ_V}));
-            for (int k : {VX_PROJ_Q, VX_PROJ_K, VX_PROJ_V}) VX_TRY(gemm(l, k));
-        }
+        VX_TRY(gemm(l, 0));
         PfRopeArgs ra{};
         ra.ctl = d->d_ctl;
         ra.n_tok = n;
@@ -3435,30 +3418,12 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
         // the o input: attention output (sub-norm or none)
         in = stage_input(d, kInPlain, d->qd, d->pf_att, nullptr, sub ? nw[VX_NORM_ATTN_SUB] : nullptr);
         VX_TRY(stage(in, static_cast<uint32_t>(d->qd), 0, as_o));
-        VX_TRY(gemm_stage(d->qd, {VX_PROJ_O}));
-        VX_TRY(gemm(l, VX_PROJ_O));
+        VX_TRY(gemm(l, 1));
         // x + o, FFN norm
         in = stage_input(d, kInResidual, H, d->pf_x, d->pf_x, nw[VX_NORM_FFN]);
         in.a = pf_proj_out(d, l, VX_PROJ_O, as_o);
         VX_TRY(stage(in, static_cast<uint32_t>(H), d->pf_ld[VX_PROJ_O], as_ffn));
-        VX_TRY(gemm_stage(H, {VX_PROJ_GATE, VX_PROJ_UP}));
-        {
-            // a staged gate/up pair as one launch when that needs no K split (twice the workgroups of one matrix)
-            const vx_matrix* mg = d->proj[l * kProjKinds + VX_PROJ_GATE];
-            const vx_matrix* mu = d->proj[l * kProjKinds + VX_PROJ_UP];
-            GemmSub gu[2] = {GemmSub{mg->d_w, &mg->g, d->pf_y[VX_PROJ_GATE], d->pf_ld[VX_PROJ_GATE]},
-                             GemmSub{mu->d_w, &mu->g, d->pf_y[VX_PROJ_UP], d->pf_ld[VX_PROJ_UP]}};
-            if (gemm_group_small_path(gu, 2, n, d->num_cus)) {
-                VX_TRY(launch_gemm_group(gu, 2, d->num_cus, d->pf_codes, n, d->pf_codes_ld, d->pf_part, st));
-            } else if (!small(VX_PROJ_GATE) && !small(VX_PROJ_UP) && d->pf_ld[VX_PROJ_GATE] == d->pf_ld[VX_PROJ_UP] &&
-                mg->g.rows == mu->g.rows && mg->g.cols == mu->g.cols && gemm_staged_pair_ok(mg->g, n, d->num_cus)) {
-                VX_TRY(launch_gemm_staged_pair(mg->d_w, mu->d_w, mg->g, d->num_cus, d->pf_staged, n,
-                                               d->pf_y[VX_PROJ_GATE], d->pf_y[VX_PROJ_UP], d->pf_ld[VX_PROJ_GATE], st));
-            } else {
-                VX_TRY(gemm(l, VX_PROJ_GATE));
-                VX_TRY(gemm(l, VX_PROJ_UP));
-            }
-        }
+        VX_TRY(gemm(l, 2));
         PfActArgs aa{};
         aa.yg = d->pf_y[VX_PROJ_GATE];
         aa.yu = d->pf_y[VX_PROJ_UP];
@@ -3475,8 +3440,7 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
         // the down input: the gated activation (sub-norm or none)
         in = stage_input(d, kInPlain, F, d->pf_act, nullptr, sub ? nw[VX_NORM_FFN_SUB] : nullptr);
         VX_TRY(stage(in, static_cast<uint32_t>(F), 0, as_down));
-        VX_TRY(gemm_stage(F, {VX_PROJ_DOWN}));
-        VX_TRY(gemm(l, VX_PROJ_DOWN));
+        VX_TRY(gemm(l, 3));
     }
     if (!head) return VX_OK;
     HeadArgs h{};

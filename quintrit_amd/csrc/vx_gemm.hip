@@ -18,18 +18,15 @@
 // (t4_bytes). The activation staging writes X in exactly this order, so A and B pair every weight with its
 // activation.
 //
-// Work split. A wave computes 64 weight rows (two 32-row blocks, one tile of the device layout) x T groups of 32
-// tokens over a range of K steps; the A fragments of a K step are decoded once and used for all T token groups. A
-// workgroup of W = 4 or 8 waves takes W consecutive tiles with the same tokens and K range, so the B fragments of a K
-// step are staged once per workgroup in LDS (double-buffered, the next step's loaded while this one is multiplied).
-// Long K is split into slices whose int32 partial sums a second kernel adds; the host picks T, W and the number of
-// slices (4-wave workgroups while the grid fits the CUs in one round: at M <= 128 and for the 3072-row shapes they are
-// 5-25 % faster than 8-wave ones; 23040 rows at M = 512 need the 8-wave form).
+// Two kernels: up to 32 tokens gemm_small_kernel (latency: all of a slice's weights in flight at once), beyond that
+// gemm_kernel (a tile of row blocks x token groups, pipelined). Long K is split into slices whose int32 partial sums a
+// second kernel adds.
 #include "vx_gemv_core.h"
 #include "vx_internal.h"
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace vx {
 
@@ -37,6 +34,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4g __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const u32x4g g_u4g;
+typedef u32x4g u32x4u __attribute__((aligned(1)));  // 16- and 4-byte loads at any address
+typedef uint32_t u32u __attribute__((aligned(1)));
 
 // t0..t3 of every byte as int8 in a dword (trits03_word: non-values give zero trits, pack.rs:41-58), built at compile
 // time; a workgroup copies it into its LDS table with loads.
@@ -52,15 +51,53 @@ constexpr uint32_t kZeroWord = 0x7d7d7d7du;  // four bytes of five zero trits
 // decode (column_activation_index, pack.rs:230-237). In a whole 160-trit block (ks < cols / 160) the step is the 160
 // activations of block ks and half hs covers byte-columns 16 hs .. 16 hs + 15: K block kb < 4 takes, for byte-column
 // 16 hs + 4 kb + d, its activations of planes 0..3, a(160 ks + 32 e + 16 hs + 4 kb + d), e = 0..3: dword kb of the
-// four 16-byte loads at 160 ks + 32 e + 16 hs, transposed 4 x 4 bytes with v_perm; K block 4 takes plane 4 of the 16
-// byte-columns, the 16 bytes at 160 ks + 128 + 16 hs as they are. The packed tail and unaligned rows take the
-// per-byte gather. Workgroup (pair block, token group): lane j of each 32-thread row is token 32 tg + j and the rows are
+// four 16-byte loads at 160 ks + 32 e + 16 hs (at any alignment), transposed 4 x 4 bytes with v_perm; K block 4 takes
+// plane 4 of the 16 byte-columns, the 16 bytes at 160 ks + 128 + 16 hs as they are. The packed tail takes the per-byte
+// gather. Workgroup (pair block, token group): lane j of each 32-thread row is token 32 tg + j and the rows are
 // kStageRows consecutive pairs, so the 32 tokens of a row write one contiguous 512-byte run per K block.
 constexpr uint32_t kStageRows = 8;  // pairs per staging workgroup (256 threads)
 
+// The five fragments of half hs of a whole block from its pieces X[e] = activations 32 e + 16 hs .. + 15 (plane e of the
+// 16 byte-columns): K block kb < 4 the 4 x 4 byte transpose of dword kb of planes 0..3, K block 4 plane 4 as it is.
+__device__ __forceinline__ void block_fragments(const u32x4g (&X)[5], u32x4g (&o)[5]) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+        auto dw = [&](const u32x4g& v) { return kb == 0 ? v.x : (kb == 1 ? v.y : (kb == 2 ? v.z : v.w)); };
+        const uint32_t a0 = dw(X[0]), a1 = dw(X[1]), a2 = dw(X[2]), a3 = dw(X[3]);
+        const uint32_t lo01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), hi01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+        const uint32_t lo23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), hi23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+        o[kb] = u32x4g{__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                           __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+    }
+    o[4] = X[4];
+}
+
+// The same for a half of the packed tail, X its 80 consecutive activations: byte-column k holds activations 5 k .. 5 k +
+// 4, so dword d of K block kb < 4 is the four bytes from 5 (4 kb + d) on, of K block 4 bytes 5 (4 d + e) + 4, e = 0..3.
+__device__ __forceinline__ void tail_fragments(const u32x4g (&X)[5], u32x4g (&o)[5]) {
+    const uint32_t D[21] = {X[0].x, X[0].y, X[0].z, X[0].w, X[1].x, X[1].y, X[1].z, X[1].w, X[2].x, X[2].y, X[2].z,
+                            X[2].w, X[3].x, X[3].y, X[3].z, X[3].w, X[4].x, X[4].y, X[4].z, X[4].w, 0u};
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+        uint32_t v[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int b = 20 * kb + 5 * d;
+            v[d] = __builtin_amdgcn_alignbyte(D[b / 4 + 1], D[b / 4], b % 4);
+        }
+        o[kb] = u32x4g{v[0], v[1], v[2], v[3]};
+    }
+    uint32_t v[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+        v[d] = __builtin_amdgcn_perm(D[5 * d + 2], D[5 * d + 1], 0x0c0c0500u) |
+               __builtin_amdgcn_perm(D[5 * d + 4], D[5 * d + 3], 0x07020c0cu);
+    o[4] = u32x4g{v[0], v[1], v[2], v[3]};
+}
+
 __global__ __launch_bounds__(256) void gemm_stage_kernel(const int8_t* __restrict__ x, uint32_t ldx, uint32_t n_tg,
                                                          uint32_t cols, uint32_t n_ksteps,
-                                                         uint4* __restrict__ xs, uint32_t M) {
+                                                         u32x4g* __restrict__ xs, uint32_t M) {
     const uint32_t tid = threadIdx.x, j = tid & 31u;
     const uint32_t pair = blockIdx.x * kStageRows + (tid >> 5), ks = pair >> 1, hs = pair & 1u;
     const uint32_t tg = blockIdx.y, m = tg * 32u + j;
@@ -68,22 +105,13 @@ __global__ __launch_bounds__(256) void gemm_stage_kernel(const int8_t* __restric
     // columns that are never stored.
     if (ks >= n_ksteps || m >= M) return;
     const int8_t* xr = x + static_cast<size_t>(m) * ldx;
-    uint4 o[5];
-    if (ks < cols / 160u && (reinterpret_cast<uintptr_t>(xr) & 15u) == 0) {
+    u32x4g o[5];
+    if (ks < cols / 160u) {
         const int8_t* blk = xr + ks * 160u + 16u * hs;
-        uint4 X[5];
+        u32x4g X[5];
 #pragma unroll
-        for (int e = 0; e < 5; ++e) X[e] = *reinterpret_cast<const uint4*>(blk + 32 * e);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            auto dw = [&](const uint4& v) { return kb == 0 ? v.x : (kb == 1 ? v.y : (kb == 2 ? v.z : v.w)); };
-            const uint32_t a0 = dw(X[0]), a1 = dw(X[1]), a2 = dw(X[2]), a3 = dw(X[3]);
-            const uint32_t lo01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), hi01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
-            const uint32_t lo23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), hi23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
-            o[kb] = make_uint4(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u));
-        }
-        o[4] = X[4];
+        for (int e = 0; e < 5; ++e) X[e] = *reinterpret_cast<const u32x4u*>(blk + 32 * e);
+        block_fragments(X, o);
     } else {
         // byte-column 16 hs + k of the step (k < 16), activation p: in a whole block 160 ks + 32 p + 16 hs + k, in the
         // packed tail 160 ks + 5 (16 hs + k) + p (column_activation_index); past the row (and in the tail's padding
@@ -103,7 +131,7 @@ __global__ __launch_bounds__(256) void gemm_stage_kernel(const int8_t* __restric
                 for (uint32_t e = 0; e < 4; ++e) v |= (kb < 4 ? act(4u * kb + d, e) : act(4u * d + e, 4u)) << (8 * e);
                 w[d] = v;
             }
-            o[kb] = make_uint4(w[0], w[1], w[2], w[3]);
+            o[kb] = u32x4g{w[0], w[1], w[2], w[3]};
         }
     }
 #pragma unroll
@@ -112,106 +140,179 @@ __global__ __launch_bounds__(256) void gemm_stage_kernel(const int8_t* __restric
 
 // ---- GEMM -------------------------------------------------------------------------------------------------------------
 
-struct GemmArgs {
-    const uint8_t* w;      // device layout
-    const uint4* xs;       // staged activations
-    int32_t* y;            // M x ldy (kslices == 1)
-    int32_t* part;         // kslices x (n_tg * 32) x rows_p partial sums (kslices > 1)
-    uint32_t rows, n_tiles, n_chunks, n_ksteps;
-    uint32_t M, n_tg, ldy, y_vec4;   // y_vec4: y and ldy allow 16-byte stores
-    uint32_t kslices, ksteps_per_slice, rows_p;
-    // a pair of matrices of one geometry in one launch (gemm_kernel's G2): the tiles of w (tiles1 of them), then those
-    // of w2 with outputs y2; n_tiles counts both
-    const uint8_t* w2;
-    int32_t* y2;
-    uint32_t tiles1;
+// One matrix of a call: up to kGemmSubs matrices with the same columns share a launch, their tiles (and 32-row blocks)
+// concatenated. Its tiles are tiles tile0 .. tile0 + n_tiles - 1 of the call, its rows rows row0 .. row0 + rows_p - 1 of
+// the slice sums.
+constexpr int kGemmSubs = 3;
+struct GemmMat {
+    const uint8_t* w;
+    int32_t* y;
+    uint32_t ldy, rows, rows_p, n_tiles, tile0, row0;
 };
 
-// Workgroup (rg, tt, kz): W waves, wave w taking the R 32-row blocks (W rg + w) R .. + R - 1 of the matrix (block 2 t + h
-// is half h of 64-row tile t), token groups T tt .. T tt + T - 1, K steps of slice kz. LDS: the trit table (32 copies
-// of each entry in the first half of a 256-byte row; lane l reads copy l % 32, conflict-free because LDS serves a wave
-// in two 32-lane halves) and two buffers of one K step's B fragments, which every wave reads (a B fragment serves the
-// wave's R blocks, an A fragment its T token groups).
-template <int T, int R, int W, bool G2>
-__global__ __launch_bounds__(W * 64) void gemm_kernel(GemmArgs a) {
-    __shared__ uint32_t tab[256 * 64];
-    __shared__ uint4 bs[2][5 * T * 64];
-    constexpr uint32_t kNT = W * 64u;
-    constexpr uint32_t kB = 5u * T * 64u;                // B fragments of a K step
-    constexpr uint32_t kBPer = (kB + kNT - 1) / kNT;     // per thread
-    static_assert(kBPer <= 5, "at most five B fragments per thread and step");
+struct GemmArgs {
+    GemmMat sub[kGemmSubs];
+    uint32_t n_sub;
+    const int8_t* x;     // raw activations, M rows of ldx
+    const u32x4g* xs;     // staged activations (gemm_kernel without RAW)
+    int32_t* part;       // [kslices][M][rows_p] slice sums (kslices > 1)
+    uint32_t ldx, rows_p, cols, n_tiles, n_chunks, n_ksteps, M, n_tg, kslices;  // rows_p, n_tiles: of all the matrices
+    uint32_t steps;      // K steps per slice
+    uint32_t n_rg, n_tt; // gemm_kernel: row groups of 4 R blocks, token tiles of T groups
+};
 
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+// More than 32 tokens. A workgroup of 4 waves takes 4 R consecutive 32-row blocks (wave w blocks R w .. R w + R - 1 of
+// them), T groups of 32 tokens and the K steps of a slice. The A fragments are decoded in registers, once for all T
+// groups, the B fragments of a K step are in LDS for all waves.
+//
+// Everything is pipelined in units of one K block (R T matrix products): while the products of K block kb run, the
+// wave looks up the trits and reads the B fragments of K block kb + 1 into the other of two register sets. The weights
+// are requested three K steps ahead, the activations of step k + 3 during step k and written to LDS as fragments a step
+// before their use (two buffers, one barrier per step, placed where the last reads of the step have been issued). With
+// 8-wave workgroups that decoded a whole K step behind the barrier before its products, the matrix pipe idled through
+// every decode. 2560 x 2560 x 512 tokens 30.4 -> 15.9 us per call, 23040 x 3072 x 128 38 -> 23.4, 6913 x 2563 x 100 35.8
+// -> 21.3, 23040 x 3072 x 512 56.9 -> 45.9 (1.58 POP/s; a plain int8 library product of 8192^3 reaches 2.1 on this card).
+//
+// What bounds it: instruction issue. A wave issues an instruction about every 7 cycles, matrix products included, and a
+// K step of one wave is 5 R T products of 32 cycles beside 16 R lookups with their addresses, 36 R byte operations for
+// plane 4, 5 T fragment reads and about 60 others: 1.26 us per step at R = 3, T = 4, of which 0.8 are products. At 512
+// tokens of 3072-column rows the output (47 MB) and the start of the call take as long as the rest.
+//
+// RAW (cols in whole 16-byte pieces, at any alignment): the workgroup builds the B fragments from x itself: lane (token,
+// half) loads the 80 activations of its half of the K step as five 16-byte pieces and transposes them (in a whole block
+// four 4 x 4 byte transposes, in the packed tail of the row, whose byte-columns hold five consecutive activations, byte
+// shifts). Pieces past the row read its last one: the weights there are zero trits; a chunk past the row, whose weights
+// repeat the last chunk's, gets zeros. Its scattered loads cost about 0.1 us per step more than those of fragments that
+// gemm_stage_kernel or the caller has written (xs), the staging launch 5 to 8 us per call (3072 x 3072 x 64 17 against
+// 12 us, 23040 x 3072 x 128 25.5 against 23.4).
+//
+// LDS: the trit table (row B: 32 copies of byte B's entry in the first 128 bytes of a 256-byte row; lane l reads copy
+// l % 32, conflict-free because LDS serves a wave in two 32-lane halves), and in the second halves of its rows the two
+// buffers of fragments, 8 rows of 128 bytes each: 80 KiB for four token groups, so that two workgroups fit a CU where
+// their registers do.
+//
+// Workgroups: the token tiles of a row group run on one XCD (blockIdx.x mod 8), so that its L2 serves their weights.
+template <int T, int R, bool RAW>
+__global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs a) {
+    constexpr uint32_t kFrags = 5u * T;                 // B fragments of a K step
+    constexpr uint32_t kXPer = RAW ? 5u : (kFrags + 3u) / 4u;  // 16-byte loads of activations per thread and step
+    constexpr uint32_t kXSets = 2u;  // sets of activations on the way to LDS
+    constexpr int kReads = 4 * R + T, kEarly = (R * T + 1) / 2;  // the LDS reads of a K block follow its first products
+    constexpr uint32_t kLdsRows = 2u * kFrags * 8u > 256u ? 2u * kFrags * 8u : 256u;
+    __shared__ __align__(256) uint32_t tab[kLdsRows * 64u];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, half = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t blk0 = (blockIdx.x * W + wave) * R;  // the wave's first 32-row block of the launch
-    // G2: the wave's matrix (its R blocks lie in one tile, so in one matrix) and its first block there
-    const bool sec = G2 && blk0 >= 2u * a.tiles1;
-    const uint32_t lb0 = sec ? blk0 - 2u * a.tiles1 : blk0;
-    const uint32_t nt = G2 ? a.tiles1 : a.n_tiles;  // tiles of the wave's matrix
-    const uint8_t* wm = sec ? a.w2 : a.w;
-    int32_t* ym = sec ? a.y2 : a.y;
-    const uint32_t n_blk = 2u * nt;
-    const uint32_t tt = blockIdx.y, kz = blockIdx.z;
-    const uint32_t ks0 = kz * a.ksteps_per_slice;
-    const uint32_t ks1 = min(ks0 + a.ksteps_per_slice, a.n_ksteps);
+    const uint32_t slot = blockIdx.x >> 3, tt = slot % a.n_tt, rg = (slot / a.n_tt) * 8u + (blockIdx.x & 7u);
+    if (rg >= a.n_rg) return;
+    const uint32_t kz = blockIdx.z, ks0 = kz * a.steps, ks1 = min(ks0 + a.steps, a.n_ksteps), last = ks1 - 1u;
+    const uint32_t blk0 = (rg * 4u + wave) * R, n_blk = 2u * a.n_tiles;
 
-    for (uint32_t i = tid; i < 256u * 8u; i += kNT) {
-        const uint32_t e = g_gemm_trits.v[i >> 3];
-        *reinterpret_cast<uint4*>(reinterpret_cast<char*>(tab) + (i >> 3) * 256u + (i & 7u) * 16u) = make_uint4(e, e, e, e);
-    }
-    const char* tabb = reinterpret_cast<const char*>(tab);
-    const uint32_t lane_off = (lane & 31u) * 4u;
-
-    // This lane's row (i = lane % 32) of each of the wave's blocks in the device layout: block 2 t + h is rows
-    // 32 h .. 32 h + 31 of tile t (16 bytes a row per chunk, the chunks of a tile T_g KiB apart in its tile group). A
-    // block past the matrix reads the last block (and stores nothing), so every load has a valid address and none sits
-    // behind a branch (the compiler would then wait for all loads before the next use).
-    const uint8_t* wbase[R];
+    // The wave's blocks: block 2 t + h is rows 32 h .. of tile t of its matrix (16 bytes a row per chunk, the chunks of a
+    // tile T_g KiB apart in its tile group). A block past the call reads the last one and stores nothing.
+    auto sub_of = [&](uint32_t tile) -> const GemmMat& {
+        return a.n_sub > 2u && tile >= a.sub[2].tile0 ? a.sub[2] : (a.n_sub > 1u && tile >= a.sub[1].tile0 ? a.sub[1] : a.sub[0]);
+    };
+    // Addresses are a scalar base, advanced by each load until the slice's last step, and a 32-bit lane offset. A chunk
+    // past the row (odd n_chunks) repeats the one before it: its activations are zero.
+    const uint8_t* wp[R];
     uint32_t cstride[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const uint32_t blk = min(lb0 + r, n_blk - 1u), tile = blk >> 1;
-        const uint32_t grp = tile / kTileGroup, t16 = tile - grp * kTileGroup;
-        const uint32_t Tg = min(static_cast<uint32_t>(kTileGroup), nt - grp * kTileGroup);
-        wbase[r] = wm + (static_cast<size_t>(grp) * kTileGroup * a.n_chunks + t16) * 1024u + (blk & 1u) * 512u +
-                   (lane & 31u) * 16u;
+        const uint32_t blk = min(blk0 + r, n_blk - 1u);
+        const GemmMat& sb = sub_of(blk >> 1);
+        const uint32_t tile = (blk >> 1) - sb.tile0, grp = tile / kTileGroup, t16 = tile - grp * kTileGroup;
+        const uint32_t Tg = min(static_cast<uint32_t>(kTileGroup), sb.n_tiles - grp * kTileGroup);
         cstride[r] = Tg * 1024u;
+        wp[r] = sb.w + (static_cast<size_t>(grp) * kTileGroup * a.n_chunks + t16) * 1024u + (blk & 1u) * 512u +
+                static_cast<size_t>(ks0 * kStepChunks) * cstride[r];
     }
-    const uint32_t half = lane >> 5;
-
-    // Chunk 2 ks + s of the lane's rows; a chunk past the row (odd n_chunks) reads the last one and is replaced by
-    // zero trits when it is decoded.
-    auto load_w = [&](uint32_t ks, u32x4g (&wv)[R]) __attribute__((always_inline)) {
-        const uint32_t q = min(ks * kStepChunks + half, a.n_chunks - 1u);
+    const uint32_t woff = (lane & 31u) * 16u;
+    auto load_w = [&](uint32_t ks, u32x4g (&wv)[R]) __attribute__((always_inline)) {  // step min(ks, last), in order
+        const bool two = min(ks, last) * kStepChunks + 1u < a.n_chunks;
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            wv[r] = __builtin_nontemporal_load((g_u4g*)(wbase[r] + static_cast<size_t>(q) * cstride[r]));
+        for (int r = 0; r < R; ++r) {
+            wv[r] = *(g_u4g*)(wp[r] + (woff + (two && half != 0 ? cstride[r] : 0u)));
+            wp[r] += ks < last ? kStepChunks * cstride[r] : 0u;
+        }
     };
-    // B fragments of step ks (kBPer per thread, in named registers: an array here would be moved to scratch memory
-    // once the steps rotate through three sets); slots past the token groups read a valid fragment that no stored
-    // output depends on (only C columns of tokens >= M).
-    auto b_index = [&](uint32_t ks, uint32_t k) -> size_t {
-        const uint32_t idx = min(tid + k * kNT, kB - 1u);
-        const uint32_t kb = idx / (T * 64u), rem = idx - kb * T * 64u;
-        const uint32_t tg = min(tt * T + rem / 64u, a.n_tg - 1u);
-        return (static_cast<size_t>(ks * 5u + kb) * a.n_tg + tg) * 64u + (rem & 63u);
+
+    char* const lds = reinterpret_cast<char*>(tab);
+    const uint32_t frag_lane = (lane >> 3) * 256u + 128u + (lane & 7u) * 16u;  // + 2048 per fragment
+    const auto frag_at = [&](uint32_t buf, uint32_t f) { return reinterpret_cast<u32x4g*>(lds + frag_lane + (buf * kFrags + f) * 2048u); };
+    // RAW: wave w < T builds the fragments of token group w, lane (j, hs) token j's half hs; the other waves load one
+    // address and store to spare fragments (a branch around loads would make every wait after it one for all loads).
+    // Otherwise the fragments f = kb T + g are copied, wave w those with f % 4 = w (one past the last
+    // repeats it, and one of a token group past M the last group's: it reaches outputs that are never stored).
+    static_assert(2u * kFrags + 5u * (4u - T) <= kLdsRows / 8u, "spare fragments of the waves without a token group");
+    const uint32_t hs = half, full = a.cols / 160u;
+    const uint32_t xrow_m = wave < T ? min((tt * T + wave) * 32u + (lane & 31u), a.M - 1u) : 0u;
+    const int8_t* xrow = a.x + static_cast<size_t>(xrow_m) * a.ldx;
+    const uint32_t xhs = wave < T ? hs : 0u;
+    const auto raw_frag = [&](uint32_t buf, uint32_t kb) {
+        return frag_at(0u, wave < T ? buf * kFrags + kb * T + wave : 2u * kFrags + (wave - T) * 5u + kb);
     };
-#define VX_LOAD_B(ks, r0, r1, r2, r3, r4)                   \
-    do {                                                    \
-        r0 = a.xs[b_index((ks), 0)];                        \
-        if (kBPer > 1) r1 = a.xs[b_index((ks), 1)];         \
-        if (kBPer > 2) r2 = a.xs[b_index((ks), 2)];         \
-        if (kBPer > 3) r3 = a.xs[b_index((ks), 3)];         \
-        if (kBPer > 4) r4 = a.xs[b_index((ks), 4)];         \
-    } while (0)
-#define VX_STORE_B(buf, r0, r1, r2, r3, r4)                                             \
-    do {                                                                                \
-        if (tid < kB) bs[(buf)][tid] = r0;                                              \
-        if (kBPer > 1 && tid + kNT < kB) bs[(buf)][tid + kNT] = r1;                     \
-        if (kBPer > 2 && tid + 2u * kNT < kB) bs[(buf)][tid + 2u * kNT] = r2;           \
-        if (kBPer > 3 && tid + 3u * kNT < kB) bs[(buf)][tid + 3u * kNT] = r3;           \
-        if (kBPer > 4 && tid + 4u * kNT < kB) bs[(buf)][tid + 4u * kNT] = r4;           \
-    } while (0)
+    const u32x4g* xp[kXPer];
+    if constexpr (!RAW) {
+#pragma unroll
+        for (uint32_t i = 0; i < kXPer; ++i) {
+            const uint32_t f = min(wave + 4u * i, kFrags - 1u);
+            xp[i] = a.xs + (static_cast<size_t>(ks0 * 5u + f / T) * a.n_tg + min(tt * T + f % T, a.n_tg - 1u)) * 64u;
+        }
+    }
+    const uint32_t xstep = 5u * a.n_tg * 64u;
+    u32x4g X[kXSets][kXPer];
+    auto load_x = [&](uint32_t ks, u32x4g (&x)[kXPer]) __attribute__((always_inline)) {  // step min(ks, last), in order
+        if constexpr (RAW) {
+            const uint32_t k = min(ks, last), base = k * 160u + xhs * (k < full ? 16u : 80u), step = k < full ? 32u : 16u;
+#pragma unroll
+            for (uint32_t i = 0; i < kXPer; ++i) x[i] = *reinterpret_cast<const u32x4u*>(xrow + min(base + i * step, a.cols - 16u));
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < kXPer; ++i) {
+                x[i] = *(g_u4g*)(xp[i] + lane);
+                xp[i] += ks < last ? xstep : 0u;
+            }
+        }
+    };
+    auto store_x = [&](uint32_t buf, const u32x4g (&x)[kXPer]) __attribute__((always_inline)) {
+        if constexpr (RAW) {
+            u32x4g o[5];
+            block_fragments(x, o);
+#pragma unroll
+            for (uint32_t kb = 0; kb < 5; ++kb) *raw_frag(buf, kb) = o[kb];
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < kXPer; ++i) *frag_at(buf, min(wave + 4u * i, kFrags - 1u)) = x[i];
+        }
+    };
+    // RAW: the fragments of step ks in the packed tail, written over what store_x made of them
+    auto store_tail = [&](uint32_t ks, uint32_t buf, const u32x4g (&x)[kXPer]) __attribute__((always_inline)) {
+        if constexpr (RAW) {
+            u32x4g o[5];
+            tail_fragments(x, o);
+            const bool none = ks * kStepChunks + hs >= a.n_chunks;
+#pragma unroll
+            for (uint32_t kb = 0; kb < 5; ++kb) *raw_frag(buf, kb) = none ? u32x4g{0u, 0u, 0u, 0u} : o[kb];
+        }
+    };
+    const uint32_t lane_off = (lane & 31u) * 4u;
+    // the A fragments of K block kb < 4: t0..t3 of the four bytes of dword kb
+    auto dword = [](const u32x4g& v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); };
+    auto decode = [&](int kb, const u32x4g (&w)[R], v4i (&A)[R]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            int t[4];
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                t[b] = *reinterpret_cast<const int*>(lds + __builtin_amdgcn_perm(dword(w[r], kb), lane_off, 0x0c0c0000u | ((4u + b) << 8)));
+            A[r] = v4i{t[0], t[1], t[2], t[3]};
+        }
+    };
+    auto read_b = [&](uint32_t kb, uint32_t buf, v4i (&B)[T]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t g = 0; g < T; ++g)
+            B[g] = *reinterpret_cast<const v4i*>(lds + frag_lane + (buf * kFrags + kb * T + g) * 2048u);
+    };
 
     v16i acc[R][T];
 #pragma unroll
@@ -219,107 +320,101 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(GemmArgs a) {
 #pragma unroll
         for (int g = 0; g < T; ++g) acc[r][g] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 
-    // The products of step ks: weights wc, B fragments from bs[buf].
-    auto multiply = [&](uint32_t ks, const u32x4g (&wc)[R], uint32_t buf) __attribute__((always_inline)) {
-        const bool inside = ks * kStepChunks + half < a.n_chunks;
-        v4i A[R][5];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint32_t dw[4] = {inside ? wc[r].x : kZeroWord, inside ? wc[r].y : kZeroWord,
-                                    inside ? wc[r].z : kZeroWord, inside ? wc[r].w : kZeroWord};
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                int t[4];
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const uint32_t addr = __builtin_amdgcn_perm(dw[m], lane_off, 0x0c0c0000u | ((4u + b) << 8));
-                    t[b] = static_cast<int>(*reinterpret_cast<const uint32_t*>(tabb + addr));
-                }
-                A[r][m] = v4i{t[0], t[1], t[2], t[3]};
-            }
-            A[r][4] = v4i{static_cast<int>(t4_bytes(dw[0])), static_cast<int>(t4_bytes(dw[1])),
-                          static_cast<int>(t4_bytes(dw[2])), static_cast<int>(t4_bytes(dw[3]))};
-        }
-        // K block outer, token group, then block: R T independent accumulators between two MFMAs on the same one.
-#pragma unroll
-        for (int kb = 0; kb < 5; ++kb) {
-#pragma unroll
-            for (int g = 0; g < T; ++g) {
-                const uint4 b = bs[buf][(kb * T + g) * 64u + lane];
-                const v4i B = v4i{static_cast<int>(b.x), static_cast<int>(b.y), static_cast<int>(b.z), static_cast<int>(b.w)};
-#pragma unroll
-                for (int r = 0; r < R; ++r) acc[r][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[r][kb], B, acc[r][g], 0, 0, 0);
-            }
-        }
-    };
-
-    // Two K steps ahead: step ks issues the loads of step ks + 2 (B fragments first, then weights), multiplies step ks
-    // (weights loaded two steps earlier, B fragments stored in LDS at the end of the previous step) and stores the B
-    // fragments of step ks + 1 (loaded one step earlier). Three register sets rotate through the steps of a 3x
-    // unrolled loop, so no loaded register is ever copied (a copy would wait for its load). Every load is unconditional
-    // (indices clamp at the last step) and the steps past the slice's end only skip the multiply, so the compiler's
-    // waits stay exact.
-    u32x4g w0[R], w1[R], w2[R];
-    uint4 b00, b01, b02, b03, b04, b10, b11, b12, b13, b14, b20, b21, b22, b23, b24;
-    const uint32_t last = ks1 > ks0 ? ks1 - 1u : ks0;
-    VX_LOAD_B(ks0, b00, b01, b02, b03, b04);
-    load_w(ks0, w0);
-    VX_LOAD_B(min(ks0 + 1u, last), b10, b11, b12, b13, b14);
-    load_w(min(ks0 + 1u, last), w1);
-    VX_STORE_B(0, b00, b01, b02, b03, b04);
-    const bool active = blk0 < 2u * a.n_tiles;
-#define VX_STEP(ks, WC, N0, N1, N2, N3, N4, M0, M1, M2, M3, M4, WN)      \
-    do {                                                                 \
-        VX_LOAD_B(min((ks) + 2u, last), M0, M1, M2, M3, M4);             \
-        load_w(min((ks) + 2u, last), WN);                                \
-        __syncthreads();                                                 \
-        if (active && (ks) < ks1) multiply((ks), WC, ((ks) - ks0) & 1u); \
-        VX_STORE_B((((ks) - ks0) & 1u) ^ 1u, N0, N1, N2, N3, N4);        \
-    } while (0)
-    for (uint32_t ks = ks0; ks < ks1; ks += 3u) {
-        VX_STEP(ks, w0, b10, b11, b12, b13, b14, b20, b21, b22, b23, b24, w2);
-        VX_STEP(ks + 1u, w1, b20, b21, b22, b23, b24, b00, b01, b02, b03, b04, w0);
-        VX_STEP(ks + 2u, w2, b00, b01, b02, b03, b04, b10, b11, b12, b13, b14, w1);
+    u32x4g w[4][R];
+    v4i A[2][R], A4[R], B[2][T];
+    load_x(ks0, X[0]);
+    load_w(ks0, w[0]);
+    if constexpr (kXSets > 1) load_x(ks0 + 1u, X[1 % kXSets]);
+    load_w(ks0 + 1u, w[1]);
+    load_w(ks0 + 2u, w[2]);
+    for (uint32_t i = tid; i < 256u * 8u; i += 256u) {
+        const uint32_t e = g_gemm_trits.v[i >> 3];
+        *reinterpret_cast<uint4*>(lds + (i >> 3) * 256u + (i & 7u) * 16u) = make_uint4(e, e, e, e);
     }
-#undef VX_STEP
-#undef VX_LOAD_B
-#undef VX_STORE_B
-    if (!active) return;
-    // C of (block, token group g): lane l, register r -> row 8 (r / 4) + 4 (l / 32) + r % 4 of the block, token l % 32.
-    const uint32_t j = lane & 31u;
-#pragma unroll
-    for (int g = 0; g < T; ++g) {
-        const uint32_t m = (tt * T + g) * 32u + j;
-        if (m >= a.M) continue;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (lb0 + r >= n_blk) continue;
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const uint32_t n = (lb0 + r) * 32u + 8u * r4 + 4u * half;
-                const int v0 = acc[r][g][4 * r4], v1 = acc[r][g][4 * r4 + 1];
-                const int v2 = acc[r][g][4 * r4 + 2], v3 = acc[r][g][4 * r4 + 3];
-                if (a.kslices > 1) {
-                    *reinterpret_cast<int4*>(a.part + (static_cast<size_t>(kz) * a.n_tg * 32u + m) * a.rows_p + n) =
-                        make_int4(v0, v1, v2, v3);
-                } else if (a.y_vec4 && n + 3 < a.rows) {
-                    *reinterpret_cast<int4*>(ym + static_cast<size_t>(m) * a.ldy + n) = make_int4(v0, v1, v2, v3);
-                } else {
-                    int32_t* yr = ym + static_cast<size_t>(m) * a.ldy;
-                    if (n < a.rows) yr[n] = v0;
-                    if (n + 1 < a.rows) yr[n + 1] = v1;
-                    if (n + 2 < a.rows) yr[n + 2] = v2;
-                    if (n + 3 < a.rows) yr[n + 3] = v3;
-                }
+    store_x(0, X[0]);
+    if (RAW && ks0 >= full) store_tail(ks0, 0, X[0]);
+    load_x(ks0 + kXSets, X[0]);
+    __syncthreads();
+    decode(0, w[0], A[0]);
+    read_b(0, 0, B[0]);
+
+    // Step ks = ks0 + s (mod 4), with weights w[s], fragments in buffer s & 1. The loads are unconditional (indices clamp
+    // at the last step) and the loop has no other exit, so that every wait is for its own load.
+    auto step = [&](auto sc, uint32_t ks) __attribute__((always_inline)) {
+        constexpr uint32_t s = decltype(sc)::value, buf = s & 1u;
+        static_for<5>([&](auto kc) __attribute__((always_inline)) {
+            constexpr uint32_t kb = decltype(kc)::value, cur = (s + kb) & 1u, nxt = cur ^ 1u;
+            if constexpr (kb == 0) load_w(ks + 3u, w[(s + 3u) & 3u]);
+            if constexpr (kb == 2) store_x(buf ^ 1u, X[(s + 1u) % kXSets]);
+            if constexpr (kb == 3) {
+                if (RAW && ks + 1u >= full && ks + 1u < ks1) store_tail(ks + 1u, buf ^ 1u, X[(s + 1u) % kXSets]);
+                load_x(ks + 1u + kXSets, X[(s + 1u) % kXSets]);
             }
-        }
+            if constexpr (kb < 4) {
+                if constexpr (kb < 3) decode(kb + 1, w[s], A[nxt]);
+#pragma unroll
+                for (int r = 0; r < R; ++r) A4[r][kb] = static_cast<int>(t4_bytes(dword(w[s][r], kb)));
+                read_b(kb + 1u, buf, B[nxt]);
+            } else {
+                __syncthreads();  // the fragments of step ks + 1 are complete, every read of step ks has been made
+                decode(0, w[(s + 1u) & 3u], A[nxt]);
+                read_b(0, buf ^ 1u, B[nxt]);
+            }
+#pragma unroll
+            for (int g = 0; g < T; ++g)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    acc[r][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B[cur][g], kb < 4 ? A[cur][r] : A4[r], acc[r][g], 0, 0, 0);
+            // a product, then reads of the next K block and other instructions in its shadow, and nothing of a K block
+            // moved into another
+#pragma unroll
+            for (int i = 0; i < R * T; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                if (i < kEarly) __builtin_amdgcn_sched_group_barrier(0x100, (kReads + kEarly - 1) / kEarly, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    uint32_t ks = ks0;
+    for (; ks + 4u <= ks1; ks += 4u) static_for<4>([&](auto sc) __attribute__((always_inline)) { step(sc, ks + sc); });
+    if (ks < ks1) step(std::integral_constant<uint32_t, 0>{}, ks);
+    if (ks + 1u < ks1) step(std::integral_constant<uint32_t, 1>{}, ks + 1u);
+    if (ks + 2u < ks1) step(std::integral_constant<uint32_t, 2>{}, ks + 2u);
+
+    // The product is taken transposed (activations as the first operand): lane l holds row l % 32 of the block and, in
+    // register r, token 8 (r / 4) + 4 (l / 32) + r % 4 of the group, so that a store writes 128 consecutive bytes of two
+    // tokens. (With the tokens in the lanes each 16-byte store went to a line of its own.)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t blk = blk0 + r;
+        if (blk >= n_blk) break;
+        const GemmMat& sb = sub_of(blk >> 1);
+        const uint32_t n = blk * 32u - sb.tile0 * 64u + (lane & 31u);
+        const bool slices = a.kslices > 1u;
+        const uint32_t ld = slices ? a.rows_p : sb.ldy;
+        int32_t* out = slices ? a.part + static_cast<size_t>(kz) * a.M * a.rows_p + sb.row0 : sb.y;
+        if (!slices && n >= sb.rows) continue;
+#pragma unroll
+        for (int g = 0; g < T; ++g)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t m = (tt * T + g) * 32u + 8u * (e / 4) + 4u * half + (e % 4);
+                if (m < a.M) out[static_cast<size_t>(m) * ld + n] = acc[r][g][e];
+            }
     }
 }
 
+// Y[m][n] = sum over the slices of their sums (block = 256 rows of the call's slice sums, one token).
+template <bool G>
 __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs a) {
     const uint32_t n = blockIdx.x * 256u + threadIdx.x, m = blockIdx.y;
-    if (n >= a.rows) return;
-    const size_t stride = static_cast<size_t>(a.n_tg) * 32u * a.rows_p;
+    const uint32_t j = !G ? 0u : (a.n_sub > 1u && n >= a.sub[1].row0 ? 1u : 0u) + (a.n_sub > 2u && n >= a.sub[2].row0 ? 1u : 0u);
+    const GemmMat sb = j == 0u ? a.sub[0] : (j == 1u ? a.sub[1] : a.sub[2]);  // no indexing of the arguments
+    const uint32_t ln = n - sb.row0;
+    if (n >= a.rows_p || ln >= sb.rows) return;
+    const size_t stride = static_cast<size_t>(a.M) * a.rows_p;
     const int32_t* p = a.part + static_cast<size_t>(m) * a.rows_p + n;
     int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
     uint32_t k = 0;
@@ -330,165 +425,13 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs a) {
         s3 += p[(k + 3) * stride];
     }
     for (; k < a.kslices; ++k) s0 += p[k * stride];
-    a.y[static_cast<size_t>(m) * a.ldy + n] = (s0 + s1) + (s2 + s3);
-}
-
-// ---- host side ---------------------------------------------------------------------------------------------------------
-
-struct GemmPlan {
-    uint32_t n_ksteps, n_tg, T, R, W, n_tt, grid_x, kslices, ksteps_per_slice;
-    size_t xs_bytes, part_bytes;
-};
-
-// T (token groups per wave) from M; then the K split that minimises an estimate of the time: rounds of workgroups
-// times K steps per workgroup times the time of a K step, plus the HBM traffic of the partial sums and their finish.
-// A K step of a wave is 10 T MFMAs (32 cycles each, two waves per SIMD), but not less than the HBM latency (the
-// weights are loaded one step ahead).
-static GemmPlan gemm_plan(const Geometry& g, size_t M, int num_cus) {
-    GemmPlan p{};
-    p.n_ksteps = static_cast<uint32_t>((g.n_chunks + kStepChunks - 1) / kStepChunks);
-    p.n_tg = static_cast<uint32_t>((M + 31) / 32);
-    p.T = p.n_tg >= 4 ? 4u : (p.n_tg >= 2 ? 2u : 1u);
-    p.n_tt = (p.n_tg + p.T - 1) / p.T;
-    // Two 32-row blocks per wave; 4-wave workgroups while they fit the CUs in one round without a K split (more,
-    // smaller workgroups spread a narrow grid over more CUs), else 8-wave workgroups (the B fragments of a step serve
-    // twice the rows).
-    p.R = 2;
-    const uint64_t blocks = 2 * g.n_tiles;
-    p.W = (blocks + 7) / 8 * p.n_tt <= static_cast<uint64_t>(std::max(num_cus, 1)) ? 4u : 8u;
-    p.grid_x = static_cast<uint32_t>((blocks + p.R * p.W - 1) / (p.R * p.W));
-    const uint64_t base = static_cast<uint64_t>(p.grid_x) * p.n_tt;
-    const uint64_t slots = static_cast<uint64_t>(std::max(num_cus, 1)) * (p.T == 1 ? 2u : 1u);  // workgroups per CU (LDS)
-    // a K step of a wave is 10 T MFMAs (32 cycles each, W / 4 waves per SIMD), but not less than the HBM latency
-    const double t_step = std::max(0.29e-6 * p.T * p.W / 8.0, 1.0e-6);
-    double best = 1e30;
-    uint32_t best_ks = 1;
-    for (uint32_t ks = 1; ks <= std::min<uint32_t>(p.n_ksteps, 64u); ++ks) {
-        const uint32_t per = (p.n_ksteps + ks - 1) / ks;
-        const uint32_t slices = (p.n_ksteps + per - 1) / per;
-        if (slices != ks) continue;
-        const double rounds = static_cast<double>((base * slices + slots - 1) / slots);
-        const double part = slices > 1 ? 8.0 * slices * static_cast<double>(M) * g.padded_rows / 2.5e12 + 4.0e-6 : 0.0;
-        const double t = rounds * per * t_step + part;
-        if (t < best) {
-            best = t;
-            best_ks = slices;
-        }
-    }
-    p.ksteps_per_slice = (p.n_ksteps + best_ks - 1) / best_ks;
-    p.kslices = (p.n_ksteps + p.ksteps_per_slice - 1) / p.ksteps_per_slice;
-    p.xs_bytes = round_up(static_cast<size_t>(p.n_ksteps) * 5u * p.n_tg * 1024u, 256);
-    p.part_bytes = p.kslices > 1 ? static_cast<size_t>(p.kslices) * p.n_tg * 32u * g.padded_rows * 4u : 0;
-    return p;
-}
-
-static size_t small_part_bytes(const Geometry& g, size_t M, int num_cus);
-static bool small_path(const Geometry& g, size_t M, int num_cus);
-
-size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus) {
-    if (small_path(g, M, num_cus)) return std::max<size_t>(small_part_bytes(g, M, num_cus), 256);
-    const GemmPlan p = gemm_plan(g, M, num_cus);
-    return p.xs_bytes + p.part_bytes;
-}
-
-size_t gemm_stage_bytes(size_t cols, size_t M) {
-    const GemmPlan p = gemm_plan(geometry(1, cols), M, 1);  // the staged activations depend on cols and M only
-    return p.xs_bytes;
-}
-
-size_t gemm_part_bytes(const Geometry& g, size_t M, int num_cus) {
-    return small_path(g, M, num_cus) ? small_part_bytes(g, M, num_cus) : gemm_plan(g, M, num_cus).part_bytes;
-}
-
-// Stages x (M rows of cols int8) into the MFMA operand order at ws (gemm_stage_bytes(cols, M) bytes): the staged
-// activations of one call serve every matrix with cols columns.
-int launch_gemm_stage(const int8_t* x, size_t M, size_t ldx, size_t cols, uint8_t* ws, hipStream_t stream) {
-    const GemmPlan p = gemm_plan(geometry(1, cols), M, 1);
-    const dim3 grid((2u * p.n_ksteps + kStageRows - 1) / kStageRows, p.n_tg);
-    hipLaunchKernelGGL(gemm_stage_kernel, grid, dim3(256), 0, stream, x, static_cast<uint32_t>(ldx), p.n_tg,
-                       static_cast<uint32_t>(cols), p.n_ksteps,
-                       reinterpret_cast<uint4*>(ws), static_cast<uint32_t>(M));
-    VX_HIP(hipGetLastError());
-    return VX_OK;
-}
-
-// The product of matrix w with activations staged by launch_gemm_stage at `staged`; `part` holds
-// gemm_part_bytes(g, M, num_cus) bytes of K-slice partial sums (unused when the plan has one slice).
-template <bool G2>
-static void launch_staged_kernel(const GemmPlan& p, const GemmArgs& a, hipStream_t stream) {
-    const dim3 grid(p.grid_x, p.n_tt, p.kslices);
-    const dim3 block(p.W * 64);
-    if (p.W == 8) {
-        if (p.T == 4) hipLaunchKernelGGL((gemm_kernel<4, 2, 8, G2>), grid, block, 0, stream, a);
-        else if (p.T == 2) hipLaunchKernelGGL((gemm_kernel<2, 2, 8, G2>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_kernel<1, 2, 8, G2>), grid, block, 0, stream, a);
-    } else {
-        if (p.T == 4) hipLaunchKernelGGL((gemm_kernel<4, 2, 4, G2>), grid, block, 0, stream, a);
-        else if (p.T == 2) hipLaunchKernelGGL((gemm_kernel<2, 2, 4, G2>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_kernel<1, 2, 4, G2>), grid, block, 0, stream, a);
-    }
-}
-
-static GemmArgs staged_args(const GemmPlan& p, const uint8_t* w, const Geometry& g, const uint8_t* staged, size_t M,
-                            int32_t* y, size_t ldy, uint8_t* part) {
-    GemmArgs a{};
-    a.w = w;
-    a.xs = reinterpret_cast<const uint4*>(staged);
-    a.y = y;
-    a.part = p.kslices > 1 ? reinterpret_cast<int32_t*>(part) : nullptr;
-    a.rows = static_cast<uint32_t>(g.rows);
-    a.n_tiles = static_cast<uint32_t>(g.n_tiles);
-    a.n_chunks = static_cast<uint32_t>(g.n_chunks);
-    a.n_ksteps = p.n_ksteps;
-    a.M = static_cast<uint32_t>(M);
-    a.n_tg = p.n_tg;
-    a.ldy = static_cast<uint32_t>(ldy);
-    a.y_vec4 = (ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0) ? 1u : 0u;
-    a.kslices = p.kslices;
-    a.ksteps_per_slice = p.ksteps_per_slice;
-    a.rows_p = static_cast<uint32_t>(g.padded_rows);
-    return a;
-}
-
-int launch_gemm_staged(const uint8_t* w, const Geometry& g, int num_cus, const uint8_t* staged, size_t M, int32_t* y,
-                       size_t ldy, uint8_t* part, hipStream_t stream) {
-    const GemmPlan p = gemm_plan(g, M, num_cus);
-    const GemmArgs a = staged_args(p, w, g, staged, M, y, ldy, part);
-    launch_staged_kernel<false>(p, a, stream);
-    VX_HIP(hipGetLastError());
-    if (p.kslices > 1) {
-        hipLaunchKernelGGL(gemm_finish_kernel, dim3((a.rows + 255u) / 256u, static_cast<uint32_t>(M)), dim3(256), 0, stream, a);
-        VX_HIP(hipGetLastError());
-    }
-    return VX_OK;
-}
-
-// The concatenation of two matrices of one geometry as one launch, when its plan needs no K split.
-static GemmPlan pair_plan(const Geometry& g, size_t M, int num_cus) {
-    return gemm_plan(geometry(2 * g.padded_rows, g.cols), M, num_cus);
-}
-
-bool gemm_staged_pair_ok(const Geometry& g, size_t M, int num_cus) { return pair_plan(g, M, num_cus).kslices == 1; }
-
-int launch_gemm_staged_pair(const uint8_t* w, const uint8_t* w2, const Geometry& g, int num_cus, const uint8_t* staged,
-                            size_t M, int32_t* y, int32_t* y2, size_t ldy, hipStream_t stream) {
-    const GemmPlan p = pair_plan(g, M, num_cus);
-    if (p.kslices != 1) VX_FAIL(VX_ERR_INTERNAL, "a paired GEMM with %u K slices", p.kslices);
-    GemmArgs a = staged_args(p, w, g, staged, M, y, ldy, nullptr);
-    a.n_tiles = static_cast<uint32_t>(2 * g.n_tiles);
-    a.w2 = w2;
-    a.y2 = y2;
-    a.tiles1 = static_cast<uint32_t>(g.n_tiles);
-    a.y_vec4 = a.y_vec4 && reinterpret_cast<uintptr_t>(y2) % 16 == 0 ? 1u : 0u;
-    launch_staged_kernel<true>(p, a, stream);
-    VX_HIP(hipGetLastError());
-    return VX_OK;
+    sb.y[static_cast<size_t>(m) * sb.ldy + ln] = (s0 + s1) + (s2 + s3);
 }
 
 // ---- one token group (M <= 32): one launch ------------------------------------------------------------------------
 
 // Workgroup (c, kz): W waves, wave w the 64-row tile W c + w, over the K steps of slice kz (at most
-// small_max_steps(T)), for T token groups of 32 (1, 2 or 4). G: the call's tiles may belong to several matrices of the
+// kSmallSteps), for one group of 32 tokens. G: the call's tiles may belong to several matrices of the
 // same columns (each wave finds its own; without G the instance reads only the first). Each thread first loads the activations of its B-fragment tasks (task = step, token
 // group, half, token) and the trit table's entries, then each wave loads all its weights of the slice at once (2
 // chunks per K step per lane, every load unconditional: steps past the slice read its last step again), so
@@ -501,31 +444,10 @@ int launch_gemm_staged_pair(const uint8_t* w, const uint8_t* w2, const Geometry&
 // at M = 8-32.)
 constexpr uint32_t kSmallSteps = 8;  // K steps per slice at most (40 KiB of B fragments per token group in LDS)
 
-// K steps per slice at most for T token groups: the B fragments stay within 80 KiB of LDS (the table takes 64 KiB).
-constexpr uint32_t small_max_steps(int T) { return T <= 2 ? kSmallSteps : kSmallSteps / 2; }
-
-// One matrix of a small-path call (up to kSmallSubs matrices with the same columns share a launch): its tiles are
-// tiles tile0 .. tile0 + n_tiles - 1 of the call, its rows rows row0 .. row0 + rows_p - 1 of the slice sums.
-constexpr int kSmallSubs = 3;
-struct SmallSub {
-    const uint8_t* w;
-    int32_t* y;
-    uint32_t ldy, rows, rows_p, n_tiles, tile0, row0;
-};
-
-struct SmallArgs {
-    SmallSub sub[kSmallSubs];
-    uint32_t n_sub;
-    const int8_t* x;
-    int32_t* part;       // [kslices][M][rows_p] slice sums (kslices > 1)
-    uint32_t ldx, rows_p, cols, n_tiles, n_chunks, n_ksteps, M, kslices;  // rows_p, n_tiles: of all the matrices
-    uint32_t steps;      // K steps per slice (at most small_max_steps(T))
-};
-
-template <int T, int W, bool G>
-__global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
+template <int W, bool G>
+__global__ __launch_bounds__(W * 64) void gemm_small_kernel(GemmArgs a) {
     __shared__ uint32_t tab[256 * 64];
-    constexpr uint32_t S = small_max_steps(T);
+    constexpr uint32_t S = kSmallSteps, T = 1;
     __shared__ uint4 bs[S * 5 * T * 64];
     constexpr uint32_t kTasks = S * T / W;  // B-fragment tasks per thread
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -533,19 +455,19 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
     const uint32_t tile = blockIdx.x * W + wave, kz = blockIdx.y;
     // the wave's matrix (wave-uniform) and its tile there (a tile past the call's tiles falls in the last matrix)
     const uint32_t j = !G ? 0u : (a.n_sub > 1u && tile >= a.sub[1].tile0 ? 1u : 0u) + (a.n_sub > 2u && tile >= a.sub[2].tile0 ? 1u : 0u);
-    const SmallSub sb = j == 0u ? a.sub[0] : (j == 1u ? a.sub[1] : a.sub[2]);
+    const GemmMat sb = j == 0u ? a.sub[0] : (j == 1u ? a.sub[1] : a.sub[2]);
     const uint32_t lt = tile - sb.tile0;
     const uint32_t ks0 = kz * a.steps, nst = min(a.steps, a.n_ksteps - ks0);
     const uint32_t half = lane >> 5;
 
     // The activations of this thread's tasks, loaded before the weights with every load at a valid address (no
     // branch that depends on the thread separates them from the weight loads, and nothing waits for them before the
-    // weights are requested). When every row of x is 16-byte aligned: a whole 160-column block as 5 uint4 (kind 1);
+    // weights are requested). With a block in the row: a whole 160-column block as 5 uint4 (kind 1);
     // when the slice's last step is the partial last block, its task (one per thread, a task holding W / T steps) as
     // the 80 columns of its half (kind 2). Other tasks are read by bytes after the weight loads (kind 0).
-    const bool aligned = ((reinterpret_cast<uintptr_t>(a.x) | a.ldx) & 15u) == 0 && a.cols >= 160u;  // x holds a block
+    const bool blocks = a.cols >= 160u;  // x holds a block (its rows may have any alignment)
     const bool has_tail = a.cols % 160u != 0u && ks0 + nst == a.n_ksteps;
-    uint4 X[kTasks][5];
+    u32x4g X[kTasks][5];
     uint32_t kind[kTasks];
 #pragma unroll
     for (uint32_t r = 0; r < kTasks; ++r) {
@@ -553,11 +475,11 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
         const uint32_t s = t / (64u * T), rr = t - s * 64u * T, tok = 32u * (rr >> 6) + (rr & 31u), ks = ks0 + s;
         const uint32_t hs = (rr >> 5) & 1u;
         const bool live = s < nst && tok < a.M;
-        kind[r] = !live || !aligned ? 0u : (ks < a.cols / 160u ? 1u : 2u);
-        if (aligned) {
+        kind[r] = !live || !blocks ? 0u : (ks < a.cols / 160u ? 1u : 2u);
+        if (blocks) {
             const int8_t* blk = (kind[r] == 1u ? a.x + static_cast<size_t>(tok) * a.ldx + ks * 160u : a.x) + 16u * hs;
 #pragma unroll
-            for (int e = 0; e < 5; ++e) X[r][e] = *reinterpret_cast<const uint4*>(blk + 32 * e);
+            for (int e = 0; e < 5; ++e) X[r][e] = *reinterpret_cast<const u32x4u*>(blk + 32 * e);
         }
     }
     // kind 2, raw: the words at clamped addresses and the bytes of the word that straddles cols (masked where used).
@@ -565,14 +487,14 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
     // no branch joins them before the weight loads.
     uint32_t V[20], tb[3];
     {
-        const bool use = has_tail && aligned;
+        const bool use = has_tail && blocks;
         const uint32_t t = tid + (nst - 1u) * T / W * W * 64u;
         const uint32_t s = t / (64u * T), rr = t - s * 64u * T, tok = 32u * (rr >> 6) + (rr & 31u), hs = (rr >> 5) & 1u;
         const int8_t* row = use ? a.x + static_cast<size_t>(tok < a.M ? tok : 0u) * a.ldx : reinterpret_cast<const int8_t*>(sb.w);
         const uint32_t base = use ? (a.n_ksteps - 1u) * 160u + 80u * hs : 0u, lastw = use ? (a.cols - 4u) & ~3u : 0u;
         const uint32_t i0 = use ? a.cols & ~3u : 0u, lastb = use ? a.cols - 1u : 0u;
 #pragma unroll
-        for (uint32_t d = 0; d < 20; ++d) V[d] = *reinterpret_cast<const uint32_t*>(row + min(base + 4u * d, lastw));
+        for (uint32_t d = 0; d < 20; ++d) V[d] = *reinterpret_cast<const u32u*>(row + min(base + 4u * d, lastw));
 #pragma unroll
         for (uint32_t e = 0; e < 3; ++e) tb[e] = static_cast<uint8_t>(row[min(i0 + e, lastb)]);
     }
@@ -614,14 +536,14 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
         if (kind[r] == 1u) {
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
-                auto dw = [&](const uint4& v) { return kb == 0 ? v.x : (kb == 1 ? v.y : (kb == 2 ? v.z : v.w)); };
+                auto dw = [&](const u32x4g& v) { return kb == 0 ? v.x : (kb == 1 ? v.y : (kb == 2 ? v.z : v.w)); };
                 const uint32_t a0 = dw(X[r][0]), a1 = dw(X[r][1]), a2 = dw(X[r][2]), a3 = dw(X[r][3]);
                 const uint32_t lo01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), hi01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
                 const uint32_t lo23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), hi23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
                 o[kb] = make_uint4(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
                                    __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u));
             }
-            o[4] = X[r][4];
+            o[4] = make_uint4(X[r][4].x, X[r][4].y, X[r][4].z, X[r][4].w);
         } else if (kind[r] == 2u) {
             // column ks * 160 + 80 hs + 5 k + p of the partial block is byte 5 k + p of the 80 loaded
             const uint32_t base = ks * 160u + 80u * hs, i0 = a.cols & ~3u;
@@ -703,81 +625,49 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(SmallArgs a) {
             for (int g = 0; g < T; ++g) {
                 const uint4 b = bs[((s * 5u + kb) * T + g) * 64u + lane];
                 const v4i B = v4i{static_cast<int>(b.x), static_cast<int>(b.y), static_cast<int>(b.z), static_cast<int>(b.w)};
-                acc[0][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0][kb], B, acc[0][g], 0, 0, 0);
-                acc[1][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[1][kb], B, acc[1][g], 0, 0, 0);
+                acc[0][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B, A[0][kb], acc[0][g], 0, 0, 0);
+                acc[1][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B, A[1][kb], acc[1][g], 0, 0, 0);
             }
         }
     }
-    // C of (block rb, token group g): lane l, register r -> row 8 (r / 4) + 4 (l / 32) + r % 4 of the block, token
-    // 32 g + l % 32
+    // The product is transposed as gemm_kernel's: lane l holds row l % 32 of block rb and, in register r, token 8 (r / 4) +
+    // 4 (l / 32) + r % 4, so that a store writes 128 consecutive bytes of two tokens.
+    int32_t* out = a.kslices == 1 ? sb.y : a.part + static_cast<size_t>(kz) * a.M * a.rows_p + sb.row0;
+    const uint32_t ld = a.kslices == 1 ? sb.ldy : a.rows_p;
 #pragma unroll
-    for (int g = 0; g < T; ++g) {
-        const uint32_t m = 32u * g + (lane & 31u);
-        if (m >= a.M) continue;
-        if (a.kslices == 1) {
+    for (int rb = 0; rb < 2; ++rb) {
+        const uint32_t n = lt * 64u + rb * 32u + (lane & 31u);
+        if (a.kslices == 1 && n >= sb.rows) continue;
 #pragma unroll
-            for (int rb = 0; rb < 2; ++rb)
+        for (int r4 = 0; r4 < 4; ++r4) {
+            if (8u * r4 >= a.M) break;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t n = lt * 64u + rb * 32u + 8u * (r / 4) + 4u * half + (r % 4);
-                    if (n < sb.rows) sb.y[static_cast<size_t>(m) * sb.ldy + n] = acc[rb][g][r];
-                }
-        } else {  // the slice's sums; gemm_small_finish_kernel adds the slices
-            int32_t* pp = a.part + (static_cast<size_t>(kz) * a.M + m) * a.rows_p + sb.row0 + lt * 64u;
-#pragma unroll
-            for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4)
-                    *reinterpret_cast<int4*>(pp + rb * 32u + 8u * r4 + 4u * half) =
-                        make_int4(acc[rb][g][4 * r4], acc[rb][g][4 * r4 + 1], acc[rb][g][4 * r4 + 2], acc[rb][g][4 * r4 + 3]);
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t m = 8u * r4 + 4u * half + e;
+                if (m < a.M) out[static_cast<size_t>(m) * ld + n] = acc[rb][0][4 * r4 + e];
+            }
         }
     }
 }
 
-// Y[m][n] = sum over the slices of gemm_small_kernel's sums (block = 256 rows of the call's slice sums, one token).
-template <bool G>
-__global__ __launch_bounds__(256) void gemm_small_finish_kernel(SmallArgs a) {
-    const uint32_t n = blockIdx.x * 256u + threadIdx.x, m = blockIdx.y;
-    const uint32_t j = !G ? 0u : (a.n_sub > 1u && n >= a.sub[1].row0 ? 1u : 0u) + (a.n_sub > 2u && n >= a.sub[2].row0 ? 1u : 0u);
-    const SmallSub sb = j == 0u ? a.sub[0] : (j == 1u ? a.sub[1] : a.sub[2]);  // no indexing of the arguments
-    const uint32_t ln = n - sb.row0;
-    if (n >= a.rows_p || ln >= sb.rows) return;
-    const size_t stride = static_cast<size_t>(a.M) * a.rows_p;
-    const int32_t* p = a.part + static_cast<size_t>(m) * a.rows_p + n;
-    int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-    uint32_t k = 0;
-    for (; k + 4 <= a.kslices; k += 4) {
-        s0 += p[k * stride];
-        s1 += p[(k + 1) * stride];
-        s2 += p[(k + 2) * stride];
-        s3 += p[(k + 3) * stride];
-    }
-    for (; k < a.kslices; ++k) s0 += p[k * stride];
-    sb.y[static_cast<size_t>(m) * sb.ldy + ln] = (s0 + s1) + (s2 + s3);
-}
-
-
-// The small kernel's shape: waves per workgroup (4 or 8) and K steps per slice (2 to small_max_steps). A round is one
+// The small kernel's shape: waves per workgroup (4 or 8) and K steps per slice (2 to kSmallSteps). A round is one
 // workgroup per CU (the trit table and the B fragments take 104-144 KiB of LDS); a round costs about 3 K steps of
-// loads and staging plus its K steps, each T x W / 4 one-wave steps of matrix-core work per SIMD, and the finish
+// loads and staging plus its K steps, each W / 4 one-wave steps of matrix-core work per SIMD, and the finish
 // about a quarter step per slice (measured at the configs[2] shapes). The cheapest pair; on a tie the longer slices.
 struct SmallShape {
     uint32_t waves, steps, kslices;
 };
 
-static SmallShape small_shape(const Geometry& g, int num_cus, size_t M) {
+static SmallShape small_shape(const Geometry& g, int num_cus) {
     const uint64_t n_ksteps = (g.n_chunks + kStepChunks - 1) / kStepChunks;
     const uint64_t cus = static_cast<uint64_t>(std::max(num_cus, 1));
-    const int Ti = M <= 32 ? 1 : (M <= 64 ? 2 : 4);
-    const double T = Ti;
-    const uint32_t S = small_max_steps(Ti);
     double best = 1e300;
-    SmallShape sh{4, S, 1};
-    for (uint32_t st = S; st >= 2; --st)
+    SmallShape sh{4, kSmallSteps, 1};
+    for (uint32_t st = kSmallSteps; st >= 2; --st)
         for (uint32_t w : {4u, 8u}) {
             const uint64_t ks = (n_ksteps + st - 1) / st;
             const uint64_t rounds = ((g.n_tiles + w - 1) / w * ks + cus - 1) / cus;
-            const double cost = static_cast<double>(rounds) * (3.0 + st * T * w / 4.0) + (ks > 1 ? 0.25 * ks : 0.0);
+            const double cost = static_cast<double>(rounds) * (3.0 + st * w / 4.0) + (ks > 1 ? 0.25 * ks : 0.0);
             if (cost < best - 1e-9) {
                 best = cost;
                 sh = SmallShape{w, st, static_cast<uint32_t>(ks)};
@@ -786,42 +676,103 @@ static SmallShape small_shape(const Geometry& g, int num_cus, size_t M) {
     return sh;
 }
 
-static uint32_t small_kslices(const Geometry& g, int num_cus, size_t M) { return small_shape(g, num_cus, M).kslices; }
+// ---- host side ---------------------------------------------------------------------------------------------------------
 
-// M <= 32 always; 33-128 tokens (two or four token groups) only for matrices of at most 128 tiles (8192 rows) and
-// 32768 columns whose slice sums take at most 64 MiB: at 23040 x 3072 the staged kernel was faster (28.4 against
-// 31.0 us at M = 64, 41.5 against 42.6 us at M = 128), at 3072 x 23040 and 3072 x 3072 slower (24.0 against 20.0 us at
-// M = 64; 34.8 against 33.4 and 24.0 against 19.9 us at M = 128, 54 MiB of slice sums at 3072 x 23040).
-constexpr size_t kSmallPartCap = size_t(64) << 20;
-static bool small_path(const Geometry& g, size_t M, int num_cus) {
-    if (M <= 32) return true;
-    return M <= 128 && g.n_tiles <= 128 && g.cols <= 32768 && small_part_bytes(g, M, num_cus) <= kSmallPartCap;
+// The call's matrices concatenated (tiles, and rows of the slice sums).
+static Geometry group_geometry(const GemmSub* subs, int n) {
+    size_t rows_p = 0;
+    for (int i = 0; i < n; ++i) rows_p += subs[i].g->padded_rows;
+    return geometry(rows_p, subs[0].g->cols);
 }
 
-bool gemm_small_path(const Geometry& g, size_t M, int num_cus) { return small_path(g, M, num_cus); }
+size_t gemm_ksteps(size_t cols) { return (geometry(1, cols).n_chunks + kStepChunks - 1) / kStepChunks; }
 
-static size_t small_part_bytes(const Geometry& g, size_t M, int num_cus) {
-    const uint32_t ks = small_kslices(g, num_cus, M);
+size_t gemm_stage_bytes(size_t cols, size_t M) {
+    return M <= kGemmSmallM ? 0 : round_up(gemm_ksteps(cols) * 5u * ((M + 31) / 32) * 1024u, 256);
+}
+
+struct GemmPlan {
+    uint32_t T, R, n_tt, n_rg, kslices, steps;
+};
+
+// The tile (T token groups, R blocks per wave) and the K slices of least estimated time, in us: 7 for the call and, per
+// K step, 0.4 + 0.095 T R for a workgroup alone on a CU (0.068 T R of it matrix work at 2.4 GHz; a wave issues an
+// instruction every 7 cycles or so, which keeps the rest from running beside it), 0.7 of that for each of several on
+// one CU, plus for more than one slice the finish kernel, 3.5 and its traffic. Over 19 shapes of 512 x 512 to 46080 x 3072
+// and 64 to 512 tokens, timed with every tile and 1 to 12 slices, the choice was 2.7 % slower than the best on average
+// (14 % at worst). Slice sums are kept within the scratch of the no-allocation entry point.
+static GemmPlan gemm_plan(const Geometry& g, size_t M, int num_cus) {
+    const uint32_t n_ksteps = static_cast<uint32_t>(gemm_ksteps(g.cols));
+    const uint32_t n_tg = static_cast<uint32_t>((M + 31) / 32);
+    const uint64_t blocks = 2 * g.n_tiles, cus = static_cast<uint64_t>(std::max(num_cus, 1));
+    const size_t xs = gemm_stage_bytes(g.cols, M), out = M * g.padded_rows * 4u;
+    GemmPlan best{};
+    double best_t = 1e300;
+    constexpr uint32_t kShapes[][2] = {{4, 3}, {4, 1}, {2, 2}, {2, 1}};
+    for (const auto& sh : kShapes) {
+        const uint32_t T = sh[0], R = sh[1];
+        if (T > 2 && n_tg <= 2) continue;
+        GemmPlan p{T, R, (n_tg + T - 1) / T, static_cast<uint32_t>((blocks + 4 * R - 1) / (4 * R)), 1, n_ksteps};
+        const double step = 0.4 + 0.095 * T * R;
+        for (uint32_t want = 1; want <= std::min<uint32_t>(n_ksteps, 32u); ++want) {
+            p.steps = (n_ksteps + want - 1) / want;
+            p.kslices = (n_ksteps + p.steps - 1) / p.steps;
+            if (p.kslices != want) continue;
+            if (want > 1 && xs + want * out > kNoAllocScratchBytes) break;
+            const uint64_t per_cu = (static_cast<uint64_t>(p.n_rg) * p.n_tt * want + cus - 1) / cus;
+            double t = 7.0 + p.steps * step * per_cu * (per_cu > 1 && T * R < 8 ? 0.7 : 1.0);
+            if (want > 1) t += 3.5 + 2.0 * want * out * 0.2e-6;
+            if (t < best_t) {
+                best_t = t;
+                best = p;
+            }
+        }
+    }
+    return best;
+}
+
+size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, int num_cus) {
+    const Geometry g = group_geometry(subs, n);
+    const uint32_t ks = M <= kGemmSmallM ? small_shape(g, num_cus).kslices : gemm_plan(g, M, num_cus).kslices;
     return ks > 1 ? round_up(static_cast<size_t>(ks) * M * g.padded_rows * 4u, 256) : 0;
 }
 
-// The small path over n matrices of the same columns (tiles and slice-sum rows concatenated in order).
-template <bool G>
-static int launch_small(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* ws,
-                        hipStream_t stream) {
-    SmallArgs a{};
+size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus) {
+    const GemmSub sub{nullptr, &g, nullptr, 0};
+    return std::max<size_t>(gemm_stage_bytes(g.cols, M) + gemm_group_part_bytes(&sub, 1, M, num_cus), 256);
+}
+
+template <bool RAW>
+static void launch_tiles(const GemmPlan& p, const GemmArgs& a, hipStream_t stream) {
+    const dim3 grid(round_up(p.n_rg, 8) * p.n_tt, 1, p.kslices), block(256);
+    if (p.T == 4) {
+        if (p.R == 3) hipLaunchKernelGGL((gemm_kernel<4, 3, RAW>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((gemm_kernel<4, 1, RAW>), grid, block, 0, stream, a);
+    } else {
+        if (p.R == 2) hipLaunchKernelGGL((gemm_kernel<2, 2, RAW>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((gemm_kernel<2, 1, RAW>), grid, block, 0, stream, a);
+    }
+}
+
+int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* staged,
+                      uint8_t* part, hipStream_t stream) {
+    if (n < 1 || n > kGemmSubs) VX_FAIL(VX_ERR_INTERNAL, "a GEMM of %d matrices", n);
+    for (int i = 1; i < n; ++i)
+        if (subs[i].g->cols != subs[0].g->cols) VX_FAIL(VX_ERR_INTERNAL, "a grouped GEMM of different columns");
+    const Geometry g = group_geometry(subs, n);
+    GemmArgs a{};
     a.n_sub = static_cast<uint32_t>(n);
     uint32_t tiles = 0, rows_p = 0;
     for (int i = 0; i < n; ++i) {
         const Geometry& gi = *subs[i].g;
-        a.sub[i] = SmallSub{subs[i].w, subs[i].y, static_cast<uint32_t>(subs[i].ldy), static_cast<uint32_t>(gi.rows),
-                            static_cast<uint32_t>(gi.padded_rows), static_cast<uint32_t>(gi.n_tiles), tiles, rows_p};
+        a.sub[i] = GemmMat{subs[i].w, subs[i].y, static_cast<uint32_t>(subs[i].ldy), static_cast<uint32_t>(gi.rows),
+                           static_cast<uint32_t>(gi.padded_rows), static_cast<uint32_t>(gi.n_tiles), tiles, rows_p};
         tiles += static_cast<uint32_t>(gi.n_tiles);
         rows_p += static_cast<uint32_t>(gi.padded_rows);
     }
-    const Geometry g = geometry(rows_p, subs[0].g->cols);  // the call's tiles, for the planner
     a.x = x;
-    a.part = reinterpret_cast<int32_t*>(ws);
+    a.xs = reinterpret_cast<const u32x4g*>(staged);
+    a.part = reinterpret_cast<int32_t*>(part);
     a.ldx = static_cast<uint32_t>(ldx);
     a.rows_p = rows_p;
     a.cols = static_cast<uint32_t>(g.cols);
@@ -829,55 +780,50 @@ static int launch_small(const GemmSub* subs, int n, int num_cus, const int8_t* x
     a.n_chunks = static_cast<uint32_t>(g.n_chunks);
     a.n_ksteps = static_cast<uint32_t>((g.n_chunks + kStepChunks - 1) / kStepChunks);
     a.M = static_cast<uint32_t>(M);
-    const SmallShape sh = small_shape(g, num_cus, M);
-    a.kslices = sh.kslices;
-    a.steps = sh.steps;
-    const dim3 grid((a.n_tiles + sh.waves - 1) / sh.waves, a.kslices), block(sh.waves * 64);
-    if (M <= 32) {
-        if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<1, 8, G>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_small_kernel<1, 4, G>), grid, block, 0, stream, a);
-    } else if (M <= 64) {
-        if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<2, 8, G>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_small_kernel<2, 4, G>), grid, block, 0, stream, a);
+    a.n_tg = static_cast<uint32_t>((M + 31) / 32);
+    if (M <= kGemmSmallM) {
+        const SmallShape sh = small_shape(g, num_cus);
+        a.kslices = sh.kslices;
+        a.steps = sh.steps;
+        const dim3 grid((a.n_tiles + sh.waves - 1) / sh.waves, a.kslices), block(sh.waves * 64);
+        if (n > 1) {
+            if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<8, true>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((gemm_small_kernel<4, true>), grid, block, 0, stream, a);
+        } else {
+            if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<8, false>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((gemm_small_kernel<4, false>), grid, block, 0, stream, a);
+        }
     } else {
-        if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<4, 8, G>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((gemm_small_kernel<4, 4, G>), grid, block, 0, stream, a);
+        const GemmPlan p = gemm_plan(g, M, num_cus);
+        a.kslices = p.kslices;
+        a.steps = p.steps;
+        a.n_rg = p.n_rg;
+        a.n_tt = p.n_tt;
+        if (x == nullptr) {  // staged by the caller
+            launch_tiles<false>(p, a, stream);
+        } else if (g.cols % 16 == 0) {
+            launch_tiles<true>(p, a, stream);
+        } else {
+            hipLaunchKernelGGL(gemm_stage_kernel, dim3((2u * a.n_ksteps + kStageRows - 1) / kStageRows, a.n_tg), dim3(256), 0,
+                               stream, x, a.ldx, a.n_tg, a.cols, a.n_ksteps, reinterpret_cast<u32x4g*>(staged), a.M);
+            VX_HIP(hipGetLastError());
+            launch_tiles<false>(p, a, stream);
+        }
     }
     VX_HIP(hipGetLastError());
     if (a.kslices > 1) {
-        hipLaunchKernelGGL(gemm_small_finish_kernel<G>, dim3((a.rows_p + 255u) / 256u, a.M), dim3(256), 0, stream, a);
+        const dim3 grid((a.rows_p + 255u) / 256u, a.M);
+        if (n > 1) hipLaunchKernelGGL(gemm_finish_kernel<true>, grid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL(gemm_finish_kernel<false>, grid, dim3(256), 0, stream, a);
         VX_HIP(hipGetLastError());
     }
     return VX_OK;
 }
 
-bool gemm_group_small_path(const GemmSub* subs, int n, size_t M, int num_cus) {
-    if (n < 1 || n > kSmallSubs) return false;
-    for (int i = 0; i < n; ++i)
-        if (subs[i].g->cols != subs[0].g->cols || !small_path(*subs[i].g, M, num_cus)) return false;
-    return true;
-}
-
-size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, int num_cus) {
-    size_t rows_p = 0;
-    for (int i = 0; i < n; ++i) rows_p += subs[i].g->padded_rows;
-    return small_part_bytes(geometry(rows_p, subs[0].g->cols), M, num_cus);
-}
-
-int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* ws,
-                      hipStream_t stream) {
-    if (!gemm_group_small_path(subs, n, M, num_cus)) VX_FAIL(VX_ERR_INTERNAL, "a grouped GEMM of %d matrices off the small path", n);
-    return launch_small<true>(subs, n, num_cus, x, M, ldx, ws, stream);
-}
-
 int launch_gemm(const uint8_t* w, const Geometry& g, int num_cus, const int8_t* x, size_t M, size_t ldx, int32_t* y,
                 size_t ldy, uint8_t* ws, hipStream_t stream) {
-    if (small_path(g, M, num_cus)) {
-        const GemmSub sub{w, &g, y, ldy};
-        return launch_small<false>(&sub, 1, num_cus, x, M, ldx, ws, stream);
-    }
-    VX_TRY(launch_gemm_stage(x, M, ldx, g.cols, ws, stream));
-    return launch_gemm_staged(w, g, num_cus, ws, M, y, ldy, ws + gemm_stage_bytes(g.cols, M), stream);
+    const GemmSub sub{w, &g, y, ldy};
+    return launch_gemm_group(&sub, 1, num_cus, x, M, ldx, ws, ws + gemm_stage_bytes(g.cols, M), stream);
 }
 
 // ---- the no-allocation entry point's workspace -----------------------------------------------------------------------

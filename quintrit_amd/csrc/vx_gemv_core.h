@@ -2,6 +2,7 @@
 // GEMV of vx_decode.hip): the digit nibbles of a byte and the broadcast 4-bit dot products.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -58,6 +59,46 @@ __host__ __device__ constexpr uint32_t t4_bytes(uint32_t w) {
     const uint32_t x = (w >> 1) & 0x7f7f7f7fu;
     const uint32_t d4 = (((x + 0x56565656u) >> 7) & 0x01010101u) + (((x + 0x2c2c2c2cu) >> 7) & 0x01010101u);
     return (d4 + 0x7f7f7f7fu) ^ 0x80808080u;
+}
+
+// One lane's 16 bytes of a B fragment of the batched GEMM (vx_gemm.hip): K block kb and half hs of K step ks of a token
+// whose activations x[0..n) are in LDS, 4-byte aligned. In a whole 160-trit block K block kb < 4 takes, for byte-column
+// 16 hs + 4 kb + d, its activations of planes 0..3 (dword d the bytes 160 ks + 32 e + 16 hs + 4 kb + d, e = 0..3), K
+// block 4 plane 4 of the 16 byte-columns; in the packed tail byte-column c holds the activations from 160 ks + 5 c on.
+// Zero past the row.
+__device__ __forceinline__ uint4 gemm_fragment(const int8_t* x, uint32_t n, uint32_t ks, uint32_t kb, uint32_t hs) {
+    if (ks < n / 160u) {
+        const int8_t* b = x + ks * 160u + 16u * hs;
+        if (kb == 4u) return *reinterpret_cast<const uint4*>(b + 128);
+        const uint32_t a0 = *reinterpret_cast<const uint32_t*>(b + 4u * kb), a1 = *reinterpret_cast<const uint32_t*>(b + 4u * kb + 32u);
+        const uint32_t a2 = *reinterpret_cast<const uint32_t*>(b + 4u * kb + 64u), a3 = *reinterpret_cast<const uint32_t*>(b + 4u * kb + 96u);
+        const uint32_t lo01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), hi01 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+        const uint32_t lo23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), hi23 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+        return make_uint4(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                          __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u));
+    }
+    uint32_t w[4];
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) {
+        uint32_t v = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            const uint32_t i = ks * 160u + (kb < 4u ? 5u * (16u * hs + 4u * kb + d) + e : 5u * (16u * hs + 4u * d + e) + 4u);
+            v |= (i < n ? static_cast<uint32_t>(static_cast<uint8_t>(x[i])) : 0u) << (8u * e);
+        }
+        w[d] = v;
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// f(std::integral_constant<uint32_t, k>) for k = 0 .. N - 1: a loop body with its index as a compile-time constant, so that
+// arrays indexed by it stay in fixed registers (a counted loop may be kept rolled, with the registers rotated).
+template <uint32_t N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<uint32_t, N - 1>{});
+    }
 }
 
 __host__ __device__ inline int trit_of(uint32_t b, uint32_t p) {

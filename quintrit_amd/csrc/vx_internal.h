@@ -211,39 +211,27 @@ int launch_device_layout(const uint8_t* planar_dev, const Geometry& g, uint8_t* 
 int launch_digit_sums(const uint8_t* w, const Geometry& g, int32_t* dsum, hipStream_t stream);
 int launch_find_invalid(const uint8_t* planar_dev, uint64_t n, unsigned long long* first, hipStream_t stream);
 int launch_fill_f32(float* out, size_t n, float v, hipStream_t stream);
-size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus);
-// Up to 32 tokens, and up to 128 on matrices of at most 8192 rows and 32768 columns with at most 64 MiB of slice sums
-// (gemm_small_path), a call runs without a staging kernel (gemm_small_kernel builds the B fragments in LDS from x; a
-// finish kernel adds the K slices when there are several) and needs gemm_part_bytes of workspace; otherwise it runs
-// as staging + GEMM + finish.
-bool gemm_small_path(const Geometry& g, size_t M, int num_cus);
-// One matrix of a grouped small-path GEMM: its weights, geometry and output.
+// One matrix of a GEMM: its weights, geometry and output.
 struct GemmSub {
     const uint8_t* w;
     const Geometry* g;
     int32_t* y;
     size_t ldy;
 };
-// Up to 3 matrices with the same columns in one small-path launch (their tiles concatenated), when each of them would
-// take the small path at M tokens; gemm_group_part_bytes of workspace.
-bool gemm_group_small_path(const GemmSub* subs, int n, size_t M, int num_cus);
+// Up to 3 matrices with the same columns in one launch (their tiles concatenated). Up to 32 tokens one kernel builds the
+// B fragments of its K slice from x; more tokens run the tiled kernel, on x itself where its rows allow 16-byte pieces,
+// else after a staging kernel that writes the fragments to `staged` (gemm_stage_bytes); a finish kernel adds the K
+// slices when there are several, from `part` (gemm_group_part_bytes). gemm_workspace_bytes is the sum of both. x may be
+// null where the caller has written the fragments (gemm_fragment) to `staged`.
+constexpr size_t kGemmSmallM = 32;  // tokens of the kernel without staged fragments
+size_t gemm_ksteps(size_t cols);
+size_t gemm_stage_bytes(size_t cols, size_t M);
 size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, int num_cus);
-int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* ws,
-                      hipStream_t stream);
+size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus);
+int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* staged,
+                      uint8_t* part, hipStream_t stream);
 int launch_gemm(const uint8_t* w, const Geometry& g, int num_cus, const int8_t* x, size_t M, size_t ldx, int32_t* y,
                 size_t ldy, uint8_t* ws, hipStream_t stream);
-// The two halves of launch_gemm: staging of the activations (shared by every matrix with the same cols) and the
-// product; gemm_workspace_bytes = gemm_stage_bytes + gemm_part_bytes outside the small path.
-size_t gemm_stage_bytes(size_t cols, size_t M);
-size_t gemm_part_bytes(const Geometry& g, size_t M, int num_cus);
-int launch_gemm_stage(const int8_t* x, size_t M, size_t ldx, size_t cols, uint8_t* ws, hipStream_t stream);
-// Two matrices of one geometry (a gated pair) as one staged launch over the same staged activations, when that launch
-// needs no K split (gemm_staged_pair_ok).
-bool gemm_staged_pair_ok(const Geometry& g, size_t M, int num_cus);
-int launch_gemm_staged_pair(const uint8_t* w, const uint8_t* w2, const Geometry& g, int num_cus, const uint8_t* staged,
-                            size_t M, int32_t* y, int32_t* y2, size_t ldy, hipStream_t stream);
-int launch_gemm_staged(const uint8_t* w, const Geometry& g, int num_cus, const uint8_t* staged, size_t M, int32_t* y,
-                       size_t ldy, uint8_t* part, hipStream_t stream);
 // The same GEMM with its workspace in the library's per-device scratch array (kNoAllocScratchBytes): no allocation.
 constexpr size_t kNoAllocScratchBytes = VX_GEMM_NOALLOC_SCRATCH_BYTES;
 // Looks up (once per device; `device` must be current) the device address of the no-allocation GEMM's scratch, so

@@ -95,3 +95,21 @@ def test_gemm_config2_equals_bruteforce(torch_dev, oracle, rows, cols):
     layer.gemv_i32(torch.from_numpy(x[5]).cuda(), out)
     assert np.array_equal(out.cpu().numpy(), got[5])
     layer.close()
+
+
+@pytest.mark.parametrize("pad", [0, 3])  # rows of x in whole 16-byte pieces (where cols allows), and unaligned ones
+@pytest.mark.parametrize("rows,cols,m", [(24000, 640, 480), (24001, 336, 511), (13824, 336, 500), (33000, 336, 64),
+                                         (200, 2656, 90), (5000, 2672, 100), (60, 112, 33), (300, 14992, 200),
+                                         (1000, 80, 129)])
+def test_gemm_tiles(torch_dev, oracle, rows, cols, m, pad):
+    """The tiled kernel (more than 32 tokens) in each of its tiles, with and without K slices, at the edges of row blocks
+    and token groups, with packed tails of one and of two chunks, against a float64 product (exact)."""
+    from quintrit_amd import VelurexHipLayer
+    print(f"[gemm tiles] {rows}x{cols} m={m} pad={pad}", flush=True)
+    rng = np.random.default_rng(rows + cols + m)
+    t = rng.integers(-1, 2, size=(rows, cols), dtype=np.int8)
+    x = rng.integers(-128, 128, size=(m, cols), dtype=np.int8)
+    layer = VelurexHipLayer(oracle.pack_matrix(t), rows, cols, 1.0)
+    got = gemm(torch_dev, layer, x, ldx=cols + pad)
+    assert np.array_equal(got.astype(np.float64), x.astype(np.float64) @ t.astype(np.float64).T)
+    layer.close()
