@@ -119,11 +119,11 @@ static int alloc_matrix(size_t rows, size_t cols, float weight_scale, vx_matrix*
     if (e == hipSuccess && m->kslices > 1) e = hipMalloc(&m->d_part, static_cast<size_t>(m->kslices) * m->g.padded_rows * 4);
     // the atomic slice sums and tickets of the lone calls (the table GEMV splits K more finely than the digit GEMV,
     // so every matrix has them)
-    const size_t accum_bytes = (m->g.padded_rows + m->g.n_groups + 1) * 4;
+    const size_t accum_bytes = (m->g.padded_rows + m->g.n_tiles + 1) * 4;
     if (e == hipSuccess) e = hipMalloc(&m->d_accum, accum_bytes);
     if (e == hipSuccess) e = hipMemset(m->d_accum, 0, accum_bytes);
     if (e == hipSuccess) m->d_tickets = reinterpret_cast<uint32_t*>(m->d_accum + m->g.padded_rows);
-    if (e == hipSuccess) m->d_done = m->d_tickets + m->g.n_groups;
+    if (e == hipSuccess) m->d_done = m->d_tickets + m->g.n_tiles;
     if (e == hipSuccess) e = hipMalloc(&m->d_dsum, m->g.padded_rows * 4);
     if (e == hipSuccess) e = hipMalloc(&m->d_staged, staged_bytes(cols));
     if (e == hipSuccess) e = hipMalloc(&m->d_io, io_bytes);
@@ -203,39 +203,55 @@ static int check_io(const vx_matrix_t* m, const void* acts, size_t acts_len, con
     return VX_OK;
 }
 
-// A lone GEMV of matrix m on staged activations, or (raw) on int8 activations that every workgroup stages for its own
-// K slice: one launch (a split matrix's K slices add their sums atomically and the last of each tile group writes the
-// outputs). Calls on one matrix share its sums and tickets, so they must not overlap. With `flag`, the launch's last
-// workgroup stores `seq` there once every output is written. K slices hold min_slice_chunks chunks at least (1 where the
-// activations are read from host memory).
-static int run_single(const vx_matrix* m, const uint8_t* staged, void* out, uint32_t out_kind, float post,
-                      hipStream_t s, uint32_t* flag = nullptr, uint32_t seq = 0, const int8_t* raw = nullptr,
-                      uint32_t min_slice_chunks = kLoneMinSliceChunks) {
+// A lone GEMV of matrix m on activations in device memory, staged or (raw) int8: one launch (a split row's K slices add
+// their sums atomically and the last of each tile writes the outputs). Calls on one matrix share its sums and tickets,
+// so they must not overlap.
+static int run_single(const vx_matrix* m, const uint8_t* staged, const int8_t* raw, void* out, uint32_t out_kind, float post,
+                      hipStream_t s) {
+    LoneArgs a{};
+    a.w = m->d_w;
+    a.acts = raw;
+    a.staged = staged;
+    a.dsum = m->d_dsum;
+    a.accum = m->d_accum;
+    a.tickets = m->d_tickets;
+    a.out = out;
+    a.post = post;
+    a.out_kind = out_kind;
+    a.rows = static_cast<uint32_t>(m->g.rows);
+    a.cols = static_cast<uint32_t>(m->g.cols);
+    a.tbr = static_cast<uint32_t>(m->g.tbr);
+    a.n_tiles = static_cast<uint32_t>(m->g.n_tiles);
+    a.n_chunks = static_cast<uint32_t>(m->g.n_chunks);
+    return launch_gemv_lone(a, s);
+}
+
+// The same on host memory (vx_layer_forward): acts and out are pinned host buffers that the kernel reads and writes over
+// the bus, and the launch's last workgroup stores `seq` in `flag` once every output is written. A workgroup takes 16 tiles
+// and one of many K slices, so that the activations cross the bus once per 16 tiles and not once per tile.
+static int run_single_host(const vx_matrix* m, const int8_t* acts, void* out, float post, hipStream_t s, uint32_t* flag,
+                           uint32_t seq) {
     LaunchArgs a{};
-    a.done = flag != nullptr ? m->d_done : nullptr;
+    a.done = m->d_done;
     a.flag = flag;
     a.seq = seq;
-    a.acts = raw;
+    a.acts = acts;
     a.cols = static_cast<uint32_t>(m->g.cols);
-    a.jobs = nullptr;
     a.n_jobs = 1;
     Job& j = a.one;
-    plan_job(j, m->g, static_cast<uint32_t>(m->num_cus), min_slice_chunks);
+    plan_job(j, m->g, static_cast<uint32_t>(m->num_cus));
     j.w = m->d_w;
-    j.staged = staged;
     j.part = m->d_part;
     j.accum = m->d_accum;
     j.tickets = m->d_tickets;
     j.dsum = m->d_dsum;
     j.out = out;
-    j.act_scale = nullptr;
     j.post = post;
     j.weight_scale = m->weight_scale;
-    j.out_kind = out_kind;
-    j.item_begin = 0;
+    j.out_kind = kOutF32Post;
     j.tbr = static_cast<uint32_t>(m->g.tbr);
     a.total_items = job_items(j);
-    return launch_gemv(a, j.rows, nullptr, j.kslices > 1 && j.accum == nullptr ? 1u : 0u, m->num_cus, s);
+    return launch_gemv(a, j.rows, nullptr, 0u, m->num_cus, s);
 }
 
 // A lone GEMV of matrix m through the compact activation tables `lut` (its K slices add up in m's atomic sums, as
@@ -261,18 +277,18 @@ static int run_single_lut(const vx_matrix* m, const int8_t* lut, void* out, uint
 // out = float(acc) * (ws / as) with the division done once here, as the layers do; zeros when as <= 0 or NaN
 // (layer.rs:246-253).
 static int gemv_f32_staged(const vx_matrix* m, const uint8_t* staged, float act_scale, float* out, hipStream_t s) {
-    if (act_scale > 0.0f) return run_single(m, staged, out, kOutF32Post, m->weight_scale / act_scale, s);
+    if (act_scale > 0.0f) return run_single(m, staged, nullptr, out, kOutF32Post, m->weight_scale / act_scale, s);
     return launch_fill_f32(out, m->g.rows, 0.0f, s);
 }
 
 // The raw-activation calls: one launch, each workgroup staging its own K slice.
 static int gemv_f32_dev(vx_matrix* m, const int8_t* acts, float act_scale, float* out, hipStream_t s) {
     if (!(act_scale > 0.0f)) return launch_fill_f32(out, m->g.rows, 0.0f, s);
-    return run_single(m, nullptr, out, kOutF32Post, m->weight_scale / act_scale, s, nullptr, 0, acts);
+    return run_single(m, nullptr, acts, out, kOutF32Post, m->weight_scale / act_scale, s);
 }
 
 static int gemv_i32_dev(vx_matrix* m, const int8_t* acts, int32_t* out, hipStream_t s) {
-    return run_single(m, nullptr, out, kOutI32, 1.0f, s, nullptr, 0, acts);
+    return run_single(m, nullptr, acts, out, kOutI32, 1.0f, s);
 }
 
 }  // namespace vx
@@ -410,7 +426,7 @@ int vx_gemv_staged_i32_dev(const vx_matrix_t* matrix, const void* staged, size_t
         VX_TRY(check_kind(matrix, kKindVelurex));
         VX_TRY(check_staged(matrix, staged, staged_len, out, out_capacity));
         VX_TRY(set_device_of(matrix));
-        return run_single(matrix, static_cast<const uint8_t*>(staged), out, kOutI32, 1.0f, static_cast<hipStream_t>(stream));
+        return run_single(matrix, static_cast<const uint8_t*>(staged), nullptr, out, kOutI32, 1.0f, static_cast<hipStream_t>(stream));
     });
 }
 
@@ -589,8 +605,9 @@ int vx_layer_forward(const vx_matrix_t* matrix, const int8_t* acts, size_t acts_
         const uint32_t seq = m->io_seq + 1u == 0u ? 1u : m->io_seq + 1u;  // never 0, the buffer's initial value
         m->io_seq = seq;
         std::memcpy(m->h_io, acts, m->g.cols);
-        VX_TRY(run_single(m, nullptr, m->h_io_dev + out_off, kOutF32Post, m->weight_scale / act_scale, m->io_stream,
-                          reinterpret_cast<uint32_t*>(m->h_io_dev + flag_off), seq, m->h_io_dev, 1u));
+        VX_TRY(run_single_host(m, reinterpret_cast<const int8_t*>(m->h_io_dev), m->h_io_dev + out_off,
+                               m->weight_scale / act_scale, m->io_stream, reinterpret_cast<uint32_t*>(m->h_io_dev + flag_off),
+                               seq));
         // Wait for the flag; every 65536 reads (tens of microseconds, longer than a call), ask the stream whether it
         // has ended (an error, or an end without the flag, is reported instead of waiting on).
         for (uint32_t i = 1;; ++i) {
@@ -623,7 +640,7 @@ static int planar_oneshot(const uint8_t* weights, size_t weights_len, size_t row
     hipError_t e = hipMemcpy(d_acts, acts, cols, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         st = launch_stage(d_acts, cols, m->d_staged, nullptr);
-        if (st == VX_OK) st = run_single(m, m->d_staged, d_out, f32 ? kOutF32Post : kOutI32, scale, nullptr);
+        if (st == VX_OK) st = run_single(m, m->d_staged, nullptr, d_out, f32 ? kOutF32Post : kOutI32, scale, nullptr);
         if (st == VX_OK) e = hipMemcpy(out, d_out, rows * 4, hipMemcpyDeviceToHost);
     }
     (void)hipDeviceSynchronize();

@@ -444,6 +444,96 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(8, 
     }
 }
 
+// ---- a GEMV on its own (activations in device memory) -----------------------------------------------------------------
+
+// Workgroup (tile, K slice): its 16 waves split the slice's chunks of one 64-row tile and add their sums in LDS, and wave
+// 0 writes the rows (one slice) or adds them atomically to the matrix's sums, the tile's last slice writing the outputs
+// (gemv_kernel's hand-off). What bounds such a call is latency: with a wave per tile and K split over workgroups instead
+// (gemv_kernel), up to 13 slices of a tile group met in atomics and a ticket, about 2 us of a 6.6 us call, where this
+// form has none up to kLoneChunks chunks a row. Kernel time at 640 x 2560 7.0 -> 4.5 us and at 23040 x 3072 8.9 -> 7.3;
+// per call at 3072 x 23040 9.9 -> 8.4 and at 12000 x 8000 12.2 -> 10.9. More slices than that are not faster anywhere
+// (3072 x 3072: 1 to 8 slices the same, 23040 x 3072: 8.7 us with one, 11.7 with two).
+// The activations of a slice are staged by every workgroup (from acts, or copied from the staged vector), one byte-column
+// per thread, while its weights are in flight.
+template <bool RAW>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(8, 8))) void gemv_lone_kernel(LoneArgs a) {
+    __shared__ uint32_t tab[256 * 64];  // row B: 32 copies of the digit nibbles of byte B (first half)
+    __shared__ uint2 ae[kLoneChunks * 16];
+    __shared__ int red[kWaves][64];
+    __shared__ int xsum[kWaves];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t tile = blockIdx.x, ks = blockIdx.y;
+    const uint32_t grp = tile / kTileGroup, t16 = tile - grp * kTileGroup;
+    const uint32_t T = min(static_cast<uint32_t>(kTileGroup), a.n_tiles - grp * kTileGroup);
+    const uint32_t q0 = ks * a.slice_chunks, nq = min(a.slice_chunks, a.n_chunks - q0);
+
+    // the wave's chunks q0 + wave, + 16, ... (one past the slice repeats its last and is not used)
+    const uint32_t cnt = wave < nq ? (nq - wave + kWaves - 1) / kWaves : 0u;
+    const g_u4* wp = (const g_u4*)(a.w) + (static_cast<size_t>(grp) * kTileGroup * a.n_chunks + t16) * 64u + lane;
+    u32x4 b[kGroup];
+#pragma unroll
+    for (uint32_t i = 0; i < kGroup; ++i)
+        b[i] = __builtin_nontemporal_load(wp + static_cast<size_t>(q0 + min(wave + kWaves * i, nq - 1u)) * T * 64u);
+    const uint32_t row = tile * kTileRows + lane;
+    const int dsum = wave == 0 ? a.dsum[row] : 0;
+    int xs = 0;
+    const uint32_t full = a.cols / 160u * 32u;
+    for (uint32_t i = tid; i < nq * 16u; i += kWaves * 64u) {
+        if constexpr (RAW) ae[i] = raw_entry(a.acts, a.cols, a.tbr, full, q0 * 16u + i, &xs);
+        else ae[i] = reinterpret_cast<const uint2*>(a.staged + kStageHeader)[q0 * 16u + i];
+    }
+    if constexpr (!RAW) {  // the header's 16 parts of the whole vector's sum, once
+        if (ks == 0 && tid < 16u) xs = reinterpret_cast<const int*>(a.staged)[tid];
+    }
+    for (uint32_t i = tid; i < 256u * 8u; i += kWaves * 64u) {
+        const uint32_t e = digit_nibbles(i >> 3);
+        *reinterpret_cast<uint4*>(reinterpret_cast<char*>(tab) + (i >> 3) * 256u + (i & 7u) * 16u) = make_uint4(e, e, e, e);
+    }
+    for (int off = 32; off > 0; off >>= 1) xs += __shfl_xor(xs, off);
+    if (lane == 0) xsum[wave] = xs;
+    __syncthreads();
+
+    const char* tabb = reinterpret_cast<const char*>(tab);
+    const uint32_t lane_off = (lane & 31u) * 4u;
+    int acc_lo = 0, acc_hi = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kGroup; ++i) {
+        if (i >= cnt) break;  // wave-uniform; kLoneChunks is kGroup rounds of the workgroup
+        const uint32_t dw[4] = {b[i].x, b[i].y, b[i].z, b[i].w};
+        const uint2 e = ae[(wave + kWaves * i) * 16u + (lane & 15u)];
+        uint32_t t[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const uint32_t addr = __builtin_amdgcn_perm(dw[k >> 2], lane_off, 0x0c0c0000u | ((4u + (k & 3)) << 8));
+            t[k] = *reinterpret_cast<const uint32_t*>(tabb + addr);
+        }
+        dot4_bcast<0>(acc_lo, acc_hi, e.x, e.y, t[0], t[1], t[2], t[3]);
+        dot4_bcast<4>(acc_lo, acc_hi, e.x, e.y, t[4], t[5], t[6], t[7]);
+        dot4_bcast<8>(acc_lo, acc_hi, e.x, e.y, t[8], t[9], t[10], t[11]);
+        dot4_bcast<12>(acc_lo, acc_hi, e.x, e.y, t[12], t[13], t[14], t[15]);
+    }
+    red[wave][lane] = acc_lo + 16 * acc_hi;
+    __syncthreads();
+    if (wave != 0) return;
+    int v = 0;  // the slice's sums of 16 hi + lo, less its activation sum (staged: the vector's, in slice 0)
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) v += red[w][lane] - xsum[w];
+    if (a.kslices > 1u) {
+        atomicAdd(a.accum + row, v);
+        __builtin_amdgcn_s_waitcnt(0);  // performed before the ticket (take_ticket's hand-off; this wave alone writes)
+        uint32_t last = 0;
+        if (lane == 0) last = take_ticket(a.tickets + tile, a.kslices - 1u);
+        if (__builtin_amdgcn_readfirstlane(last) == 0u) return;
+        v = atomicExch(a.accum + row, 0);
+        if (lane == 0) atomicExch(a.tickets + tile, 0u);
+    }
+    if (row >= a.rows) return;
+    const int acc = v + 8 * dsum;
+    if (a.out_kind == kOutI32) static_cast<int32_t*>(a.out)[row] = acc;
+    else static_cast<float*>(a.out)[row] = static_cast<float>(acc) * a.post;
+}
+
 // Adds the K-slice partial sums of the split jobs and applies their epilogue. Block = 64 rows x 4 waves; wave w adds
 // the slices w, w + 4, ... of its 64 rows, then the 4 waves combine through LDS. blockIdx.y indexes `split` (the
 // plan's split jobs) or, without a job array, the one job.
@@ -476,14 +566,11 @@ __global__ __launch_bounds__(256) void finish_kernel(LaunchArgs args, const uint
 
 // ---- host side ---------------------------------------------------------------------------------------------------------------
 
-void plan_job(Job& j, const Geometry& g, uint32_t target_items, uint32_t min_slice_chunks) {
+void plan_job(Job& j, const Geometry& g, uint32_t target_items) {
     const uint32_t nc = static_cast<uint32_t>(g.n_chunks);
     const uint32_t groups = static_cast<uint32_t>(g.n_groups);
     uint32_t ks = (nc + kMaxSliceChunks - 1) / kMaxSliceChunks;
-    if (target_items) {
-        const uint32_t most = std::max(nc / std::max(min_slice_chunks, 1u), 1u);  // slices of min_slice_chunks at most
-        ks = std::max(ks, std::min(most, (target_items + groups - 1) / groups));
-    }
+    if (target_items) ks = std::max(ks, std::min(nc, (target_items + groups - 1) / groups));
     const uint32_t sc = (nc + ks - 1) / ks;
     j.slice_chunks = sc;
     j.kslices = (nc + sc - 1) / sc;
@@ -522,7 +609,7 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
     const uint32_t grid = std::min<uint32_t>(a.total_items, 2u * static_cast<uint32_t>(num_cus));
     if (a.jobs) hipLaunchKernelGGL((gemv_kernel<true, false>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
     else if (a.acts) hipLaunchKernelGGL((gemv_kernel<false, true>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
-    else hipLaunchKernelGGL((gemv_kernel<false, false>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
+    else VX_FAIL(VX_ERR_INTERNAL, "a lone GEMV without activations");
     VX_HIP(hipGetLastError());
     if (n_split) {
         const dim3 fgrid((max_rows + 63u) / 64u, n_split);
@@ -530,6 +617,18 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
         else hipLaunchKernelGGL(finish_kernel<false>, fgrid, dim3(256), 0, stream, a, split);
         VX_HIP(hipGetLastError());
     }
+    return VX_OK;
+}
+
+// A lone GEMV's K slices: one while a row has at most kLoneChunks chunks, else the fewest, of equal length.
+int launch_gemv_lone(LoneArgs a, hipStream_t stream) {
+    a.kslices = (a.n_chunks + kLoneChunks - 1u) / kLoneChunks;
+    a.slice_chunks = (a.n_chunks + a.kslices - 1u) / a.kslices;
+    a.kslices = (a.n_chunks + a.slice_chunks - 1u) / a.slice_chunks;
+    const dim3 grid(a.n_tiles, a.kslices);
+    if (a.acts != nullptr) hipLaunchKernelGGL(gemv_lone_kernel<true>, grid, dim3(kWaves * 64), 0, stream, a);
+    else hipLaunchKernelGGL(gemv_lone_kernel<false>, grid, dim3(kWaves * 64), 0, stream, a);
+    VX_HIP(hipGetLastError());
     return VX_OK;
 }
 

@@ -179,16 +179,9 @@ struct LaunchArgs {
 
 constexpr uint32_t kMaxSliceChunks = 40;  // chunks per K slice staged in LDS (5 KiB of activations)
 
-// Host planner: fills kslices/slice_chunks of a job. `target_items` spreads a lone GEMV over the GPU, with at least
-// `min_slice_chunks` chunks per slice where the row has them; 0 keeps slices as long as kMaxSliceChunks allows (the
-// batched launches, which have work enough).
-void plan_job(Job& j, const Geometry& g, uint32_t target_items, uint32_t min_slice_chunks = 1);
-// The chunks per K slice a lone GEMV on activations in device memory keeps at least: below that the slices' atomic
-// sums and tickets cost more than their parallelism gains at the shapes of one to three tile groups (2560 x 2560: 7.16
-// -> 6.57 us per call, 3072 x 3072: 7.95 -> 7.03 us, 1024 x 3072: 7.2 -> 6.7-7.0 us; 4 chunks were slower again), and
-// the wide shapes keep their split. Activations read from host memory keep one chunk per slice (vx_layer_forward at
-// 3072 x 3072: 19 us with one, 22-37 us with two or three).
-constexpr uint32_t kLoneMinSliceChunks = 3;
+// Host planner: fills kslices/slice_chunks of a job. `target_items` spreads a lone GEMV over the GPU; 0 keeps slices as
+// long as kMaxSliceChunks allows (the batched launches, which have work enough).
+void plan_job(Job& j, const Geometry& g, uint32_t target_items);
 inline uint32_t job_items(const Job& j) {
     return (j.n_tiles + kTileGroup - 1) / kTileGroup * j.kslices;
 }
@@ -206,6 +199,23 @@ int launch_stage_batch(const StageJob* jobs, uint32_t n, uint32_t max_groups, hi
 // indices in a.jobs; unused without a job array).
 int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, uint32_t n_split, int num_cus,
                 hipStream_t stream);
+// A lone GEMV on activations in device memory: raw (acts) or staged. accum (padded_rows) and tickets (one per tile) are
+// zero between calls and used when the row is split.
+struct LoneArgs {
+    const uint8_t* w;
+    const int8_t* acts;
+    const uint8_t* staged;
+    const int32_t* dsum;
+    int32_t* accum;
+    uint32_t* tickets;
+    void* out;
+    float post;         // kOutF32Post
+    uint32_t out_kind;  // kOutI32 or kOutF32Post
+    uint32_t rows, cols, tbr, n_tiles, n_chunks;
+    uint32_t kslices, slice_chunks;  // set by launch_gemv_lone
+};
+constexpr uint32_t kLoneChunks = 64;  // chunks of a K slice at most: 4 per wave
+int launch_gemv_lone(LoneArgs a, hipStream_t stream);
 int launch_device_layout(const uint8_t* planar_dev, const Geometry& g, uint8_t* dst, hipStream_t stream);
 // dsum[r] = digit sum of the device row r (every byte of the device layout, padding included).
 int launch_digit_sums(const uint8_t* w, const Geometry& g, int32_t* dsum, hipStream_t stream);
@@ -305,7 +315,7 @@ struct vx_matrix {
     uint32_t kslices, slice_chunks;  // K split of a lone GEMV on this matrix
     uint8_t* d_w;       // weights, device layout (vx_layout)
     int32_t* d_part;    // K-slice partial sums of a lone GEMV
-    int32_t* d_accum;   // a lone GEMV's atomic K-slice sums (padded_rows), tickets (one per tile group) and
+    int32_t* d_accum;   // a lone GEMV's atomic K-slice sums (padded_rows), tickets (one per tile) and
     uint32_t* d_tickets;  // completion counter (d_done), zero between calls
     uint32_t* d_done;
     int32_t* d_dsum;    // per padded row: digit sum of the device row (the signed low-nibble correction)

@@ -409,3 +409,37 @@ def test_plan_in_hip_graph_replays(torch_dev, oracle):
         assert np.array_equal(out.cpu().numpy(), eager)
     plan.close()
     layer.close()
+
+
+@pytest.mark.parametrize("cols", [80, 5120, 5121, 10241])  # one chunk, the longest single K slice, two and three slices
+@pytest.mark.parametrize("rows", [1, 64, 65, 1090])        # partial and whole tiles, a second tile group
+def test_lone_gemv_slices(torch_dev, oracle, rows, cols):
+    """Lone GEMVs on raw and on staged activations around the K-slice boundary, twice each (the atomic sums and tickets of
+    a split row are zero again after a call), int32 and f32 outputs against brute force, bit for bit."""
+    from quintrit_amd import VelurexHipLayer, _lib
+    import ctypes
+    torch = torch_dev
+    rng = np.random.default_rng(rows + cols)
+    t = rng.integers(-1, 2, size=(rows, cols), dtype=np.int8)
+    layer = VelurexHipLayer(oracle.pack_matrix(t), rows, cols, 0.5)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    n = _lib.staged_bytes(cols)
+    staged = torch.empty(n, dtype=torch.uint8, device="cuda")
+    for _ in range(2):
+        a = rng.integers(-128, 128, size=cols, dtype=np.int8)
+        want = t.astype(np.int64) @ a.astype(np.int64)
+        x = torch.from_numpy(a).cuda()
+        yi = torch.full((rows,), -7, dtype=torch.int32, device="cuda")
+        yf = torch.full((rows,), -7.0, dtype=torch.float32, device="cuda")
+        ys = torch.full((rows,), -7, dtype=torch.int32, device="cuda")
+        layer.gemv_i32(x, yi)
+        layer.gemv_f32(x, 3.0, yf)
+        _lib.check(_lib.lib().vx_stage_acts_dev(ctypes.c_void_p(x.data_ptr()), cols, cols,
+                                                ctypes.c_void_p(staged.data_ptr()), n, stream))
+        _lib.check(_lib.lib().vx_gemv_staged_i32_dev(layer.handle, ctypes.c_void_p(staged.data_ptr()), n,
+                                                     ctypes.c_void_p(ys.data_ptr()), rows, stream))
+        assert np.array_equal(yi.cpu().numpy(), want)
+        assert np.array_equal(ys.cpu().numpy(), want)
+        post = np.float32(0.5) / np.float32(3.0)
+        assert np.array_equal(yf.cpu().numpy().view(np.uint32), (want.astype(np.float32) * post).view(np.uint32))
+    layer.close()
