@@ -66,9 +66,7 @@ class VelurexHipLayer:
             raise ValueError(f"activations hold {a.size} values, cols = {self._cols}")
         if out.dtype != np.float32 or not out.flags.c_contiguous or out.size != self._rows:
             raise ValueError("out must be a contiguous float32 array of rows values")
-        _lib.check(_lib.lib().vx_layer_forward(self._h, a.ctypes.data_as(ctypes.c_void_p), a.size,
-                                               ctypes.c_float(act_scale), out.ctypes.data_as(ctypes.c_void_p),
-                                               out.size))
+        _lib.check(_lib.lib().vx_layer_forward(self._h, a.ctypes.data, a.size, act_scale, out.ctypes.data, out.size))
 
     def kernel_type(self) -> str:
         return KERNEL_TYPE
@@ -92,14 +90,12 @@ class VelurexHipLayer:
 
     def gemv_i32(self, acts_dev, out_dev, stream=None) -> None:
         """Exact int32 GEMV of device tensors (torch int8 [cols] -> int32 [rows]), enqueued on ``stream``."""
-        _lib.check(_lib.lib().vx_gemv_i32_dev(self._h, ctypes.c_void_p(acts_dev.data_ptr()), acts_dev.numel(),
-                                              ctypes.c_void_p(out_dev.data_ptr()), out_dev.numel(),
-                                              _stream_ptr(stream)))
+        _lib.check(_lib.lib().vx_gemv_i32_dev(self._h, acts_dev.data_ptr(), acts_dev.numel(), out_dev.data_ptr(),
+                                              out_dev.numel(), _stream_ptr(stream)))
 
     def gemv_f32(self, acts_dev, act_scale: float, out_dev, stream=None) -> None:
-        _lib.check(_lib.lib().vx_gemv_f32_dev(self._h, ctypes.c_void_p(acts_dev.data_ptr()), acts_dev.numel(),
-                                              ctypes.c_float(act_scale), ctypes.c_void_p(out_dev.data_ptr()),
-                                              out_dev.numel(), _stream_ptr(stream)))
+        _lib.check(_lib.lib().vx_gemv_f32_dev(self._h, acts_dev.data_ptr(), acts_dev.numel(), act_scale,
+                                              out_dev.data_ptr(), out_dev.numel(), _stream_ptr(stream)))
 
     def gemv_lut_i32(self, lut_dev, out_dev, stream=None) -> None:
         """The int32 GEMV through compact activation tables (torch int8 tensor built by compact_lut_dev for this
@@ -123,10 +119,12 @@ def compact_lut(acts_dev, cols: int, stream=None):
 
 
 def _stream_ptr(stream):
+    """The HIP stream handle of a torch stream, or of the current device's current stream. (Building the stream object
+    that torch.cuda.current_stream returns took more of a small call than everything else on the host.)"""
     if stream is None:
         import torch
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def gemv_planar_i32(planar: np.ndarray, rows: int, cols: int, acts: np.ndarray) -> np.ndarray:
