@@ -1610,6 +1610,83 @@ __device__ __forceinline__ float score_dot4(const uint16_t* q, const uint4 (&kr)
     return (t0 + t1) + (t2 + t3);
 }
 
+// Prefill attention of passes that end below position kTinyCtx: a workgroup per (query head, token), a context of one
+// position per 4-lane group, everything requested at the start (K, V and q), the factors in the lanes of every wave
+// (position = lane) and read as scalars by its chain. Such passes are bound by latency: the tiled kernel, whose single
+// position tile is a chain of 32-cycle products, takes 7.8 us for 4 and 12.0 for 64 tokens of 12 heads of 256, this form
+// 4.7 and 8.4.
+constexpr uint32_t kTinyCtx = 64;
+template <int HD>
+__global__ __launch_bounds__(256) void pf_attn_tiny_kernel(PfAttnArgs a) {
+    constexpr int kBlk = HD / 32;
+    __shared__ __align__(16) uint16_t qs[HD];
+    __shared__ float sc[kTinyCtx];
+    __shared__ uint64_t etab[32];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = blockIdx.x, kvh = h / a.gqa, t = blockIdx.y;
+    const uint32_t seq = a.ctl->pos + 2u - a.n_tok + t;  // at most kTinyCtx
+    const uint16_t* kb = a.kc + static_cast<size_t>(kvh) * a.max_ctx * HD;
+    const uint16_t* vt = a.vc + static_cast<size_t>(kvh) * HD * a.vstride;
+    const size_t row0 = (static_cast<size_t>(t) * a.n_heads + h) * HD;
+
+    const uint32_t j = tid & 3u, p = tid >> 2;
+    const uint16_t qv = tid < HD ? a.qbuf[row0 + tid] : static_cast<uint16_t>(0);
+    uint4 kr[kBlk];
+    const uint16_t* row = kb + static_cast<size_t>(min(p, seq - 1u)) * HD + 8u * j;
+#pragma unroll
+    for (int i = 0; i < kBlk; ++i) kr[i] = *reinterpret_cast<const uint4*>(row + 32 * i);
+    const bool chain = wave * 64u < HD, has_d = wave * 64u + lane < HD;
+    const uint32_t d = has_d ? wave * 64u + lane : 0u;
+    u32x4 v[kTinyCtx / 8];
+#pragma unroll
+    for (uint32_t g = 0; g < kTinyCtx / 8; ++g)
+        v[g] = *reinterpret_cast<const u32x4*>(vt + (static_cast<size_t>(min(g, (seq - 1u) / 8u)) * HD + d) * 8u);
+    if (tid < HD) qs[tid] = qv;
+    if (tid < 32u) etab[tid] = expf_tab(tid);
+    __syncthreads();
+    const float dot = score_dot4<HD>(qs, kr, j);
+    if (j == 0) sc[p] = dot * a.scale;
+    __syncthreads();
+    if (!chain) return;
+
+    const auto tab = [&](uint32_t k) { return etab[k]; };
+    const float s = lane < seq ? sc[lane] : -__builtin_inff();
+    float m = s != s ? -__builtin_inff() : s;  // the running maximum: NaN never moves it
+#pragma unroll
+    for (int sh = 1; sh < 64; sh <<= 1) {
+        const float o = __shfl_up(m, sh);
+        if (lane >= static_cast<uint32_t>(sh)) m = o > m ? o : m;
+    }
+    const float before = __shfl_up(m, 1);
+    const float prev = lane == 0 ? -__builtin_inff() : before;
+    const bool up = s > prev;
+    const float x = expf_nonpos(up ? prev - s : s - prev, tab);
+    const float f = up ? -x : x;
+    float y = 0.0f, ssum = 0.0f;
+    static_for<kTinyCtx / 8>([&](auto gc) {
+        constexpr uint32_t g = decltype(gc)::value;
+        if (8u * g >= seq) return;
+        const uint32_t w[4] = {v[g].x, v[g].y, v[g].z, v[g].w};
+#pragma unroll
+        for (uint32_t e = 0; e < 8; ++e) {
+            if (8u * g + e >= seq) break;  // uniform
+            const float fe = bits_f32(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(f32_bits(f)), static_cast<int>(8u * g + e))));
+            const float ve = f16_f32(static_cast<uint16_t>(w[e >> 1] >> ((e & 1u) * 16u)));
+            if (__builtin_signbit(fe)) {  // a new maximum
+                y = r16(y * -fe);
+                y = r16(__builtin_fmaf(ve, 1.0f, y));
+                ssum = __builtin_fmaf(ssum, -fe, 1.0f);
+            } else {
+                y = r16(__builtin_fmaf(ve, fe, y));
+                ssum = ssum + fe;
+            }
+        }
+    });
+    const float s_inv = ssum == 0.0f ? 0.0f : 1.0f / ssum;
+    if (has_d) a.out[row0 + d] = y * s_inv;
+}
+
 // Scores of positions p0 .. p0 + 63 (p0 = blockIdx.y * 64, below pos + 1) for up to kScoreHeads query heads of one KV
 // head (blockIdx.x: KV head, head group), so that each K row is read once for the heads that share it. The workgroup
 // whose range holds the position itself rotates its k (the first head group also appends k and v to the cache); every
@@ -2641,6 +2718,10 @@ int launch_attention_short(const AttnArgs& a, uint32_t head_dim, hipStream_t s) 
     return VX_OK;
 }
 
+// The attention of a prefill pass by the positions it reaches: below kTinyCtx, below a padded length of 512, or beyond,
+// where the context is split in chunks.
+enum class PfForm : uint32_t { kTiny, kWhole, kSplit };
+
 template <int HD, int TOK, int POS, int W, int SL>
 static void launch_pf_attn_as(const PfAttnArgs& a, bool split, hipStream_t s) {
     // one tile more than the tokens fill: they need not start at a multiple of TOK
@@ -2654,7 +2735,12 @@ static void launch_pf_attn_as(const PfAttnArgs& a, bool split, hipStream_t s) {
 // them 42.6 instead of 53.2 (192); 256 tokens of 20 heads of 128 29.7 instead of 38.5 (320); with 300 tokens (912 and
 // 1520 workgroups, the split context) the two forms take the same time.
 template <int HD>
-static void launch_pf_attn(const PfAttnArgs& a, int num_cus, bool split, hipStream_t s) {
+static void launch_pf_attn(const PfAttnArgs& a, int num_cus, PfForm form, hipStream_t s) {
+    if (form == PfForm::kTiny) {
+        hipLaunchKernelGGL(pf_attn_tiny_kernel<HD>, dim3(a.n_heads, a.n_tok), dim3(256), 0, s, a);
+        return;
+    }
+    const bool split = form == PfForm::kSplit;
     const uint32_t wgs = a.n_heads * ((a.n_tok + 15u) / 16u) * (split ? 4u : 1u);
     if (wgs < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 16, 16, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
     else launch_pf_attn_as<HD, 16, 16, 4, 1>(a, split, s);
@@ -2662,12 +2748,11 @@ static void launch_pf_attn(const PfAttnArgs& a, int num_cus, bool split, hipStre
         hipLaunchKernelGGL(pf_attn_combine_kernel<HD>, dim3((a.n_heads * HD + 2047u) / 2048u, a.n_tok), dim3(256), 0, s, a);
 }
 
-// The attention of a prefill pass; split: some position of the pass has a padded length of 512 or more.
-int launch_attention_prefill(const PfAttnArgs& a, uint32_t head_dim, int num_cus, bool split, hipStream_t s) {
-    if (head_dim == 256) launch_pf_attn<256>(a, num_cus, split, s);
-    else if (head_dim == 128) launch_pf_attn<128>(a, num_cus, split, s);
-    else if (head_dim == 64) launch_pf_attn<64>(a, num_cus, split, s);
-    else if (head_dim == 32) launch_pf_attn<32>(a, num_cus, split, s);
+int launch_attention_prefill(const PfAttnArgs& a, uint32_t head_dim, int num_cus, PfForm form, hipStream_t s) {
+    if (head_dim == 256) launch_pf_attn<256>(a, num_cus, form, s);
+    else if (head_dim == 128) launch_pf_attn<128>(a, num_cus, form, s);
+    else if (head_dim == 64) launch_pf_attn<64>(a, num_cus, form, s);
+    else if (head_dim == 32) launch_pf_attn<32>(a, num_cus, form, s);
     else VX_FAIL(VX_ERR_INTERNAL, "no attention kernel for head_dim %u", head_dim);
     VX_HIP(hipGetLastError());
     return VX_OK;
@@ -2752,7 +2837,8 @@ struct vx_decoder {
     uint8_t* pf_part;                 // the GEMM's K-slice partial sums
     struct PfGraph {
         uint32_t n;
-        bool head, split;
+        bool head;
+        vx::PfForm form;
         hipGraph_t graph;
         hipGraphExec_t exec;
     };
@@ -3319,8 +3405,7 @@ static ProjOut pf_proj_out(const vx_decoder* d, size_t layer, int kind, const fl
 
 // Enqueues one prefill pass over n tokens (the last at the loop state's position) on `st`; with `head`, the final norm,
 // head and greedy argmax of the last token follow and advance the loop state as a decode step does.
-// split: some position of the pass is at kShortCtx or beyond, where the attention runs in chunks.
-static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split, hipStream_t st) {
+static int record_prefill(const vx_decoder* d, uint32_t n, bool head, PfForm form, hipStream_t st) {
     const vx_decoder_config_t& c = d->cfg;
     const size_t L = c.n_layers, H = c.hidden, F = c.ffn;
     const bool sub = has_sub_norms(d);
@@ -3414,7 +3499,7 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
         at.scale = 1.0f / sqrtf(static_cast<float>(c.head_dim));
         at.qbuf = d->pf_q;
         at.n_tok = n;
-        VX_TRY(launch_attention_prefill(at, c.head_dim, d->num_cus, split, st));
+        VX_TRY(launch_attention_prefill(at, c.head_dim, d->num_cus, form, st));
         // the o input: attention output (sub-norm or none)
         in = stage_input(d, kInPlain, d->qd, d->pf_att, nullptr, sub ? nw[VX_NORM_ATTN_SUB] : nullptr);
         VX_TRY(stage(in, static_cast<uint32_t>(d->qd), 0, as_o));
@@ -3461,9 +3546,9 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, bool split
 }
 
 // The graph of a prefill pass over n tokens (recorded on first use; a few are kept).
-static int prefill_graph(vx_decoder* d, uint32_t n, bool head, bool split, hipGraphExec_t* out) {
+static int prefill_graph(vx_decoder* d, uint32_t n, bool head, PfForm form, hipGraphExec_t* out) {
     for (const auto& g : d->pf_graphs)
-        if (g.n == n && g.head == head && g.split == split) {
+        if (g.n == n && g.head == head && g.form == form) {
             *out = g.exec;
             return VX_OK;
         }
@@ -3474,7 +3559,7 @@ static int prefill_graph(vx_decoder* d, uint32_t n, bool head, bool split, hipGr
         d->pf_graphs.erase(d->pf_graphs.begin());
     }
     VX_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-    const int st = record_prefill(d, n, head, split, d->stream);
+    const int st = record_prefill(d, n, head, form, d->stream);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(d->stream, &graph);
     if (st != VX_OK) {
@@ -3488,7 +3573,7 @@ static int prefill_graph(vx_decoder* d, uint32_t n, bool head, bool split, hipGr
         (void)hipGraphDestroy(graph);
         VX_HIP(ei);
     }
-    d->pf_graphs.push_back({n, head, split, graph, exec});
+    d->pf_graphs.push_back({n, head, form, graph, exec});
     *out = exec;
     return VX_OK;
 }
@@ -3503,8 +3588,10 @@ static int run_prefill(vx_decoder* d, uint32_t pos0, uint32_t n, uint32_t n_prom
         const bool last = done + m == n;
         hipGraphExec_t exec = nullptr;
         // the split starts at a padded length of 512 (kv_split), so at position 256, unless max_ctx caps it below
-        const bool split = d->cfg.max_ctx >= 2 * kShortCtx && pos0 + done + m > kShortCtx;
-        VX_TRY(prefill_graph(d, m, last, split, &exec));
+        const uint32_t end = pos0 + done + m;
+        const bool split = d->cfg.max_ctx >= 2 * kShortCtx && end > kShortCtx;
+        const PfForm form = end <= kTinyCtx ? PfForm::kTiny : (split ? PfForm::kSplit : PfForm::kWhole);
+        VX_TRY(prefill_graph(d, m, last, form, &exec));
         hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(64), 0, d->stream, d->d_ctl, pos0 + done + m - 1, 0u, n_prompt, n_out);
         VX_HIP(hipGetLastError());
         VX_HIP(hipGraphLaunch(exec, d->stream));
