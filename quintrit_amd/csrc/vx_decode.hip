@@ -18,7 +18,8 @@
 //                     projections' outputs, RMSNorm, int8 quantization, GEMV staging, all in LDS) while its weights
 //                     are in flight, then its 16 waves split the row's chunks and add their exact int32 sums in LDS;
 //                     one wave applies the layer epilogue and stores the tile's fp32 outputs
-//   attention_kernel  per query head: RoPE of q and k, the KV append, attention
+//   attn_*_kernel     per query head: RoPE of q and k, the KV append, attention (one kernel while the context is short,
+//                     else scores and accumulator chains)
 //   head_kernel       final residual + RMSNorm, the bf16 head, and the greedy argmax across workgroups
 // Computing a stage input in every workgroup repeats a few microseconds of work that one workgroup would do alone, but
 // it runs in parallel with the weight loads and saves a launch and a wait on a single-CU kernel.
@@ -2530,7 +2531,7 @@ __global__ __launch_bounds__(kNT) void pf_stage_kernel(PfStageArgs a) {
     if (tid == 0) a.as_out[t] = sc;
 }
 
-// RoPE of every token's q and k and the KV append (the first part of attention_kernel, for n tokens): q, k, v of token
+// RoPE of every token's q and k and the KV append (as the decode step's attention does them, for n tokens): q, k, v of token
 // t from the GEMM outputs with the layer epilogue (layer.rs:246-253), rotated at the token's position (ops.rs:199-221),
 // rounded to f16; k and v into the cache, q into qbuf.
 struct PfRopeArgs {
