@@ -62,6 +62,30 @@ def test_q2_bit_exact_vs_oracle(torch_dev, oracle, rows, cols):
     mat.close()
 
 
+@pytest.mark.parametrize("rows", [31, 33, 64, 1057])                     # edges of a 32-row group, a second tile group
+@pytest.mark.parametrize("cols", [64, 2560, 2624, 5120, 5184, 12288])  # one block, whole rounds of 16 blocks and one more
+def test_q2_lone_rounds(torch_dev, oracle, rows, cols):
+    """A single GEMV around the edges of its rounds and row groups, with the widest codes (lane sums of +-512) and
+    infinite activation scales in the last block of some inputs, bit for bit (NaN where the oracle has NaN)."""
+    from quintrit_amd import _lib
+    rng = np.random.default_rng(rows * 7 + cols)
+    for wide in (False, True):
+        t, ws16, acts, as32 = make_case(oracle, rng, rows, cols)
+        if wide:
+            acts = np.full(cols, -128, np.int8)
+            t[0, :] = 1
+            t[rows - 1, :] = -1
+            as32[-1] = np.inf
+        planar = oracle.pack_matrix(t)
+        mat = _lib.Q2Matrix(planar, ws16, rows, cols)
+        got, _ = run_q2(torch_dev, mat, acts, as32)
+        want = oracle.q2_0_gemv(planar, ws16.astype(np.float32), acts, as32, rows, cols)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan)
+        assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+        mat.close()
+
+
 def test_q2_config4_shapes_and_plan(torch_dev, oracle):
     """The Qwen3-8B-like projections of configs[4] (hidden 4096, FFN 12288, q/o 4096x4096, k/v 1024x4096), one plan."""
     from quintrit_amd import _lib
