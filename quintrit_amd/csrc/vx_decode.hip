@@ -1688,6 +1688,234 @@ __global__ __launch_bounds__(256) void pf_attn_tiny_kernel(PfAttnArgs a) {
     if (has_d) a.out[row0 + d] = y * s_inv;
 }
 
+// Prefill attention of few tokens over a longer context: a workgroup per (query head, token). Its threads compute every
+// score (four lanes per position), then the factors, then each of the 4 chunks of a split context has token_waves(HD) / 4
+// waves for its accumulators, a lane token_cpl(HD) coordinates (independent chains), with kVDepth groups of 8 positions of
+// V in flight ahead of the chain, and the chunks are combined in LDS. What bounds it is the latency of these phases, but
+// only once over the context, where pf_attn_kernel alternates between them every kRange positions.
+constexpr uint32_t kVDepth = 8;
+__host__ __device__ constexpr uint32_t token_cpl(uint32_t hd) { return hd >= 256u ? hd / 128u : 1u; }
+__host__ __device__ constexpr uint32_t token_waves(uint32_t hd) { return hd >= 128u ? 8u : 4u; }
+
+template <int HD>
+__global__ __launch_bounds__(64 * token_waves(HD)) void pf_attn_token_kernel(PfAttnArgs a) {
+    constexpr uint32_t kCpl = token_cpl(HD);
+    constexpr uint32_t kWpc = token_waves(HD) / 4u;   // waves per chunk
+    constexpr uint32_t kLanes = HD / (kWpc * kCpl);   // lanes of a wave with coordinates (64, or fewer below head_dim 64)
+    constexpr uint32_t kThreads = 64u * token_waves(HD);
+    constexpr int kBlk = HD / 32;
+    __shared__ __align__(16) float sc[kAttnMaxCtx];
+    __shared__ float pm[kAttnMaxCtx];
+    __shared__ __align__(16) uint16_t qs[HD];
+    __shared__ float cm[4], cs[4];
+    __shared__ uint16_t cv[4][HD];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = blockIdx.x, kvh = h / a.gqa, t = blockIdx.y;
+    const uint32_t seq = a.ctl->pos + 2u - a.n_tok + t;
+    const KvSplit kv = kv_split(seq, a.max_ctx);
+    const uint16_t* kb = a.kc + static_cast<size_t>(kvh) * a.max_ctx * HD;
+    const uint16_t* vt = a.vc + static_cast<size_t>(kvh) * HD * a.vstride;
+    const size_t row0 = (static_cast<size_t>(t) * a.n_heads + h) * HD;
+    // this wave's chunk; the lane's coordinates are d0 + 64 m (m < kCpl) when it has any
+    const uint32_t c = wave / kWpc;
+    const uint32_t d0 = (wave % kWpc) * 64u * kCpl + lane;
+    const bool has_d = lane < kLanes;
+    const uint32_t st = c < kv.n_chunks ? c * kv.chunk : 0u;
+    const uint32_t en = c < kv.n_chunks ? min(min(st + kv.chunk, kv.n_kv), seq) : 0u;
+    if (tid < HD) qs[tid] = a.qbuf[row0 + tid];
+    __syncthreads();
+
+    // Scores, the next position's k loaded while the current one is summed.
+    {
+        const uint32_t j = tid & 3u;
+        constexpr uint32_t kGroups = kThreads / 4u;
+        auto load_k = [&](uint32_t p, uint4 (&kr)[kBlk]) {
+            const uint16_t* row = kb + static_cast<size_t>(p) * HD + 8 * j;
+#pragma unroll
+            for (int i = 0; i < kBlk; ++i) kr[i] = *reinterpret_cast<const uint4*>(row + 32 * i);
+        };
+        auto score = [&](uint32_t p, const uint4 (&kr)[kBlk]) {
+            uint32_t qo = 0;
+            asm volatile("" : "+v"(qo));  // q is read from LDS at each use (hoisted, it would take 4 kBlk registers)
+            const float s = score_dot4<HD>(qs + qo, kr, j);
+            if (j == 0) sc[p] = s * a.scale;
+        };
+        uint4 ka[kBlk], kn[kBlk];
+        uint32_t p = tid >> 2;
+        if (p < seq) load_k(p, ka);
+        for (; p < seq; p += 2u * kGroups) {  // unrolled by two so that the buffers keep their registers
+            if (p + kGroups < seq) load_k(p + kGroups, kn);
+            score(p, ka);
+            if (p + kGroups >= seq) break;
+            if (p + 2u * kGroups < seq) load_k(p + 2u * kGroups, ka);
+            score(p + kGroups, kn);
+        }
+    }
+    // V: group g holds positions 8 g .. 8 g + 7 (groups run to the chunk's end rounded up to 8, so every read is below
+    // vstride). The first kVDepth groups arrive during the scan and the exponentials.
+    const bool chain = st < en;
+    const uint32_t g_first = st / 8u, g_end = chain ? (en + 7u) / 8u : g_first + 1u;
+    const uint32_t dl = has_d ? d0 : 0u;  // a lane without coordinates reads coordinate 0 and never uses it
+    u32x4 ring[kVDepth][kCpl];
+    auto load_group = [&](uint32_t g, u32x4 (&r)[kCpl]) {
+        const uint32_t gg = min(g, g_end - 1u);
+#pragma unroll
+        for (uint32_t m = 0; m < kCpl; ++m)
+            r[m] = *reinterpret_cast<const u32x4*>(vt + (static_cast<size_t>(gg) * HD + dl + 64u * m) * 8u);
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < kVDepth; ++k) load_group(g_first + k, ring[k]);
+    __syncthreads();
+
+    if (wave < kv.n_chunks) {  // the running maximum of chunk `wave`
+        const uint32_t s0 = wave * kv.chunk, s1 = min(min(s0 + kv.chunk, kv.n_kv), seq);
+        float carry = -__builtin_inff();
+        for (uint32_t base = s0; base < s1; base += 64u) {
+            const uint32_t p = base + lane;
+            const float s = p < s1 ? sc[p] : -__builtin_inff();
+            float v = s != s ? -__builtin_inff() : s;  // NaN never moves it
+#pragma unroll
+            for (int sh = 1; sh < 64; sh <<= 1) {
+                const float o = __shfl_up(v, sh);
+                if (lane >= static_cast<uint32_t>(sh)) v = v > o ? v : o;
+            }
+            v = v > carry ? v : carry;
+            if (p < s1) pm[p] = v;
+            carry = __shfl(v, 63);
+        }
+    }
+    __syncthreads();
+
+    for (uint32_t p = tid; p < seq; p += kThreads) {
+        const float prev = p % kv.chunk == 0u ? -__builtin_inff() : pm[p - 1];
+        const float s = sc[p];
+        sc[p] = s > prev ? -glibc_expf(prev - s) : glibc_expf(s - prev);
+    }
+    __syncthreads();
+
+    // The accumulators of the lane's coordinates over positions st .. en - 1, eight positions per group; a group with no
+    // new maximum (ms = 1 throughout) takes the shorter step.
+    float y[kCpl], ssum = 0.0f;
+#pragma unroll
+    for (uint32_t m = 0; m < kCpl; ++m) y[m] = 0.0f;
+    if (chain) {
+        // the factors of the next group are read from LDS while the current group is summed, into the other of two
+        // slots (slot k & 1 of group slot k: kVDepth is even, so the pattern repeats on every pass of the loop)
+        static_assert(kVDepth % 2 == 0, "two factor slots alternate over the ring");
+        float4 fq[2][2];
+        fq[0][0] = *reinterpret_cast<const float4*>(sc + 8u * g_first);
+        fq[0][1] = *reinterpret_cast<const float4*>(sc + 8u * g_first + 4u);
+        for (uint32_t g0 = g_first; g0 < g_end; g0 += kVDepth) {
+            static_for<kVDepth>([&](auto kc) {  // the ring's slot as a constant: no rotation of its registers
+                constexpr uint32_t k = decltype(kc)::value;
+                const uint32_t gg = g0 + k;
+                {
+                    const uint32_t pn = 8u * min(gg + 1u, g_end - 1u);
+                    fq[(k + 1u) & 1u][0] = *reinterpret_cast<const float4*>(sc + pn);
+                    fq[(k + 1u) & 1u][1] = *reinterpret_cast<const float4*>(sc + pn + 4u);
+                }
+                if (gg < g_end) {  // wave-uniform
+                    u32x4(&w)[kCpl] = ring[k];
+                    const uint32_t p0 = 8u * gg;
+                    const float4 fa = fq[k & 1u][0], fb = fq[k & 1u][1];
+                    float f[8] = {fa.x, fa.y, fa.z, fa.w, fb.x, fb.y, fb.z, fb.w};
+                    // Positions outside [st, en): the factor becomes +0 (vs = 0, no new maximum) and V -0, so that a step
+                    // there adds -0 and leaves y and the sum as they are.
+                    if (p0 < st || p0 + 8u > en) {
+#pragma unroll
+                        for (uint32_t e = 0; e < 8; ++e) f[e] = p0 + e >= st && p0 + e < en ? f[e] : 0.0f;
+                        uint32_t keep[4];
+#pragma unroll
+                        for (uint32_t q = 0; q < 4; ++q) {
+                            const uint32_t pa = p0 + 2u * q, pb = pa + 1u;
+                            keep[q] = (pa >= st && pa < en ? 0xffffu : 0u) | (pb >= st && pb < en ? 0xffff0000u : 0u);
+                        }
+#pragma unroll
+                        for (uint32_t m = 0; m < kCpl; ++m) {
+                            w[m].x = (w[m].x & keep[0]) | (0x80008000u & ~keep[0]);
+                            w[m].y = (w[m].y & keep[1]) | (0x80008000u & ~keep[1]);
+                            w[m].z = (w[m].z & keep[2]) | (0x80008000u & ~keep[2]);
+                            w[m].w = (w[m].w & keep[3]) | (0x80008000u & ~keep[3]);
+                        }
+                    }
+                    auto value = [&](uint32_t m, int e) {
+                        const uint32_t word = e < 2 ? w[m].x : (e < 4 ? w[m].y : (e < 6 ? w[m].z : w[m].w));
+                        return f16_f32(static_cast<uint16_t>(word >> ((e & 1) * 16)));
+                    };
+                    uint32_t neg = 0;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) neg |= f32_bits(f[e]) >> 31;
+                    if (__builtin_amdgcn_readfirstlane(neg) == 0u) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+                            for (uint32_t m = 0; m < kCpl; ++m) y[m] = __builtin_fmaf(value(m, e), f[e], y[m]);
+                            r16_all(y);
+                            ssum = ssum + f[e];
+                        }
+                    } else {  // the full step at every position (ms = 1 where there is no new maximum)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const bool up = __builtin_signbit(f[e]);
+                            const float ev = __builtin_fabsf(f[e]);
+                            const float ms = up ? ev : 1.0f, vs = up ? 1.0f : ev;
+#pragma unroll
+                            for (uint32_t m = 0; m < kCpl; ++m) y[m] = y[m] * ms;
+                            r16_all(y);
+#pragma unroll
+                            for (uint32_t m = 0; m < kCpl; ++m) y[m] = __builtin_fmaf(value(m, e), vs, y[m]);
+                            r16_all(y);
+                            ssum = __builtin_fmaf(ssum, ms, vs);
+                        }
+                    }
+                }
+                // every slot is refilled, used or not, so that the wait for a slot is the same on every path
+                load_group(gg + kVDepth, ring[k]);
+            });
+        }
+    }
+    float* out = a.out + row0;
+    if (kv.n_chunks == 1u) {
+        if (c == 0 && has_d) {
+            const float s_inv = ssum == 0.0f ? 0.0f : 1.0f / ssum;
+#pragma unroll
+            for (uint32_t m = 0; m < kCpl; ++m) out[d0 + 64u * m] = y[m] * s_inv;
+        }
+        return;
+    }
+    if (has_d) {
+#pragma unroll
+        for (uint32_t m = 0; m < kCpl; ++m) cv[c][d0 + 64u * m] = f32_f16(y[m]);
+    }
+    if (wave % kWpc == 0 && lane == 0) {
+        cm[c] = chain ? pm[en - 1] : -__builtin_inff();
+        cs[c] = ssum;
+    }
+    __syncthreads();
+    if (c != 0 || !has_d) return;
+    // the chunks in order (attention.rs:526-541)
+#pragma unroll
+    for (uint32_t m = 0; m < kCpl; ++m) {
+        const uint32_t d = d0 + 64u * m;
+        float mf = -__builtin_inff(), sf = 0.0f, acc = 0.0f;
+        for (uint32_t k = 0; k < 4; ++k) {
+            const float sk = cs[k];
+            if (sk == 0.0f) continue;  // no positions, or a sum of zero
+            const float mk = cm[k];
+            const float mn = __builtin_fmaxf(mf, mk);
+            const float so = glibc_expf(mf - mn);
+            const float sn = glibc_expf(mk - mn);
+            const float vn = f16_f32(cv[k][d]) * sn;
+            acc = __builtin_fmaf(acc, so, vn);
+            const float ssn = sk * sn;
+            sf = __builtin_fmaf(sf, so, ssn);
+            mf = mn;
+        }
+        out[d] = sf != 0.0f ? acc * (1.0f / sf) : acc;
+    }
+}
+
 // Scores of positions p0 .. p0 + 63 (p0 = blockIdx.y * 64, below pos + 1) for up to kScoreHeads query heads of one KV
 // head (blockIdx.x: KV head, head group), so that each K row is read once for the heads that share it. The workgroup
 // whose range holds the position itself rotates its k (the first head group also appends k and v to the cache); every
@@ -2719,9 +2947,30 @@ int launch_attention_short(const AttnArgs& a, uint32_t head_dim, hipStream_t s) 
     return VX_OK;
 }
 
-// The attention of a prefill pass by the positions it reaches: below kTinyCtx, below a padded length of 512, or beyond,
-// where the context is split in chunks.
-enum class PfForm : uint32_t { kTiny, kWhole, kSplit };
+// The attention of a prefill pass: the forms of kTiny (every position below kTinyCtx) and kToken (few tokens), else the
+// tiled kernel over one chunk (kWhole) or, beyond a padded length of 512, four (kSplit).
+enum class PfForm : uint32_t { kTiny, kToken, kWhole, kSplit };
+
+// Workgroups of 16 tokens and all coordinates of a head.
+static uint32_t pf_attn_tiles(uint32_t n_heads, uint32_t n_tok, bool split) {
+    return n_heads * ((n_tok + 15u) / 16u) * (split ? 4u : 1u);
+}
+
+// The form of a pass of n_tok tokens that ends before position `end`. The split starts at a padded length of 512
+// (kv_split), so at position 256, unless max_ctx caps it below. A workgroup per (head, token) where all of them run at
+// once (its LDS admits two per CU), and up to three or four rounds of them where the tiled kernel would compute each score
+// HD / 64 = 4 times to share a head's coordinates. A call of 4 layers, tiled against this form: 12 heads of 256, 1 token
+// at position 300 307 and 284 us, 17 at 7000 1145 and 734, 33 at 7000 1467 and 900, 128 at 3500 1610 and 1229, but 200
+// (tiles of whole heads) at 3500 1371 and 1804; 20 heads of 128, 1 token at 3500 562 and 432, 24 (480 workgroups) at
+// 3500 634 and 551, 32 (640) 640 and 688; 32 heads of 64, 16 tokens (512) at 1500 413 and 397, 17 (544) 451 and 480.
+static PfForm pf_form(const vx_decoder_config_t& c, uint32_t n_tok, uint32_t end, int num_cus) {
+    if (end <= kTinyCtx) return PfForm::kTiny;
+    const bool split = c.max_ctx >= 2 * kShortCtx && end > kShortCtx;
+    const uint32_t two_per_cu = 2u * static_cast<uint32_t>(num_cus);
+    if (c.n_heads * n_tok <= two_per_cu) return PfForm::kToken;
+    if (split && c.head_dim >= 256 && pf_attn_tiles(c.n_heads, n_tok, split) < two_per_cu) return PfForm::kToken;
+    return split ? PfForm::kSplit : PfForm::kWhole;
+}
 
 template <int HD, int TOK, int POS, int W, int SL>
 static void launch_pf_attn_as(const PfAttnArgs& a, bool split, hipStream_t s) {
@@ -2741,9 +2990,12 @@ static void launch_pf_attn(const PfAttnArgs& a, int num_cus, PfForm form, hipStr
         hipLaunchKernelGGL(pf_attn_tiny_kernel<HD>, dim3(a.n_heads, a.n_tok), dim3(256), 0, s, a);
         return;
     }
+    if (form == PfForm::kToken) {
+        hipLaunchKernelGGL(pf_attn_token_kernel<HD>, dim3(a.n_heads, a.n_tok), dim3(64 * token_waves(HD)), 0, s, a);
+        return;
+    }
     const bool split = form == PfForm::kSplit;
-    const uint32_t wgs = a.n_heads * ((a.n_tok + 15u) / 16u) * (split ? 4u : 1u);
-    if (wgs < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 16, 16, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
+    if (pf_attn_tiles(a.n_heads, a.n_tok, split) < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 16, 16, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
     else launch_pf_attn_as<HD, 16, 16, 4, 1>(a, split, s);
     if (split)
         hipLaunchKernelGGL(pf_attn_combine_kernel<HD>, dim3((a.n_heads * HD + 2047u) / 2048u, a.n_tok), dim3(256), 0, s, a);
@@ -3588,11 +3840,7 @@ static int run_prefill(vx_decoder* d, uint32_t pos0, uint32_t n, uint32_t n_prom
         const uint32_t m = std::min(d->pf_cap, n - done);
         const bool last = done + m == n;
         hipGraphExec_t exec = nullptr;
-        // the split starts at a padded length of 512 (kv_split), so at position 256, unless max_ctx caps it below
-        const uint32_t end = pos0 + done + m;
-        const bool split = d->cfg.max_ctx >= 2 * kShortCtx && end > kShortCtx;
-        const PfForm form = end <= kTinyCtx ? PfForm::kTiny : (split ? PfForm::kSplit : PfForm::kWhole);
-        VX_TRY(prefill_graph(d, m, last, form, &exec));
+        VX_TRY(prefill_graph(d, m, last, pf_form(d->cfg, m, pos0 + done + m, d->num_cus), &exec));
         hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(64), 0, d->stream, d->d_ctl, pos0 + done + m - 1, 0u, n_prompt, n_out);
         VX_HIP(hipGetLastError());
         VX_HIP(hipGraphLaunch(exec, d->stream));
