@@ -3798,18 +3798,20 @@ static int record_prefill(const vx_decoder* d, uint32_t n, bool head, PfForm for
     return launch_head(h, c.emb_f16 != 0, grid, st);
 }
 
-// The graph of a prefill pass over n tokens (recorded on first use; a few are kept).
+// The graph of a prefill pass over n tokens (recorded on first use; the last four of each attention form are kept, so that
+// up to four lengths in turn record nothing, whatever positions they start at).
 static int prefill_graph(vx_decoder* d, uint32_t n, bool head, PfForm form, hipGraphExec_t* out) {
     for (const auto& g : d->pf_graphs)
         if (g.n == n && g.head == head && g.form == form) {
             *out = g.exec;
             return VX_OK;
         }
-    if (d->pf_graphs.size() >= 4) {
-        auto& g = d->pf_graphs.front();
-        (void)hipGraphExecDestroy(g.exec);
-        (void)hipGraphDestroy(g.graph);
-        d->pf_graphs.erase(d->pf_graphs.begin());
+    const auto same = [&](const vx_decoder::PfGraph& g) { return g.form == form; };
+    if (std::count_if(d->pf_graphs.begin(), d->pf_graphs.end(), same) >= 4) {
+        const auto g = std::find_if(d->pf_graphs.begin(), d->pf_graphs.end(), same);  // the oldest
+        (void)hipGraphExecDestroy(g->exec);
+        (void)hipGraphDestroy(g->graph);
+        d->pf_graphs.erase(g);
     }
     VX_HIP(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     const int st = record_prefill(d, n, head, form, d->stream);
