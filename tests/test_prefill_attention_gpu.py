@@ -4,6 +4,8 @@ and many (a workgroup per head), every head dimension, passes that start and end
 that caps the padded length at 603, so that the four chunks start at multiples of 151 (inside a group of 8 positions).
 The KV cache (the second layer's depends on the first layer's attention) and each pass' last logits equal single decode
 steps, or the oracle's loop, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -46,8 +48,22 @@ def test_prefill_attention_every_form(oracle, n_heads, head_dim, passes):
     check_passes(oracle, model, passes, head_dim)
 
 
+@pytest.mark.parametrize("head_dim,exponent", [(32, 14.4), (64, 14.3), (128, 14.25), (256, 14.25)])
+def test_prefill_attention_infinities(oracle, head_dim, exponent):
+    """Infinities in q, K and V, and the NaN that they make of scores and outputs: the first layer's attention norm is
+    scaled until a few of its f16 values overflow, first in the middle of the context (outputs of layer 0 are then finite,
+    NaN or infinite, between a few and most of them NaN). Without sub-norms a NaN output quantizes to 0 and the others to
+    their codes, so the second layer's cache shows which outputs were NaN, and stays finite."""
+    cfg = oracle.ModelConfig(2, 256, 8, 4, head_dim, 384, 500, 603, 1e-5, 10000.0, oracle.ACT_RELU2, oracle.ROPE_NORMAL, 1, 1, 0)
+    model = oracle.Model(cfg, 7)
+    gamma = (ctypes.c_float * cfg.hidden).from_address(oracle.lib().vxo_model_norm(model._h, 0, 0))
+    np.ctypeslib.as_array(gamma)[:] *= np.float32(2.0 ** exponent)
+    infinite = check_passes(oracle, model, EVERY_FORM, head_dim)
+    assert 5 <= infinite <= 300, infinite
+
+
 def check_passes(oracle, model, passes, seed):
-    """Prefills the passes and compares with the oracle."""
+    """Prefills the passes and compares with the oracle; returns how many (position, KV head) hold an infinity."""
     pre = load_decoder(oracle, model)
     try:
         n = passes[-1][1]
@@ -59,6 +75,8 @@ def check_passes(oracle, model, passes, seed):
                 _, want = model.forward(int(tokens[pos]), pos)
             assert_same_bits(got, want, f"prefill {p0}..{p1}")
         kv_equal(pre, model, model.cfg, range(n))
+        return sum(bool(np.isinf(np.concatenate(model.kv(0, pos, h)).view(np.float16)).any())
+                   for pos in range(n) for h in range(model.cfg.n_kv_heads))
     finally:
         pre.close()
         model.close()
