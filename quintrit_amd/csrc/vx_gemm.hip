@@ -191,7 +191,12 @@ struct GemmArgs {
 // buffers of fragments, 8 rows of 128 bytes each: 80 KiB for four token groups, so that two workgroups fit a CU where
 // their registers do.
 //
-// Workgroups: the token tiles of a row group run on one XCD (blockIdx.x mod 8), so that its L2 serves their weights.
+// Workgroups: the list (row group, K slice, token tile), token tiles fastest, in eight equal parts, one per XCD
+// (blockIdx.x mod 8): the token tiles that read the same weights share an L2, and every XCD has work however few row
+// groups there are. (With whole row groups per XCD, row group mod 8, most of the card idled below 8 of them and parts of
+// it at 9 to 15: 300 x 23040 x 512 36.1 -> 20.2 us, 3072 x 23040 x 64 26.4 -> 21.1, 40 x 3072 x 512 20.6 -> 11.2.) Row
+// groups in whole eights keep that assignment within the list: neighbouring row groups on one XCD instead took 14.5 us
+// against 11.8 at 8192 x 3072 x 33.
 template <int T, int R, bool RAW>
 __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs a) {
     constexpr uint32_t kFrags = 5u * T;                 // B fragments of a K step
@@ -202,9 +207,13 @@ __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs 
     __shared__ __align__(256) uint32_t tab[kLdsRows * 64u];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, half = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t slot = blockIdx.x >> 3, tt = slot % a.n_tt, rg = (slot / a.n_tt) * 8u + (blockIdx.x & 7u);
-    if (rg >= a.n_rg) return;
-    const uint32_t kz = blockIdx.z, ks0 = kz * a.steps, ks1 = min(ks0 + a.steps, a.n_ksteps), last = ks1 - 1u;
+    const uint32_t total = a.n_rg * a.kslices * a.n_tt, item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (item >= total) return;
+    uint32_t tt = 0, kz = 0, rg = item;  // (divisions only where they are needed: they cost the smallest calls 0.25 us)
+    if (a.n_tt > 1u) tt = rg % a.n_tt, rg /= a.n_tt;
+    if (a.kslices > 1u) kz = rg % a.kslices, rg /= a.kslices;
+    if (a.n_rg % 8u == 0u && a.n_rg > 8u) rg = rg % (a.n_rg >> 3) * 8u + rg / (a.n_rg >> 3);
+    const uint32_t ks0 = kz * a.steps, ks1 = min(ks0 + a.steps, a.n_ksteps), last = ks1 - 1u;
     const uint32_t blk0 = (rg * 4u + wave) * R, n_blk = 2u * a.n_tiles;
 
     // The wave's blocks: block 2 t + h is rows 32 h .. of tile t of its matrix (16 bytes a row per chunk, the chunks of a
@@ -744,7 +753,7 @@ size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus) {
 
 template <bool RAW>
 static void launch_tiles(const GemmPlan& p, const GemmArgs& a, hipStream_t stream) {
-    const dim3 grid(round_up(p.n_rg, 8) * p.n_tt, 1, p.kslices), block(256);
+    const dim3 grid(static_cast<uint32_t>(round_up(p.n_rg * p.kslices * p.n_tt, 8))), block(256);
     if (p.T == 4) {
         if (p.R == 3) hipLaunchKernelGGL((gemm_kernel<4, 3, RAW>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((gemm_kernel<4, 1, RAW>), grid, block, 0, stream, a);

@@ -102,14 +102,34 @@ def test_gemm_config2_equals_bruteforce(torch_dev, oracle, rows, cols):
                                          (200, 2656, 90), (5000, 2672, 100), (60, 112, 33), (300, 14992, 200),
                                          (1000, 80, 129)])
 def test_gemm_tiles(torch_dev, oracle, rows, cols, m, pad):
-    """The tiled kernel (more than 32 tokens) in each of its tiles, with and without K slices, at the edges of row blocks
-    and token groups, with packed tails of one and of two chunks, against a float64 product (exact)."""
+    """The tiled kernel (more than 32 tokens) on x itself (cols in whole 16-byte pieces) in each of its tiles, with and
+    without K slices, at the edges of row blocks and token groups, with packed tails of one and of two chunks, against a
+    float64 product (exact)."""
+    check_gemm(torch_dev, oracle, rows, cols, m, cols + pad)
+
+
+def check_gemm(torch, oracle, rows, cols, m, ldx):
     from quintrit_amd import VelurexHipLayer
-    print(f"[gemm tiles] {rows}x{cols} m={m} pad={pad}", flush=True)
+    print(f"[gemm] {rows}x{cols} m={m} ldx={ldx}", flush=True)
     rng = np.random.default_rng(rows + cols + m)
     t = rng.integers(-1, 2, size=(rows, cols), dtype=np.int8)
     x = rng.integers(-128, 128, size=(m, cols), dtype=np.int8)
     layer = VelurexHipLayer(oracle.pack_matrix(t), rows, cols, 1.0)
-    got = gemm(torch_dev, layer, x, ldx=cols + pad)
+    got = gemm(torch, layer, x, ldx=ldx)
     assert np.array_equal(got.astype(np.float64), x.astype(np.float64) @ t.astype(np.float64).T)
     layer.close()
+
+
+# The plan on 256 CUs: tile (token groups, row blocks), K slices and steps, row groups.
+@pytest.mark.parametrize("rows,cols,m", [(24001, 641, 480),     # 4 x 3, 63 row groups
+                                         (13825, 337, 500),     # 4 x 1, 109 row groups
+                                         (33000, 337, 64),      # 2 x 2, 129 row groups
+                                         (12000, 5003, 60),     # 2 x 2, 4 slices of 8 steps, 47 row groups
+                                         (5000, 14001, 500),    # 4 x 1, 3 slices of 30 steps, 40 row groups
+                                         (3072, 23041, 512),    # 4 x 1, 5 slices of 29 steps, 24 row groups
+                                         (300, 4003, 300),      # 2 x 1, 9 slices of 3 steps, 3 row groups
+                                         (513, 12001, 200)])    # 2 x 1, 11 slices of 7 steps, 5 row groups
+def test_gemm_tiles_staged(torch_dev, oracle, rows, cols, m):
+    """The tiled kernel on fragments that the staging kernel has written (cols not a multiple of 16), in each of its tiles,
+    with row groups below, in and beside whole eights, against a float64 product (exact)."""
+    check_gemm(torch_dev, oracle, rows, cols, m, cols)
