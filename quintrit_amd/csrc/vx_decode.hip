@@ -3615,7 +3615,7 @@ static int ensure_prefill(vx_decoder* d) {
         GemmSub subs[kMaxStageJobs];
         int k = 0;
         for (; k < kMaxStageJobs && kinds[k] >= 0; ++k) subs[k] = GemmSub{nullptr, &d->proj[kinds[k]]->g, nullptr, 0};
-        for (uint32_t m = 1; m <= cap; ++m) part_bytes = std::max(part_bytes, gemm_group_part_bytes(subs, k, m, d->num_cus));
+        for (uint32_t m = 1; m <= cap; ++m) part_bytes = std::max(part_bytes, gemm_group_part_bytes(subs, k, m, m <= kGemmSmallM, d->num_cus));
     }
     hipError_t e = hipSuccess;
     auto grab = [&](auto** p, size_t bytes) {

@@ -194,7 +194,7 @@ struct GemmArgs {
 // Workgroups: the list (row group, K slice, token tile), token tiles fastest, in eight equal parts, one per XCD
 // (blockIdx.x mod 8): the token tiles that read the same weights share an L2, and every XCD has work however few row
 // groups there are. (With whole row groups per XCD, row group mod 8, most of the card idled below 8 of them and parts of
-// it at 9 to 15: 300 x 23040 x 512 36.1 -> 20.2 us, 3072 x 23040 x 64 26.4 -> 21.1, 40 x 3072 x 512 20.6 -> 11.2.) Row
+// it at 9 to 15: 300 x 23040 x 512 36.1 -> 20.2 us, 3072 x 23040 x 64 26.4 -> 21.1, 40 x 3072 x 512 20.6 -> 9.8.) Row
 // groups in whole eights keep that assignment within the list: neighbouring row groups on one XCD instead took 14.5 us
 // against 11.8 at 8192 x 3072 x 33.
 template <int T, int R, bool RAW>
@@ -437,26 +437,24 @@ __global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs a) {
     sb.y[static_cast<size_t>(m) * sb.ldy + ln] = (s0 + s1) + (s2 + s3);
 }
 
-// ---- one token group (M <= 32): one launch ------------------------------------------------------------------------
+// ---- one or two token groups: one launch --------------------------------------------------------------------------
 
-// Workgroup (c, kz): W waves, wave w the 64-row tile W c + w, over the K steps of slice kz (at most
-// kSmallSteps), for one group of 32 tokens. G: the call's tiles may belong to several matrices of the
-// same columns (each wave finds its own; without G the instance reads only the first). Each thread first loads the activations of its B-fragment tasks (task = step, token
-// group, half, token) and the trit table's entries, then each wave loads all its weights of the slice at once (2
-// chunks per K step per lane, every load unconditional: steps past the slice read its last step again), so
-// the wait for the activations and the table does
-// not include the weights' latency (loads return in order); the
-// workgroup then builds the trit table and the slice's B fragments in LDS (the staging of gemm_stage_kernel, so no
-// staging kernel runs) and each wave multiplies with no further barrier. With one slice the wave writes Y; otherwise
-// it stores its slice's sums, which gemm_small_finish_kernel adds. (Gathering them in the kernel instead, each tile's
-// last slice reading the others' sums with agent-scope atomic loads after a ticket, was slower: 30-160 us per call
-// at M = 8-32.)
+// Workgroup (c, kz): W waves, wave w the 64-row tile W c + w, over the K steps of slice kz (at most kSmallSteps), for T
+// groups of 32 tokens. G: the call's tiles may belong to several matrices of the same columns (each wave finds its own;
+// without G the instance reads only the first). Each thread first loads the activations of its B-fragment tasks (task =
+// step, token group, half, token) and the trit table's entries, then each wave loads all its weights of the slice at once
+// (2 chunks per K step per lane, every load unconditional: steps past the slice read its last step again), so the wait
+// for the activations and the table does not include the weights' latency (loads return in order); the workgroup then
+// builds the trit table and the slice's B fragments in LDS (the staging of gemm_stage_kernel, so no staging kernel runs)
+// and each wave multiplies with no further barrier. With one slice the wave writes Y; otherwise it stores its slice's
+// sums, which gemm_finish_kernel adds. (Gathering them in the kernel instead, each tile's last slice reading the others'
+// sums with agent-scope atomic loads after a ticket, was slower: 30-160 us per call at M = 8-32.)
 constexpr uint32_t kSmallSteps = 8;  // K steps per slice at most (40 KiB of B fragments per token group in LDS)
 
-template <int W, bool G>
+template <int T, int W, bool G, bool TOKENS>
 __global__ __launch_bounds__(W * 64) void gemm_small_kernel(GemmArgs a) {
     __shared__ uint32_t tab[256 * 64];
-    constexpr uint32_t S = kSmallSteps, T = 1;
+    constexpr uint32_t S = kSmallSteps;
     __shared__ uint4 bs[S * 5 * T * 64];
     constexpr uint32_t kTasks = S * T / W;  // B-fragment tasks per thread
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -634,10 +632,29 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(GemmArgs a) {
             for (int g = 0; g < T; ++g) {
                 const uint4 b = bs[((s * 5u + kb) * T + g) * 64u + lane];
                 const v4i B = v4i{static_cast<int>(b.x), static_cast<int>(b.y), static_cast<int>(b.z), static_cast<int>(b.w)};
-                acc[0][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B, A[0][kb], acc[0][g], 0, 0, 0);
-                acc[1][g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B, A[1][kb], acc[1][g], 0, 0, 0);
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb)
+                    acc[rb][g] = TOKENS ? __builtin_amdgcn_mfma_i32_32x32x32_i8(A[rb][kb], B, acc[rb][g], 0, 0, 0)
+                                        : __builtin_amdgcn_mfma_i32_32x32x32_i8(B, A[rb][kb], acc[rb][g], 0, 0, 0);
             }
         }
+    }
+    if constexpr (TOKENS) {
+        // Lane l holds token l % 32 of the group and, in register r, row 8 (r / 4) + 4 (l / 32) + r % 4 of block rb: a slice's
+        // sums go out as 16-byte pieces.
+#pragma unroll
+        for (int g = 0; g < T; ++g) {
+            const uint32_t m = 32u * g + (lane & 31u);
+            if (m >= a.M) continue;
+            int32_t* out = a.part + (static_cast<size_t>(kz) * a.M + m) * a.rows_p + sb.row0 + lt * 64u + 4u * half;
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4)
+                    *reinterpret_cast<int4*>(out + rb * 32 + 8 * r4) =
+                        make_int4(acc[rb][g][4 * r4], acc[rb][g][4 * r4 + 1], acc[rb][g][4 * r4 + 2], acc[rb][g][4 * r4 + 3]);
+        }
+        return;
     }
     // The product is transposed as gemm_kernel's: lane l holds row l % 32 of block rb and, in register r, token 8 (r / 4) +
     // 4 (l / 32) + r % 4, so that a store writes 128 consecutive bytes of two tokens.
@@ -648,40 +665,41 @@ __global__ __launch_bounds__(W * 64) void gemm_small_kernel(GemmArgs a) {
         const uint32_t n = lt * 64u + rb * 32u + (lane & 31u);
         if (a.kslices == 1 && n >= sb.rows) continue;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
+        for (int r4 = 0; r4 < 4 * T; ++r4) {
             if (8u * r4 >= a.M) break;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const uint32_t m = 8u * r4 + 4u * half + e;
-                if (m < a.M) out[static_cast<size_t>(m) * ld + n] = acc[rb][0][4 * r4 + e];
+                if (m < a.M) out[static_cast<size_t>(m) * ld + n] = acc[rb][r4 / 4][4 * (r4 % 4) + e];
             }
         }
     }
 }
 
-// The small kernel's shape: waves per workgroup (4 or 8) and K steps per slice (2 to kSmallSteps). A round is one
-// workgroup per CU (the trit table and the B fragments take 104-144 KiB of LDS); a round costs about 3 K steps of
-// loads and staging plus its K steps, each W / 4 one-wave steps of matrix-core work per SIMD, and the finish
-// about a quarter step per slice (measured at the configs[2] shapes). The cheapest pair; on a tie the longer slices.
+// The small kernel's shape for T token groups: waves per workgroup (4 or 8) and K steps per slice (2 to kSmallSteps). A
+// round is one workgroup per CU (the trit table and the B fragments take 104-144 KiB of LDS); a round costs about 3 K
+// steps of loads and staging plus its K steps, each T W / 4 one-wave steps of matrix-core work per SIMD, and the finish
+// about a quarter step per slice (measured at 23040 x 3072 and 3072 x 23040). The cheapest pair; on a tie the longer slices.
 struct SmallShape {
     uint32_t waves, steps, kslices;
 };
 
-static SmallShape small_shape(const Geometry& g, int num_cus) {
-    const uint64_t n_ksteps = (g.n_chunks + kStepChunks - 1) / kStepChunks;
-    const uint64_t cus = static_cast<uint64_t>(std::max(num_cus, 1));
+static SmallShape small_shape(const Geometry& g, int num_cus, uint32_t T) {
+    const uint32_t n_ksteps = static_cast<uint32_t>((g.n_chunks + kStepChunks - 1) / kStepChunks);
+    const uint32_t n_tiles = static_cast<uint32_t>(g.n_tiles), cus = static_cast<uint32_t>(std::max(num_cus, 1));
     double best = 1e300;
     SmallShape sh{4, kSmallSteps, 1};
-    for (uint32_t st = kSmallSteps; st >= 2; --st)
+    for (uint32_t st = kSmallSteps; st >= 2; --st) {
+        const uint32_t ks = (n_ksteps + st - 1) / st;
         for (uint32_t w : {4u, 8u}) {
-            const uint64_t ks = (n_ksteps + st - 1) / st;
-            const uint64_t rounds = ((g.n_tiles + w - 1) / w * ks + cus - 1) / cus;
-            const double cost = static_cast<double>(rounds) * (3.0 + st * w / 4.0) + (ks > 1 ? 0.25 * ks : 0.0);
+            const uint32_t rounds = ((n_tiles + w - 1) / w * ks + cus - 1) / cus;
+            const double cost = static_cast<double>(rounds) * (3.0 + st * T * w / 4.0) + (ks > 1 ? 0.25 * ks : 0.0);
             if (cost < best - 1e-9) {
                 best = cost;
-                sh = SmallShape{w, st, static_cast<uint32_t>(ks)};
+                sh = SmallShape{w, st, ks};
             }
         }
+    }
     return sh;
 }
 
@@ -694,10 +712,12 @@ static Geometry group_geometry(const GemmSub* subs, int n) {
     return geometry(rows_p, subs[0].g->cols);
 }
 
+static uint32_t token_groups(size_t M) { return static_cast<uint32_t>((M + 31) / 32); }
+
 size_t gemm_ksteps(size_t cols) { return (geometry(1, cols).n_chunks + kStepChunks - 1) / kStepChunks; }
 
 size_t gemm_stage_bytes(size_t cols, size_t M) {
-    return M <= kGemmSmallM ? 0 : round_up(gemm_ksteps(cols) * 5u * ((M + 31) / 32) * 1024u, 256);
+    return M <= kGemmSmallM ? 0 : round_up(gemm_ksteps(cols) * 5u * token_groups(M) * 1024u, 256);
 }
 
 struct GemmPlan {
@@ -712,7 +732,7 @@ struct GemmPlan {
 // (14 % at worst). Slice sums are kept within the scratch of the no-allocation entry point.
 static GemmPlan gemm_plan(const Geometry& g, size_t M, int num_cus) {
     const uint32_t n_ksteps = static_cast<uint32_t>(gemm_ksteps(g.cols));
-    const uint32_t n_tg = static_cast<uint32_t>((M + 31) / 32);
+    const uint32_t n_tg = token_groups(M);
     const uint64_t blocks = 2 * g.n_tiles, cus = static_cast<uint64_t>(std::max(num_cus, 1));
     const size_t xs = gemm_stage_bytes(g.cols, M), out = M * g.padded_rows * 4u;
     GemmPlan best{};
@@ -740,15 +760,30 @@ static GemmPlan gemm_plan(const Geometry& g, size_t M, int num_cus) {
     return best;
 }
 
-size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, int num_cus) {
+// Whether a call on x itself (raw; fragments that the caller has staged take the tiled kernel) of more than 32 tokens takes
+// the small kernel with two token groups: in one round of workgroups of long slices, where all of a slice's weights in
+// flight beat the tiled kernel's three steps ahead. Small against tiled at 33 and 64 tokens: 3072 x 23040 (7 K steps) 15.9
+// against 19.1 and 19.2 against 20.6 us, 8192 x 6912 (6) 12.7 against 14.5 and 15.8 against 18.2, 4000 x 18000 (8) 14.5
+// against 17.2 and 17.6 against 19.4 (at worst, 4000 x 16001 x 64, 22.7 against 20.3); with shorter slices 3072 x 14336
+// (5) 15.7 against 16.9 and 19.6 against 17.1, 2560 x 9216 (3) 13.1 against 12.1 and 17.1 against 14.3; beyond 128 tiles
+// 17132 x 2562 x 63 (6) 25.7 against 15.9.
+static bool small_form(const Geometry& g, size_t M, bool raw, int num_cus) {
+    if (M <= kGemmSmallM) return true;
+    if (!raw || M > 64) return false;  // (raw calls are of one matrix)
+    const SmallShape sh = small_shape(g, num_cus, 2u);
+    return g.n_tiles <= 128u && sh.waves == 4u && sh.steps >= 6u && sh.kslices > 1u &&
+           (g.n_tiles + 3) / 4 * sh.kslices <= static_cast<size_t>(std::max(num_cus, 1));
+}
+
+size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, bool raw, int num_cus) {
     const Geometry g = group_geometry(subs, n);
-    const uint32_t ks = M <= kGemmSmallM ? small_shape(g, num_cus).kslices : gemm_plan(g, M, num_cus).kslices;
+    const uint32_t ks = small_form(g, M, raw, num_cus) ? small_shape(g, num_cus, token_groups(M)).kslices : gemm_plan(g, M, num_cus).kslices;
     return ks > 1 ? round_up(static_cast<size_t>(ks) * M * g.padded_rows * 4u, 256) : 0;
 }
 
 size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus) {
     const GemmSub sub{nullptr, &g, nullptr, 0};
-    return std::max<size_t>(gemm_stage_bytes(g.cols, M) + gemm_group_part_bytes(&sub, 1, M, num_cus), 256);
+    return std::max<size_t>(gemm_stage_bytes(g.cols, M) + gemm_group_part_bytes(&sub, 1, M, true, num_cus), 256);
 }
 
 template <bool RAW>
@@ -760,6 +795,22 @@ static void launch_tiles(const GemmPlan& p, const GemmArgs& a, hipStream_t strea
     } else {
         if (p.R == 2) hipLaunchKernelGGL((gemm_kernel<2, 2, RAW>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((gemm_kernel<2, 1, RAW>), grid, block, 0, stream, a);
+    }
+}
+
+// Slices of more than 16 tokens are stored with the tokens in the lanes (8 stores a wave and token group instead of up to
+// 32: 300 x 1600 x 32 7.4 -> 7.1 us, 1024 x 3072 x 32 11.1 -> 10.7); at 8 tokens both take as many, and rows in the lanes
+// write whole lines (3072 x 23040 x 8 11.1 -> 10.8).
+template <int W>
+static void launch_small(const GemmArgs& a, hipStream_t stream) {
+    const dim3 grid((a.n_tiles + W - 1) / W, a.kslices), block(W * 64);
+    const bool tokens = a.kslices > 1u && a.M > 16u;
+    if (a.n_sub > 1u) {
+        if (tokens) hipLaunchKernelGGL((gemm_small_kernel<1, W, true, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((gemm_small_kernel<1, W, true, false>), grid, block, 0, stream, a);
+    } else {
+        if (tokens) hipLaunchKernelGGL((gemm_small_kernel<1, W, false, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((gemm_small_kernel<1, W, false, false>), grid, block, 0, stream, a);
     }
 }
 
@@ -789,19 +840,16 @@ int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, 
     a.n_chunks = static_cast<uint32_t>(g.n_chunks);
     a.n_ksteps = static_cast<uint32_t>((g.n_chunks + kStepChunks - 1) / kStepChunks);
     a.M = static_cast<uint32_t>(M);
-    a.n_tg = static_cast<uint32_t>((M + 31) / 32);
-    if (M <= kGemmSmallM) {
-        const SmallShape sh = small_shape(g, num_cus);
+    a.n_tg = token_groups(M);
+    if (small_form(g, M, x != nullptr, num_cus)) {
+        const SmallShape sh = small_shape(g, num_cus, token_groups(M));
         a.kslices = sh.kslices;
         a.steps = sh.steps;
-        const dim3 grid((a.n_tiles + sh.waves - 1) / sh.waves, a.kslices), block(sh.waves * 64);
-        if (n > 1) {
-            if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<8, true>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((gemm_small_kernel<4, true>), grid, block, 0, stream, a);
-        } else {
-            if (sh.waves == 8) hipLaunchKernelGGL((gemm_small_kernel<8, false>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((gemm_small_kernel<4, false>), grid, block, 0, stream, a);
-        }
+        if (M > kGemmSmallM) {  // small_form: several slices of one matrix, 4 waves
+            if (n != 1 || sh.waves != 4u || sh.kslices < 2u) VX_FAIL(VX_ERR_INTERNAL, "a small GEMM of %zu tokens", M);
+            hipLaunchKernelGGL((gemm_small_kernel<2, 4, false, true>), dim3((a.n_tiles + 3) / 4, a.kslices), dim3(256), 0, stream, a);
+        } else if (sh.waves == 8) launch_small<8>(a, stream);
+        else launch_small<4>(a, stream);
     } else {
         const GemmPlan p = gemm_plan(g, M, num_cus);
         a.kslices = p.kslices;

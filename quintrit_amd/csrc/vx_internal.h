@@ -228,15 +228,16 @@ struct GemmSub {
     int32_t* y;
     size_t ldy;
 };
-// Up to 3 matrices with the same columns in one launch (their tiles concatenated). Up to 32 tokens one kernel builds the
-// B fragments of its K slice from x; more tokens run the tiled kernel, on x itself where its rows allow 16-byte pieces,
-// else after a staging kernel that writes the fragments to `staged` (gemm_stage_bytes); a finish kernel adds the K
-// slices when there are several, from `part` (gemm_group_part_bytes). gemm_workspace_bytes is the sum of both. x may be
-// null where the caller has written the fragments (gemm_fragment) to `staged`.
+// Up to 3 matrices with the same columns in one launch (their tiles concatenated). Up to 32 tokens (and for some long rows
+// up to 64) one kernel builds the B fragments of its K slice from x; more tokens run the tiled kernel, on x itself where
+// its rows allow 16-byte pieces, else after a staging kernel that writes the fragments to `staged` (gemm_stage_bytes); a
+// finish kernel adds the K slices when there are several, from `part` (gemm_group_part_bytes; raw: of a call on x).
+// gemm_workspace_bytes is the sum of both. x may be null where the caller has written the fragments (gemm_fragment) to
+// `staged`.
 constexpr size_t kGemmSmallM = 32;  // tokens of the kernel without staged fragments
 size_t gemm_ksteps(size_t cols);
 size_t gemm_stage_bytes(size_t cols, size_t M);
-size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, int num_cus);
+size_t gemm_group_part_bytes(const GemmSub* subs, int n, size_t M, bool raw, int num_cus);
 size_t gemm_workspace_bytes(const Geometry& g, size_t M, int num_cus);
 int launch_gemm_group(const GemmSub* subs, int n, int num_cus, const int8_t* x, size_t M, size_t ldx, uint8_t* staged,
                       uint8_t* part, hipStream_t stream);

@@ -133,3 +133,11 @@ def test_gemm_tiles_staged(torch_dev, oracle, rows, cols, m):
     """The tiled kernel on fragments that the staging kernel has written (cols not a multiple of 16), in each of its tiles,
     with row groups below, in and beside whole eights, against a float64 product (exact)."""
     check_gemm(torch_dev, oracle, rows, cols, m, cols)
+
+
+@pytest.mark.parametrize("rows,cols,m", [(3072, 20003, 40), (2500, 23043, 64), (6000, 9001, 49), (8192, 6912, 33),
+                                         (1024, 3072, 16), (1024, 3072, 17), (300, 1600, 32), (1023, 1601, 31)])
+def test_gemm_small_forms(torch_dev, oracle, rows, cols, m):
+    """The small kernel with two token groups (long rows, 33 to 64 tokens, K slices of 6 steps or more), and with one on both
+    sides of the token count from which a slice's sums are stored with the tokens in the lanes."""
+    check_gemm(torch_dev, oracle, rows, cols, m, cols + 3)
