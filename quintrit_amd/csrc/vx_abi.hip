@@ -66,7 +66,6 @@ static int set_device_of(const vx_matrix_t* m) {
 
 static void destroy(vx_matrix* m) {
     if (m->d_w) (void)hipFree(m->d_w);
-    if (m->d_part) (void)hipFree(m->d_part);
     if (m->d_accum) (void)hipFree(m->d_accum);
     if (m->d_dsum) (void)hipFree(m->d_dsum);
     if (m->d_staged) (void)hipFree(m->d_staged);
@@ -101,7 +100,6 @@ static int alloc_matrix(size_t rows, size_t cols, float weight_scale, vx_matrix*
     m->device = di.device;
     m->num_cus = di.num_cus;
     m->d_w = nullptr;
-    m->d_part = nullptr;
     m->d_accum = nullptr;
     m->d_tickets = nullptr;
     m->d_done = nullptr;
@@ -109,14 +107,10 @@ static int alloc_matrix(size_t rows, size_t cols, float weight_scale, vx_matrix*
     m->d_staged = nullptr;
     m->d_io = nullptr;
     m->owner = nullptr;
-    Job probe{};
-    plan_job(probe, m->g, static_cast<uint32_t>(di.num_cus));
-    m->kslices = probe.kslices;
-    m->slice_chunks = probe.slice_chunks;
+    m->lone = lone_plan(m->g, di.num_cus);
 
     const size_t io_bytes = round_up(cols, 256) + m->g.padded_rows * 4;
     hipError_t e = hipMalloc(&m->d_w, m->g.device_bytes);
-    if (e == hipSuccess && m->kslices > 1) e = hipMalloc(&m->d_part, static_cast<size_t>(m->kslices) * m->g.padded_rows * 4);
     // the atomic slice sums and tickets of the lone calls (the table GEMV splits K more finely than the digit GEMV,
     // so every matrix has them)
     const size_t accum_bytes = (m->g.padded_rows + m->g.n_tiles + 1) * 4;
@@ -203,11 +197,44 @@ static int check_io(const vx_matrix_t* m, const void* acts, size_t acts_len, con
     return VX_OK;
 }
 
+// A lone GEMV of matrix m by gemv_kernel: a workgroup takes 16 tiles and one K slice (`device`: by m's plan; else as many
+// slices as fill the CUs). Activations staged, or (raw) int8 that every workgroup stages for its own slice. With `flag`,
+// the launch's last workgroup stores `seq` there once every output is written.
+static int run_single_grouped(const vx_matrix* m, const uint8_t* staged, const int8_t* raw, void* out, uint32_t out_kind,
+                              float post, hipStream_t s, bool device, uint32_t* flag = nullptr, uint32_t seq = 0) {
+    LaunchArgs a{};
+    a.done = flag != nullptr ? m->d_done : nullptr;
+    a.flag = flag;
+    a.seq = seq;
+    a.acts = raw;
+    a.cols = static_cast<uint32_t>(m->g.cols);
+    a.n_jobs = 1;
+    Job& j = a.one;
+    plan_job(j, m->g, device ? 0u : static_cast<uint32_t>(m->num_cus));
+    if (device) {
+        j.kslices = m->lone.kslices;
+        j.slice_chunks = m->lone.slice_chunks;
+    }
+    j.w = m->d_w;
+    j.staged = staged;
+    j.accum = m->d_accum;
+    j.tickets = m->d_tickets;
+    j.dsum = m->d_dsum;
+    j.out = out;
+    j.post = post;
+    j.weight_scale = m->weight_scale;
+    j.out_kind = out_kind;
+    j.tbr = static_cast<uint32_t>(m->g.tbr);
+    a.total_items = job_items(j);
+    return launch_gemv(a, j.rows, nullptr, 0u, m->num_cus, s);
+}
+
 // A lone GEMV of matrix m on activations in device memory, staged or (raw) int8: one launch (a split row's K slices add
-// their sums atomically and the last of each tile writes the outputs). Calls on one matrix share its sums and tickets,
-// so they must not overlap.
+// their sums atomically and the last of each tile, or tile group, writes the outputs). Calls on one matrix share its sums
+// and tickets, so they must not overlap.
 static int run_single(const vx_matrix* m, const uint8_t* staged, const int8_t* raw, void* out, uint32_t out_kind, float post,
                       hipStream_t s) {
+    if (!m->lone.tiled) return run_single_grouped(m, staged, raw, out, out_kind, post, s, true);
     LoneArgs a{};
     a.w = m->d_w;
     a.acts = raw;
@@ -223,35 +250,9 @@ static int run_single(const vx_matrix* m, const uint8_t* staged, const int8_t* r
     a.tbr = static_cast<uint32_t>(m->g.tbr);
     a.n_tiles = static_cast<uint32_t>(m->g.n_tiles);
     a.n_chunks = static_cast<uint32_t>(m->g.n_chunks);
+    a.kslices = m->lone.kslices;
+    a.slice_chunks = m->lone.slice_chunks;
     return launch_gemv_lone(a, s);
-}
-
-// The same on host memory (vx_layer_forward): acts and out are pinned host buffers that the kernel reads and writes over
-// the bus, and the launch's last workgroup stores `seq` in `flag` once every output is written. A workgroup takes 16 tiles
-// and one of many K slices, so that the activations cross the bus once per 16 tiles and not once per tile.
-static int run_single_host(const vx_matrix* m, const int8_t* acts, void* out, float post, hipStream_t s, uint32_t* flag,
-                           uint32_t seq) {
-    LaunchArgs a{};
-    a.done = m->d_done;
-    a.flag = flag;
-    a.seq = seq;
-    a.acts = acts;
-    a.cols = static_cast<uint32_t>(m->g.cols);
-    a.n_jobs = 1;
-    Job& j = a.one;
-    plan_job(j, m->g, static_cast<uint32_t>(m->num_cus));
-    j.w = m->d_w;
-    j.part = m->d_part;
-    j.accum = m->d_accum;
-    j.tickets = m->d_tickets;
-    j.dsum = m->d_dsum;
-    j.out = out;
-    j.post = post;
-    j.weight_scale = m->weight_scale;
-    j.out_kind = kOutF32Post;
-    j.tbr = static_cast<uint32_t>(m->g.tbr);
-    a.total_items = job_items(j);
-    return launch_gemv(a, j.rows, nullptr, 0u, m->num_cus, s);
 }
 
 // A lone GEMV of matrix m through the compact activation tables `lut` (its K slices add up in m's atomic sums, as
@@ -605,9 +606,11 @@ int vx_layer_forward(const vx_matrix_t* matrix, const int8_t* acts, size_t acts_
         const uint32_t seq = m->io_seq + 1u == 0u ? 1u : m->io_seq + 1u;  // never 0, the buffer's initial value
         m->io_seq = seq;
         std::memcpy(m->h_io, acts, m->g.cols);
-        VX_TRY(run_single_host(m, reinterpret_cast<const int8_t*>(m->h_io_dev), m->h_io_dev + out_off,
-                               m->weight_scale / act_scale, m->io_stream, reinterpret_cast<uint32_t*>(m->h_io_dev + flag_off),
-                               seq));
+        // pinned host buffers that the kernel reads and writes over the bus: 16 tiles and one of many short K slices per
+        // workgroup, so that the activations cross the bus once per 16 tiles and not once per tile
+        VX_TRY(run_single_grouped(m, nullptr, reinterpret_cast<const int8_t*>(m->h_io_dev), m->h_io_dev + out_off, kOutF32Post,
+                                  m->weight_scale / act_scale, m->io_stream, false,
+                                  reinterpret_cast<uint32_t*>(m->h_io_dev + flag_off), seq));
         // Wait for the flag; every 65536 reads (tens of microseconds, longer than a call), ask the stream whether it
         // has ended (an error, or an end without the flag, is reported instead of waiting on).
         for (uint32_t i = 1;; ++i) {
@@ -977,10 +980,8 @@ int vx_q2_matrix_create(const uint8_t* planar, size_t planar_len, const uint16_t
         m->weight_scale = 1.0f;
         m->device = di.device;
         m->num_cus = di.num_cus;
-        m->kslices = 1;
-        m->slice_chunks = 0;
+        m->lone = LonePlan{};
         m->d_w = nullptr;
-        m->d_part = nullptr;
         m->d_dsum = nullptr;
         m->d_staged = nullptr;
         m->d_io = nullptr;

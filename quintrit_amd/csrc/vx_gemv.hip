@@ -609,7 +609,7 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
     const uint32_t grid = std::min<uint32_t>(a.total_items, 2u * static_cast<uint32_t>(num_cus));
     if (a.jobs) hipLaunchKernelGGL((gemv_kernel<true, false>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
     else if (a.acts) hipLaunchKernelGGL((gemv_kernel<false, true>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
-    else VX_FAIL(VX_ERR_INTERNAL, "a lone GEMV without activations");
+    else hipLaunchKernelGGL((gemv_kernel<false, false>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
     VX_HIP(hipGetLastError());
     if (n_split) {
         const dim3 fgrid((max_rows + 63u) / 64u, n_split);
@@ -620,11 +620,20 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
     return VX_OK;
 }
 
-// A lone GEMV's K slices: one while a row has at most kLoneChunks chunks, else the fewest, of equal length.
-int launch_gemv_lone(LoneArgs a, hipStream_t stream) {
-    a.kslices = (a.n_chunks + kLoneChunks - 1u) / kLoneChunks;
-    a.slice_chunks = (a.n_chunks + a.kslices - 1u) / a.kslices;
-    a.kslices = (a.n_chunks + a.slice_chunks - 1u) / a.slice_chunks;
+LonePlan lone_plan(const Geometry& g, int num_cus) {
+    const uint32_t nc = static_cast<uint32_t>(g.n_chunks), cus = static_cast<uint32_t>(num_cus);
+    LonePlan p{true, (nc + kLoneChunks - 1u) / kLoneChunks, 0};
+    p.tiled = g.n_tiles * p.kslices <= 2u * static_cast<size_t>(cus);
+    if (!p.tiled) {
+        const uint32_t groups = static_cast<uint32_t>(g.n_groups), least = (nc + kMaxSliceChunks - 1) / kMaxSliceChunks;
+        p.kslices = std::max(least, std::max(1u, std::min(nc / 3u, cus / groups)));
+    }
+    p.slice_chunks = (nc + p.kslices - 1u) / p.kslices;
+    p.kslices = (nc + p.slice_chunks - 1u) / p.slice_chunks;
+    return p;
+}
+
+int launch_gemv_lone(const LoneArgs& a, hipStream_t stream) {
     const dim3 grid(a.n_tiles, a.kslices);
     if (a.acts != nullptr) hipLaunchKernelGGL(gemv_lone_kernel<true>, grid, dim3(kWaves * 64), 0, stream, a);
     else hipLaunchKernelGGL(gemv_lone_kernel<false>, grid, dim3(kWaves * 64), 0, stream, a);

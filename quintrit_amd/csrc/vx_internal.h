@@ -212,10 +212,21 @@ struct LoneArgs {
     float post;         // kOutF32Post
     uint32_t out_kind;  // kOutI32 or kOutF32Post
     uint32_t rows, cols, tbr, n_tiles, n_chunks;
-    uint32_t kslices, slice_chunks;  // set by launch_gemv_lone
+    uint32_t kslices, slice_chunks;
 };
 constexpr uint32_t kLoneChunks = 64;  // chunks of a K slice at most: 4 per wave
-int launch_gemv_lone(LoneArgs a, hipStream_t stream);
+// How a lone GEMV on activations in device memory runs. tiled: gemv_lone_kernel, a workgroup per tile and K slice (one
+// slice while a row has at most kLoneChunks chunks, else the fewest, of equal length), while all of its workgroups, two to
+// a CU, run at once (raw, 512 workgroups: 30000 x 3072 8.5 against 9.8 us, 8192 x 20000 11.8 against 11.9). Beyond that
+// gemv_kernel, 16 tiles and a K slice per workgroup, in slices of 3 chunks at least, rounded down to at most one workgroup
+// per CU where they are short enough: 36000 x 2000 8.2 against 10.0, 20000 x 9000 12.8 against 15.6, 23040 x 23040 22.3
+// against 32.5. (Rounded up, a few CUs with two workgroups set the time: 23040 x 9000 16.9 -> 12.8.)
+struct LonePlan {
+    bool tiled;
+    uint32_t kslices, slice_chunks;
+};
+LonePlan lone_plan(const Geometry& g, int num_cus);
+int launch_gemv_lone(const LoneArgs& a, hipStream_t stream);
 int launch_device_layout(const uint8_t* planar_dev, const Geometry& g, uint8_t* dst, hipStream_t stream);
 // dsum[r] = digit sum of the device row r (every byte of the device layout, padding included).
 int launch_digit_sums(const uint8_t* w, const Geometry& g, int32_t* dsum, hipStream_t stream);
@@ -313,9 +324,8 @@ struct vx_matrix {
     float weight_scale;
     int device;
     int num_cus;
-    uint32_t kslices, slice_chunks;  // K split of a lone GEMV on this matrix
+    vx::LonePlan lone;  // a lone GEMV on device activations
     uint8_t* d_w;       // weights, device layout (vx_layout)
-    int32_t* d_part;    // K-slice partial sums of a lone GEMV
     int32_t* d_accum;   // a lone GEMV's atomic K-slice sums (padded_rows), tickets (one per tile) and
     uint32_t* d_tickets;  // completion counter (d_done), zero between calls
     uint32_t* d_done;

@@ -443,3 +443,10 @@ def test_lone_gemv_slices(torch_dev, oracle, rows, cols):
         post = np.float32(0.5) / np.float32(3.0)
         assert np.array_equal(yf.cpu().numpy().view(np.uint32), (want.astype(np.float32) * post).view(np.uint32))
     layer.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(32768, 64), (32769, 64), (33000, 1003), (17000, 5121), (12289, 10241)])
+def test_lone_gemv_many_tiles(torch_dev, oracle, rows, cols):
+    """The same around the 512 workgroups (tiles times K slices, on 256 CUs) from which a lone GEMV takes 16 tiles per
+    workgroup: 512 and 513 tiles of one chunk, 516 of 13, and 266 and 193 tiles of rows in two and three slices."""
+    test_lone_gemv_slices(torch_dev, oracle, rows, cols)
