@@ -111,9 +111,10 @@ def test_prefill_variants(torch_dev, oracle, name):
 @pytest.mark.parametrize("name", ["pair_range", "gqa16"])
 @pytest.mark.parametrize("n", [7, 64, 128])
 def test_prefill_grouped_k_split(torch_dev, oracle, name, n):
-    """Prompts of up to 128 tokens at hidden 2560 (pair_range) and 512 (gqa16): their grouped q/k/v and gate/up GEMMs
-    take the small path with their K range split into 8 (2) slices, which the grouped finish kernel adds and
-    distributes to each matrix by its first row. KV cache and last logits equal the steps and the oracle."""
+    """Grouped q/k/v (three matrices) and gate/up GEMMs with their K range split, which the grouped finish kernel adds and
+    distributes to each matrix by its first row: 7 tokens take the small kernel, in 8 (pair_range, hidden 2560) or 2 (gqa16,
+    hidden 512) slices, 64 and 128 the tiled one, in 8 and 4 slices (pair_range; gqa16 in one). KV cache and last logits
+    equal the steps and the oracle."""
     model = oracle.Model(variant_cfg(oracle, name), 47 + n)
     pre = load_decoder(oracle, model)
     ref = load_decoder(oracle, model)
@@ -131,6 +132,24 @@ def test_prefill_grouped_k_split(torch_dev, oracle, name, n):
     finally:
         pre.close()
         ref.close()
+        model.close()
+
+
+def test_prefill_wide_pair(torch_dev, oracle):
+    """A 512-token pass whose gate and up (9220 rows each) run as one launch of the tiled kernel's largest tile (on 256 CUs):
+    KV cache and last logits equal the oracle."""
+    model = oracle.Model(variant_cfg(oracle, "falcon3"), 53)
+    pre = load_decoder(oracle, model)
+    try:
+        tokens = np.random.default_rng(5).integers(0, model.cfg.vocab, 512)
+        got, got_next = pre.prefill(tokens)
+        for pos, tok in enumerate(tokens):
+            o_next, o_logits = model.forward(int(tok), pos)
+        assert_same_bits(got, o_logits, "last logits vs oracle")
+        assert got_next == o_next
+        kv_equal(pre, model, model.cfg, range(0, 512, 3))
+    finally:
+        pre.close()
         model.close()
 
 

@@ -45,12 +45,12 @@ def gemm_noalloc(torch, layer, xd, m, y):
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("rows,cols,m", [(3072, 3072, 64), (23040, 3072, 256)])
+@pytest.mark.parametrize("rows,cols,m", [(3072, 3072, 64), (23040, 3072, 256), (3072, 3072, 20), (2000, 3001, 100)])
 def test_noalloc_captured_in_a_graph(torch_dev, oracle, rows, cols, m):
     """The entry point for callers under graph capture, captured (the first test of this file, so in a full run the
     call that looks the scratch up runs inside the capture) and replayed three times with new activations and eager
-    work in between; every replay equals vx_gemm_i32_dev on the same inputs bit for bit. Two shapes: the small-M path
-    (3072 x 3072, 64 tokens) and the staged path (23040 x 3072, 256 tokens)."""
+    work in between; every replay equals vx_gemm_i32_dev on the same inputs bit for bit. The tiled kernel on x itself, with
+    and without K slices, the small kernel (20 tokens), and the staging kernel before the tiled one (3001 columns)."""
     from quintrit_amd import VelurexHipLayer, _lib
     torch = torch_dev
     L = _lib.lib()
@@ -86,10 +86,11 @@ def test_noalloc_captured_in_a_graph(torch_dev, oracle, rows, cols, m):
         layer.close()
 
 
-@pytest.mark.parametrize("rows,cols,m1,m2", [(3072, 23040, 128, 8), (23040, 3072, 512, 33), (2560, 2560, 64, 3)])
+@pytest.mark.parametrize("rows,cols,m1,m2", [(3072, 23040, 128, 8), (23040, 3072, 512, 33), (2560, 2560, 64, 3),
+                                             (3072, 23041, 512, 40)])
 def test_noalloc_equals_workspace_gemm_twice(torch_dev, oracle, rows, cols, m1, m2):
     """Two calls in a row on one matrix, the second with fewer tokens, each against vx_gemm_i32_dev on the same
-    inputs; sampled rows also against the brute-force product."""
+    inputs; sampled rows also against the brute-force product. 23041 columns: staged fragments, then K-slice sums."""
     from quintrit_amd import VelurexHipLayer
     torch = torch_dev
     t = oracle.gen_trits(0x7A + rows + cols, (rows, cols))
