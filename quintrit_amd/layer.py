@@ -120,10 +120,14 @@ def compact_lut(acts_dev, cols: int, stream=None):
 
 def _stream_ptr(stream):
     """The HIP stream handle of a torch stream, or of the current device's current stream. (Building the stream object
-    that torch.cuda.current_stream returns took more of a small call than everything else on the host.)"""
+    that torch.cuda.current_stream returns took more of a small call than everything else on the host; a torch without
+    the raw getter pays for it.)"""
     if stream is None:
         import torch
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:
+            return raw(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
     return stream.cuda_stream
 
 

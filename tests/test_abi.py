@@ -156,3 +156,20 @@ def test_decoder_config_errors_before_device():
         assert field.split("_")[0] in L.vx_last_error_message().decode() or status == 2
     assert L.vx_decoder_free(None) == 0
     assert L.vx_decoder_step(None, 0, 0, None, 0, None) == 14
+
+
+def test_current_stream_without_the_raw_getter(monkeypatch):
+    """The layer calls take the current stream's handle from torch's raw getter where it has one, else from the stream."""
+    torch = pytest.importorskip("torch")
+    from quintrit_amd import layer
+
+    class Stream:
+        cuda_stream = 4321
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 1234, raising=False)
+    assert layer._stream_ptr(None) == 1234
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert layer._stream_ptr(None) == 4321
+    assert layer._stream_ptr(Stream) == 4321
