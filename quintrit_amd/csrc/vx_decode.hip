@@ -1103,9 +1103,9 @@ __device__ __forceinline__ void r16_all(float (&y)[N]) {
 // otherwise ms = 1, vs = expf(score - max); held as -ms or vs, the sign marks the case), then per coordinate, in
 // position order, y = f16(y ms), y = f16(fma(v, vs, y)), and s = fma(s, ms, vs).
 //
-// Work split: a workgroup takes one query head, one chunk and TOK tokens at consecutive positions from a multiple of
-// TOK on (they share the padded length, so the chunk's bounds), and walks the chunk in ranges of POS positions per wave.
-// In a range wave w first computes the scores and factors of its POS positions for all tokens, and then runs the
+// Work split: a workgroup takes one query head, one chunk and 16 tokens at consecutive positions from a multiple of 16 on
+// (they share the padded length, so the chunk's bounds), and walks the chunk in ranges of 16 positions per wave. In a
+// range wave w first computes the scores and factors of its positions for all tokens, and then runs the
 // accumulators of its own tokens over the whole range, a lane holding some coordinates of each: the V words of 8
 // positions are loaded once for all of them, the factors are read from LDS (one address per wave). TOK = 16 with 4
 // waves of 16 positions measured 10.6 ms of a 1500-token prompt (30 layers of 20 heads of 128; 32 tokens with 8 waves
@@ -1170,23 +1170,23 @@ __device__ __forceinline__ float expf_nonpos(float x, Tab tab) {
     return x < -0x1.9fe368p6f ? 0.0f : y;  // underflow (and -inf)
 }
 
-// TOK tokens (16 or 32) per workgroup of W waves, POS positions (16 or 32) per wave and range; SL workgroups share the
-// coordinates of a head, each computing the scores and factors for itself.
-template <int HD, int TOK, int POS, int W, int SL>
+// kPfTok tokens per workgroup of W waves, kPfPos positions per wave and range; SL workgroups share the coordinates of a
+// head, each computing the scores and factors for itself.
+constexpr uint32_t kPfTok = 16, kPfPos = 16;
+template <int HD, int W, int SL>
 __global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel(PfAttnArgs a) {
     constexpr uint32_t kCpl = HD >= 64 ? HD / (64u * SL) : 1u;  // coordinates per lane
-    constexpr uint32_t kOwn = TOK / W;                          // tokens per wave
-    constexpr uint32_t kTh = TOK / 16u, kPh = POS / 16u;        // 16-token and 16-position halves of a wave's scores
-    constexpr uint32_t kRange = W * POS;
+    constexpr uint32_t kOwn = kPfTok / W;                       // tokens per wave
+    constexpr uint32_t kRange = W * kPfPos;
     constexpr uint32_t kRing = SL > 1 || kCpl == 1u ? 8u : 4u;  // V groups of 8 positions in flight
     constexpr int kBlk = HD / 32;
     constexpr uint32_t kQRow = HD + 8u;                         // halves per token row in LDS
     static_assert(kRange % (8u * kRing) == 0 && (kOwn == 2u || kOwn == 4u), "whole rings in a range, 2 or 4 tokens per wave");
-    __shared__ __align__(16) float fac[TOK][kRange + 4u];       // (the rows start on different banks)
-    __shared__ __align__(16) uint16_t qs[TOK][kQRow];
-    __shared__ float wmax[W][TOK];
+    __shared__ __align__(16) float fac[kPfTok][kRange + 4u];    // (the rows start on different banks)
+    __shared__ __align__(16) uint16_t qs[kPfTok][kQRow];
+    __shared__ float wmax[W][kPfTok];
     // byte [g][t]: token t has a new maximum among the first (bit 0), the last (bit 1) 4 positions of group g
-    __shared__ __align__(4) uint8_t newmax[kRange / 8u][TOK];
+    __shared__ __align__(4) uint8_t newmax[kRange / 8u][kPfTok];
     __shared__ uint64_t etab[32];
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -1194,19 +1194,19 @@ __global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel
     const uint32_t h = blockIdx.x / SL, kvh = h / a.gqa, c = blockIdx.z;
     const uint32_t last = a.ctl->pos, first = last + 1u - a.n_tok;  // the pass' positions
     // later tokens first: they have the most positions
-    const uint32_t tp = (first / TOK + (gridDim.y - 1u - blockIdx.y)) * TOK;
+    const uint32_t tp = (first / kPfTok + (gridDim.y - 1u - blockIdx.y)) * kPfTok;
     if (tp > last) return;
     const KvSplit kv = kv_split(tp + 1u, a.max_ctx);
     if (c >= kv.n_chunks) return;
     const uint32_t st = c * kv.chunk;
-    const uint32_t t_last = min(tp + TOK - 1u, last);                        // the tile's last token
+    const uint32_t t_last = min(tp + kPfTok - 1u, last);                     // the tile's last token
     const uint32_t en_max = min(min(st + kv.chunk, kv.n_kv), t_last + 1u);   // positions of the longest one
     if (st >= en_max) return;
     const uint16_t* kb = a.kc + static_cast<size_t>(kvh) * a.max_ctx * HD;
     const uint16_t* vt = a.vc + static_cast<size_t>(kvh) * HD * a.vstride;
     const size_t qd = static_cast<size_t>(a.n_heads) * HD;
 
-    for (uint32_t i = tid; i < TOK * HD / 8u; i += 64u * W) {
+    for (uint32_t i = tid; i < kPfTok * HD / 8u; i += 64u * W) {
         const uint32_t t = i / (HD / 8u), d = i % (HD / 8u) * 8u;
         const uint32_t p = min(max(tp + t, first), last);  // a token outside the pass repeats one of it (never stored)
         *reinterpret_cast<uint4*>(&qs[t][d]) = *reinterpret_cast<const uint4*>(a.qbuf + (p - first) * qd + h * HD + d);
@@ -1215,16 +1215,10 @@ __global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel
     const auto tab = [&](uint32_t k) { return etab[k]; };
     __syncthreads();
 
-    // Scores: this lane's tokens (columns cl and cl + 16) and quarter (the positions 4 qt .. + 3 of each 16).
+    // Scores: this lane's token (column cl) and quarter (the positions 4 qt .. + 3 of the wave's 16).
     const uint32_t cl = lane & 15u, qt = lane >> 4;
-    uint32_t en[kTh];     // the tokens' positions [st, en)
-    float carry[kTh];     // their running maxima
-#pragma unroll
-    for (uint32_t th = 0; th < kTh; ++th) {
-        const uint32_t p = tp + 16u * th + cl;
-        en[th] = p >= first && p <= last ? min(en_max, p + 1u) : st;
-        carry[th] = -__builtin_inff();
-    }
+    const uint32_t en = tp + cl >= first && tp + cl <= last ? min(en_max, tp + cl + 1u) : st;  // its positions [st, en)
+    float carry = -__builtin_inff();                                                           // their running maximum
 
     // Accumulators: the wave's tokens t0 .., the lane's coordinates dl + 64 m of each.
     const uint32_t t0 = wave * kOwn;
@@ -1252,121 +1246,97 @@ __global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel
     };
 
     for (uint32_t sb = st / 32u * 32u; sb < en_max; sb += kRange) {
-        const uint32_t p0 = sb + POS * wave;  // this wave's positions
-        float sc[kTh][kPh][4];  // [16 tokens][16 positions][position 4 qt + e]
+        const uint32_t p0 = sb + kPfPos * wave;  // this wave's positions
+        float sc[4];                             // of positions 4 qt + e
         if (p0 < en_max) {
             // K rows: lane (position l % 16 of 16, j = l / 16) holds its coordinates 32 i + 8 j .. + 7 (a position past
             // the chunk repeats its last one; its factor is set to +0 below)
-            uint4 kr[kPh][kBlk];
+            uint4 kr[kBlk];
+            const uint16_t* row = kb + static_cast<size_t>(min(p0 + cl, en_max - 1u)) * HD + 8u * qt;
 #pragma unroll
-            for (uint32_t ph = 0; ph < kPh; ++ph) {
-                const uint16_t* row = kb + static_cast<size_t>(min(p0 + 16u * ph + cl, en_max - 1u)) * HD + 8u * qt;
-#pragma unroll
-                for (int i = 0; i < kBlk; ++i) kr[ph][i] = *reinterpret_cast<const uint4*>(row + 32 * i);
-            }
+            for (int i = 0; i < kBlk; ++i) kr[i] = *reinterpret_cast<const uint4*>(row + 32 * i);
             auto dw = [](const uint4& v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); };
+            float t01[4];
 #pragma unroll
-            for (uint32_t tile = 0; tile < kTh * kPh; ++tile) {
-                const uint32_t th = tile / kPh, ph = tile % kPh;
-                // k's conversions are made again for the second token half (kept, they would not fit the registers)
+            for (int dp = 0; dp < 2; ++dp) {          // chain lanes l = 2 dp, 2 dp + 1 and their partners l + 4
+                float tt[2][4];
 #pragma unroll
-                for (int i = 0; i < kBlk; ++i)
-                    asm volatile("" : "+v"(kr[ph][i].x), "+v"(kr[ph][i].y), "+v"(kr[ph][i].z), "+v"(kr[ph][i].w));
-                float t01[4];
+                for (int up = 0; up < 2; ++up) {      // l = 2 dp + lo + 4 up: half lo of dword dp + 2 up
+                    // read here and not earlier: q's values of one step only are held in registers
+                    uint32_t qo = cl * kQRow + 8u * qt + 2u * (dp + 2 * up);
+                    asm volatile("" : "+v"(qo));
+                    uint32_t qw[kBlk];
 #pragma unroll
-                for (int dp = 0; dp < 2; ++dp) {          // chain lanes l = 2 dp, 2 dp + 1 and their partners l + 4
-                    float tt[2][4];
+                    for (int i = 0; i < kBlk; ++i) qw[i] = *reinterpret_cast<const uint32_t*>(&qs[0][0] + qo + 32 * i);
 #pragma unroll
-                    for (int up = 0; up < 2; ++up) {      // l = 2 dp + lo + 4 up: half lo of dword dp + 2 up
-                        // read here and not earlier: q's values of one step only are held in registers
-                        uint32_t qo = (16u * th + cl) * kQRow + 8u * qt + 2u * (dp + 2 * up);
-                        asm volatile("" : "+v"(qo));
-                        uint32_t qw[kBlk];
+                    for (int lo = 0; lo < 2; ++lo) {
+                        v16f acc = {};
 #pragma unroll
-                        for (int i = 0; i < kBlk; ++i) qw[i] = *reinterpret_cast<const uint32_t*>(&qs[0][0] + qo + 32 * i);
+                        for (int i = 0; i < kBlk; ++i)
+                            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(
+                                f16_f32(static_cast<uint16_t>(dw(kr[i], dp + 2 * up) >> (16 * lo))),
+                                f16_f32(static_cast<uint16_t>(qw[i] >> (16 * lo))), acc, 0, 0, 0);
 #pragma unroll
-                        for (int lo = 0; lo < 2; ++lo) {
-                            v16f acc = {};
-#pragma unroll
-                            for (int i = 0; i < kBlk; ++i)
-                                acc = __builtin_amdgcn_mfma_f32_16x16x1f32(
-                                    f16_f32(static_cast<uint16_t>(dw(kr[ph][i], dp + 2 * up) >> (16 * lo))),
-                                    f16_f32(static_cast<uint16_t>(qw[i] >> (16 * lo))), acc, 0, 0, 0);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const float r = (acc[e] + acc[8 + e]) + (acc[4 + e] + acc[12 + e]);
-                                tt[lo][e] = up == 0 ? r : tt[lo][e] + r;
-                            }
-                            __builtin_amdgcn_sched_barrier(0);  // one chain lane at a time: their sums would not fit
+                        for (int e = 0; e < 4; ++e) {
+                            const float r = (acc[e] + acc[8 + e]) + (acc[4 + e] + acc[12 + e]);
+                            tt[lo][e] = up == 0 ? r : tt[lo][e] + r;
                         }
+                        __builtin_amdgcn_sched_barrier(0);  // one chain lane at a time: their sums would not fit
                     }
+                }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float s = tt[0][e] + tt[1][e];
-                        if (dp == 0) t01[e] = s;
-                        else sc[th][ph][e] = (t01[e] + s) * a.scale;
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    const float s = tt[0][e] + tt[1][e];
+                    if (dp == 0) t01[e] = s;
+                    else sc[e] = (t01[e] + s) * a.scale;
                 }
             }
         }
         // the maxima of every quarter's 4 positions, and the wave's
-        float qm[kTh][kPh][4];
+        float qm[4], tmax = -__builtin_inff();
+        {
+            float m = -__builtin_inff();
 #pragma unroll
-        for (uint32_t th = 0; th < kTh; ++th) {
-            float tmax = -__builtin_inff();
-#pragma unroll
-            for (uint32_t ph = 0; ph < kPh; ++ph) {
-                float m = -__builtin_inff();
-#pragma unroll
-                for (uint32_t e = 0; e < 4; ++e) {
-                    const uint32_t p = p0 + 16u * ph + 4u * qt + e;
-                    sc[th][ph][e] = p >= st && p < en[th] ? sc[th][ph][e] : -__builtin_inff();
-                    m = sc[th][ph][e] > m ? sc[th][ph][e] : m;
-                }
-                all_quarters(m, qm[th][ph]);
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) tmax = qm[th][ph][q] > tmax ? qm[th][ph][q] : tmax;
+            for (uint32_t e = 0; e < 4; ++e) {
+                const uint32_t p = p0 + 4u * qt + e;
+                sc[e] = p >= st && p < en ? sc[e] : -__builtin_inff();
+                m = sc[e] > m ? sc[e] : m;
             }
-            if (qt == 0) wmax[wave][16u * th + cl] = tmax;
+            all_quarters(m, qm);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) tmax = qm[q] > tmax ? qm[q] : tmax;
         }
+        if (qt == 0) wmax[wave][cl] = tmax;
         __syncthreads();  // every wave is also done with the previous range's factors
+        float prev = carry;
 #pragma unroll
-        for (uint32_t th = 0; th < kTh; ++th) {
-            float m = carry[th];
+        for (uint32_t w = 0; w < W; ++w) {
+            const float v = wmax[w][cl];
+            carry = v > carry ? v : carry;
+            if (w < wave) prev = v > prev ? v : prev;
+        }
+        if (p0 < en_max) {
 #pragma unroll
-            for (uint32_t w = 0; w < W; ++w) {
-                const float v = wmax[w][16u * th + cl];
-                carry[th] = v > carry[th] ? v : carry[th];
-                if (w < wave) m = v > m ? v : m;
+            for (uint32_t q = 0; q < 3; ++q) prev = q < qt && qm[q] > prev ? qm[q] : prev;
+            float f[4];
+            uint32_t sign = 0;
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                const uint32_t p = p0 + 4u * qt + e;
+                const float s = sc[e];
+                const bool up = s > prev;
+                const float x = expf_nonpos(up ? prev - s : s - prev, tab);
+                f[e] = p >= st && p < en ? (up ? -x : x) : 0.0f;
+                sign |= f32_bits(f[e]);
+                prev = up ? s : prev;
             }
-            if (p0 >= en_max) continue;
-#pragma unroll
-            for (uint32_t ph = 0; ph < kPh; ++ph) {
-                float prev = m;
-#pragma unroll
-                for (uint32_t q = 0; q < 3; ++q) prev = q < qt && qm[th][ph][q] > prev ? qm[th][ph][q] : prev;
-                float f[4];
-                uint32_t sign = 0;
-#pragma unroll
-                for (uint32_t e = 0; e < 4; ++e) {
-                    const uint32_t p = p0 + 16u * ph + 4u * qt + e;
-                    const float s = sc[th][ph][e];
-                    const bool up = s > prev;
-                    const float x = expf_nonpos(up ? prev - s : s - prev, tab);
-                    f[e] = p >= st && p < en[th] ? (up ? -x : x) : 0.0f;
-                    sign |= f32_bits(f[e]);
-                    prev = up ? s : prev;
-                }
-                const uint32_t o = POS * wave + 16u * ph + 4u * qt;
-                *reinterpret_cast<float4*>(&fac[16u * th + cl][o]) = make_float4(f[0], f[1], f[2], f[3]);
-                float sq[4];
-                all_quarters(bits_f32(sign), sq);
-                if ((qt & 1u) == 0u) {
-                    const uint32_t s0 = qt == 0 ? f32_bits(sq[0]) : f32_bits(sq[2]), s1 = qt == 0 ? f32_bits(sq[1]) : f32_bits(sq[3]);
-                    newmax[o / 8u][16u * th + cl] = static_cast<uint8_t>(s0 >> 31 | s1 >> 31 << 1);
-                }
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) m = qm[th][ph][q] > m ? qm[th][ph][q] : m;
+            const uint32_t o = kPfPos * wave + 4u * qt;
+            *reinterpret_cast<float4*>(&fac[cl][o]) = make_float4(f[0], f[1], f[2], f[3]);
+            float sq[4];
+            all_quarters(bits_f32(sign), sq);
+            if ((qt & 1u) == 0u) {
+                const uint32_t s0 = qt == 0 ? f32_bits(sq[0]) : f32_bits(sq[2]), s1 = qt == 0 ? f32_bits(sq[1]) : f32_bits(sq[3]);
+                newmax[o / 8u][cl] = static_cast<uint8_t>(s0 >> 31 | s1 >> 31 << 1);
             }
         }
         __syncthreads();
@@ -1498,11 +1468,8 @@ __global__ __launch_bounds__(64 * W, HD / SL >= 256 ? 3 : 4) void pf_attn_kernel
             if (lane == 0 && blockIdx.x % SL == 0) a.cms[2u * slot + 1u] = s;
         }
     }
-    if (kv.n_chunks > 1u && wave == 0 && blockIdx.x % SL == 0 && qt < kTh) {
-        const uint32_t e = kTh == 1u || qt == 0 ? en[0] : en[kTh - 1u];
-        if (e > st)
-            a.cms[2u * (((tp + lane - first) * static_cast<size_t>(a.n_heads) + h) * 4u + c)] = kTh == 1u || qt == 0 ? carry[0] : carry[kTh - 1u];
-    }
+    if (kv.n_chunks > 1u && wave == 0 && blockIdx.x % SL == 0 && qt == 0 && en > st)
+        a.cms[2u * (((tp + lane - first) * static_cast<size_t>(a.n_heads) + h) * 4u + c)] = carry;
 }
 
 // The chunks of every token with a split context, combined in order (attention.rs:526-541). A thread computes the
@@ -2953,7 +2920,7 @@ enum class PfForm : uint32_t { kTiny, kToken, kWhole, kSplit };
 
 // Workgroups of 16 tokens and all coordinates of a head.
 static uint32_t pf_attn_tiles(uint32_t n_heads, uint32_t n_tok, bool split) {
-    return n_heads * ((n_tok + 15u) / 16u) * (split ? 4u : 1u);
+    return n_heads * ((n_tok + kPfTok - 1u) / kPfTok) * (split ? 4u : 1u);
 }
 
 // The form of a pass of n_tok tokens that ends before position `end`. The split starts at a padded length of 512
@@ -2972,11 +2939,11 @@ static PfForm pf_form(const vx_decoder_config_t& c, uint32_t n_tok, uint32_t end
     return split ? PfForm::kSplit : PfForm::kWhole;
 }
 
-template <int HD, int TOK, int POS, int W, int SL>
+template <int HD, int W, int SL>
 static void launch_pf_attn_as(const PfAttnArgs& a, bool split, hipStream_t s) {
-    // one tile more than the tokens fill: they need not start at a multiple of TOK
-    const dim3 grid(a.n_heads * SL, (a.n_tok + TOK - 1u) / TOK + 1u, split ? 4u : 1u);
-    hipLaunchKernelGGL((pf_attn_kernel<HD, TOK, POS, W, SL>), grid, dim3(64 * W), 0, s, a);
+    // one tile more than the tokens fill: they need not start at a multiple of kPfTok
+    const dim3 grid(a.n_heads * SL, (a.n_tok + kPfTok - 1u) / kPfTok + 1u, split ? 4u : 1u);
+    hipLaunchKernelGGL((pf_attn_kernel<HD, W, SL>), grid, dim3(64 * W), 0, s, a);
 }
 
 // A workgroup takes 16 tokens and all coordinates of a head where that gives two workgroups per CU or more. Below that
@@ -2995,8 +2962,8 @@ static void launch_pf_attn(const PfAttnArgs& a, int num_cus, PfForm form, hipStr
         return;
     }
     const bool split = form == PfForm::kSplit;
-    if (pf_attn_tiles(a.n_heads, a.n_tok, split) < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 16, 16, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
-    else launch_pf_attn_as<HD, 16, 16, 4, 1>(a, split, s);
+    if (pf_attn_tiles(a.n_heads, a.n_tok, split) < 2u * static_cast<uint32_t>(num_cus)) launch_pf_attn_as<HD, 8, HD >= 64 ? HD / 64 : 1>(a, split, s);
+    else launch_pf_attn_as<HD, 4, 1>(a, split, s);
     if (split)
         hipLaunchKernelGGL(pf_attn_combine_kernel<HD>, dim3((a.n_heads * HD + 2047u) / 2048u, a.n_tok), dim3(256), 0, s, a);
 }

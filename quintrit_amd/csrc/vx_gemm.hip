@@ -113,12 +113,10 @@ __global__ __launch_bounds__(256) void gemm_stage_kernel(const int8_t* __restric
         for (int e = 0; e < 5; ++e) X[e] = *reinterpret_cast<const u32x4u*>(blk + 32 * e);
         block_fragments(X, o);
     } else {
-        // byte-column 16 hs + k of the step (k < 16), activation p: in a whole block 160 ks + 32 p + 16 hs + k, in the
-        // packed tail 160 ks + 5 (16 hs + k) + p (column_activation_index); past the row (and in the tail's padding
-        // columns, whose indices are all >= cols) zero
-        const bool tail = ks >= cols / 160u;
+        // the packed tail: byte-column 16 hs + k of the step (k < 16), activation p is 160 ks + 5 (16 hs + k) + p
+        // (column_activation_index); past the row (and in the tail's padding columns, whose indices are all >= cols) zero
         auto act = [&](uint32_t k, uint32_t p) -> uint32_t {
-            const uint32_t idx = tail ? ks * 160u + 5u * (16u * hs + k) + p : ks * 160u + 32u * p + 16u * hs + k;
+            const uint32_t idx = ks * 160u + 5u * (16u * hs + k) + p;
             return idx < cols ? static_cast<uint32_t>(static_cast<uint8_t>(xr[idx])) : 0u;
         };
 #pragma unroll
@@ -201,7 +199,6 @@ template <int T, int R, bool RAW>
 __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs a) {
     constexpr uint32_t kFrags = 5u * T;                 // B fragments of a K step
     constexpr uint32_t kXPer = RAW ? 5u : (kFrags + 3u) / 4u;  // 16-byte loads of activations per thread and step
-    constexpr uint32_t kXSets = 2u;  // sets of activations on the way to LDS
     constexpr int kReads = 4 * R + T, kEarly = (R * T + 1) / 2;  // the LDS reads of a K block follow its first products
     constexpr uint32_t kLdsRows = 2u * kFrags * 8u > 256u ? 2u * kFrags * 8u : 256u;
     __shared__ __align__(256) uint32_t tab[kLdsRows * 64u];
@@ -269,7 +266,7 @@ __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs 
         }
     }
     const uint32_t xstep = 5u * a.n_tg * 64u;
-    u32x4g X[kXSets][kXPer];
+    u32x4g X[2][kXPer];
     auto load_x = [&](uint32_t ks, u32x4g (&x)[kXPer]) __attribute__((always_inline)) {  // step min(ks, last), in order
         if constexpr (RAW) {
             const uint32_t k = min(ks, last), base = k * 160u + xhs * (k < full ? 16u : 80u), step = k < full ? 32u : 16u;
@@ -333,7 +330,7 @@ __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs 
     v4i A[2][R], A4[R], B[2][T];
     load_x(ks0, X[0]);
     load_w(ks0, w[0]);
-    if constexpr (kXSets > 1) load_x(ks0 + 1u, X[1 % kXSets]);
+    load_x(ks0 + 1u, X[1]);
     load_w(ks0 + 1u, w[1]);
     load_w(ks0 + 2u, w[2]);
     for (uint32_t i = tid; i < 256u * 8u; i += 256u) {
@@ -342,7 +339,7 @@ __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs 
     }
     store_x(0, X[0]);
     if (RAW && ks0 >= full) store_tail(ks0, 0, X[0]);
-    load_x(ks0 + kXSets, X[0]);
+    load_x(ks0 + 2u, X[0]);
     __syncthreads();
     decode(0, w[0], A[0]);
     read_b(0, 0, B[0]);
@@ -354,10 +351,10 @@ __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs 
         static_for<5>([&](auto kc) __attribute__((always_inline)) {
             constexpr uint32_t kb = decltype(kc)::value, cur = (s + kb) & 1u, nxt = cur ^ 1u;
             if constexpr (kb == 0) load_w(ks + 3u, w[(s + 3u) & 3u]);
-            if constexpr (kb == 2) store_x(buf ^ 1u, X[(s + 1u) % kXSets]);
+            if constexpr (kb == 2) store_x(buf ^ 1u, X[(s + 1u) & 1u]);
             if constexpr (kb == 3) {
-                if (RAW && ks + 1u >= full && ks + 1u < ks1) store_tail(ks + 1u, buf ^ 1u, X[(s + 1u) % kXSets]);
-                load_x(ks + 1u + kXSets, X[(s + 1u) % kXSets]);
+                if (RAW && ks + 1u >= full && ks + 1u < ks1) store_tail(ks + 1u, buf ^ 1u, X[(s + 1u) & 1u]);
+                load_x(ks + 3u, X[(s + 1u) & 1u]);
             }
             if constexpr (kb < 4) {
                 if constexpr (kb < 3) decode(kb + 1, w[s], A[nxt]);

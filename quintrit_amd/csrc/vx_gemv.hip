@@ -536,13 +536,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(8, 
 
 // Adds the K-slice partial sums of the split jobs and applies their epilogue. Block = 64 rows x 4 waves; wave w adds
 // the slices w, w + 4, ... of its 64 rows, then the 4 waves combine through LDS. blockIdx.y indexes `split` (the
-// plan's split jobs) or, without a job array, the one job.
-template <bool MANY>
+// plan's split jobs).
 __global__ __launch_bounds__(256) void finish_kernel(LaunchArgs args, const uint32_t* __restrict__ split) {
     __shared__ int red[4][64];
     Job jb;
-    if (MANY) __builtin_memcpy(&jb, (const Job*)((const c_job*)(args.jobs) + split[blockIdx.y]), sizeof(Job));
-    else jb = args.one;
+    __builtin_memcpy(&jb, (const Job*)((const c_job*)(args.jobs) + split[blockIdx.y]), sizeof(Job));
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t row0 = blockIdx.x * 64u;
     if (row0 >= jb.rows) return;
@@ -604,8 +602,9 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
     if (a.total_items == 0) return VX_OK;
     if (a.flag != nullptr && (a.jobs != nullptr || n_split != 0))
         VX_FAIL(VX_ERR_INTERNAL, "a completion flag on a launch whose outputs are not all written by gemv_kernel");
-    if (a.acts != nullptr && (a.jobs != nullptr || n_split != 0 || (a.one.kslices > 1 && a.one.accum == nullptr)))
-        VX_FAIL(VX_ERR_INTERNAL, "raw activations on a launch that is not a lone GEMV with atomic slice sums");
+    if (a.jobs == nullptr && (n_split != 0 || (a.one.kslices > 1 && a.one.accum == nullptr)))
+        VX_FAIL(VX_ERR_INTERNAL, "a lone GEMV without atomic slice sums");
+    if (a.acts != nullptr && a.jobs != nullptr) VX_FAIL(VX_ERR_INTERNAL, "raw activations on a launch of many jobs");
     const uint32_t grid = std::min<uint32_t>(a.total_items, 2u * static_cast<uint32_t>(num_cus));
     if (a.jobs) hipLaunchKernelGGL((gemv_kernel<true, false>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
     else if (a.acts) hipLaunchKernelGGL((gemv_kernel<false, true>), dim3(grid), dim3(kWaves * 64), 0, stream, a);
@@ -613,8 +612,7 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
     VX_HIP(hipGetLastError());
     if (n_split) {
         const dim3 fgrid((max_rows + 63u) / 64u, n_split);
-        if (a.jobs) hipLaunchKernelGGL(finish_kernel<true>, fgrid, dim3(256), 0, stream, a, split);
-        else hipLaunchKernelGGL(finish_kernel<false>, fgrid, dim3(256), 0, stream, a, split);
+        hipLaunchKernelGGL(finish_kernel, fgrid, dim3(256), 0, stream, a, split);
         VX_HIP(hipGetLastError());
     }
     return VX_OK;

@@ -457,10 +457,11 @@ int launch_q2(const Q2Args& a, int num_cus, hipStream_t stream) {
     if (a.sched != nullptr && (a.jobs == nullptr || a.sched_grid == 0 || a.sched_grid > a.total_items))
         VX_FAIL(VX_ERR_INTERNAL, "a Q2_0 schedule for %u workgroups over %u items", a.sched_grid, a.total_items);
     if (a.jobs == nullptr) {
-        // A lone GEMV: a workgroup per 32 rows while every one has a CU for itself (its 114 KiB of LDS
-        // admit one per CU, and before two rounds of prefetch 384 of them took 21.6 us against the items' 20.0 at 12288 x
-        // 4096, 12.1 against 6.5 at 12288 x 256; up to 256 they are the faster at every size measured, 64 x 256 4.65
-        // against 5.95 to 8192 x 12288 17.5 against 48.6); then items of kQ2LoneWaves / 2 tiles while they fit two workgroups per CU, else the plan's form.
+        // A lone GEMV: a workgroup per 32 rows while every one has a CU for itself (its 114 KiB of LDS admit one per CU;
+        // 384 of them, with one round of prefetch instead of two, took 21.6 us against the items' 20.0 at 12288 x 4096 and
+        // 12.1 against 6.5 at 12288 x 256; up to 256 they are the faster at every size measured, 64 x 256 4.65 against 5.95
+        // to 8192 x 12288 17.5 against 48.6); then items of kQ2LoneWaves / 2 tiles while they fit two workgroups per CU,
+        // else the plan's form.
         const uint32_t groups = (a.one.rows + 31u) / 32u, cus = static_cast<uint32_t>(num_cus);
         const uint32_t per = kQ2LoneWaves / 2u, items = (a.one.n_tiles + per - 1u) / per;
         if (groups <= cus) {
