@@ -451,8 +451,8 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(8, 
 // (gemv_kernel's hand-off). What bounds such a call is latency: with a wave per tile and K split over workgroups instead
 // (gemv_kernel), up to 13 slices of a tile group met in atomics and a ticket, about 2 us of a 6.6 us call, where this
 // form has none up to kLoneChunks chunks a row. Kernel time at 640 x 2560 7.0 -> 4.5 us and at 23040 x 3072 8.9 -> 7.3;
-// per call at 3072 x 23040 9.9 -> 8.4 and at 12000 x 8000 12.2 -> 10.9. More slices than that are not faster anywhere
-// (3072 x 3072: 1 to 8 slices the same, 23040 x 3072: 8.7 us with one, 11.7 with two).
+// per call at 3072 x 23040 9.9 -> 8.4 and at 12000 x 8000 12.2 -> 10.9. A row that fits one slice is no faster in
+// more (3072 x 3072: 1 to 8 slices the same, 23040 x 3072: 8.7 us with one, 11.7 with two).
 // The activations of a slice are staged by every workgroup (from acts, or copied from the staged vector), one byte-column
 // per thread, while its weights are in flight.
 template <bool RAW>
@@ -621,6 +621,8 @@ int launch_gemv(const LaunchArgs& a, uint32_t max_rows, const uint32_t* split, u
 LonePlan lone_plan(const Geometry& g, int num_cus) {
     const uint32_t nc = static_cast<uint32_t>(g.n_chunks), cus = static_cast<uint32_t>(num_cus);
     LonePlan p{true, (nc + kLoneChunks - 1u) / kLoneChunks, 0};
+    const uint32_t halves = (nc + kLoneChunks / 2u - 1u) / (kLoneChunks / 2u);
+    if (p.kslices > 1u && 4u * g.n_tiles * halves <= 3u * static_cast<size_t>(cus)) p.kslices = halves;
     p.tiled = g.n_tiles * p.kslices <= 2u * static_cast<size_t>(cus);
     if (!p.tiled) {
         const uint32_t groups = static_cast<uint32_t>(g.n_groups), least = (nc + kMaxSliceChunks - 1) / kMaxSliceChunks;

@@ -215,9 +215,12 @@ struct LoneArgs {
     uint32_t kslices, slice_chunks;
 };
 constexpr uint32_t kLoneChunks = 64;  // chunks of a K slice at most: 4 per wave
-// How a lone GEMV on activations in device memory runs. tiled: gemv_lone_kernel, a workgroup per tile and K slice (one
-// slice while a row has at most kLoneChunks chunks, else the fewest, of equal length), while all of its workgroups, two to
-// a CU, run at once (raw, 512 workgroups: 30000 x 3072 8.5 against 9.8 us, 8192 x 20000 11.8 against 11.9). Beyond that
+// How a lone GEMV on activations in device memory runs. tiled: gemv_lone_kernel, a workgroup per tile and K slice, while all
+// of its workgroups, two to a CU, run at once (raw, 512 workgroups: 30000 x 3072 8.5 against 9.8 us, 8192 x 20000 11.8
+// against 11.9): one slice while a row has at most kLoneChunks chunks, else the fewest, of equal length, or slices of half
+// that length while they leave a quarter of the CUs idle (half of kLoneChunks against all of it, raw: 64 x 9000 4.7
+// against 5.8 us, 1000 x 15000 (96 workgroups) 5.9 against 6.7, 3072 x 10240 (192) 6.1 against 7.2, 4096 x 10240 (256)
+// 6.9 against 6.8, 2000 x 23040 (288) 8.3 against 7.4). Beyond that
 // gemv_kernel, 16 tiles and a K slice per workgroup, in slices of 3 chunks at least, rounded down to at most one workgroup
 // per CU where they are short enough: 36000 x 2000 8.2 against 10.0, 20000 x 9000 12.8 against 15.6, 23040 x 23040 22.3
 // against 32.5. (Rounded up, a few CUs with two workgroups set the time: 23040 x 9000 16.9 -> 12.8.)

@@ -411,7 +411,7 @@ def test_plan_in_hip_graph_replays(torch_dev, oracle):
     layer.close()
 
 
-@pytest.mark.parametrize("cols", [80, 5120, 5121, 10241])  # one chunk, the longest single K slice, two and three slices
+@pytest.mark.parametrize("cols", [80, 5120, 5121, 10241])  # one chunk, the longest single K slice, 3 and 5 slices
 @pytest.mark.parametrize("rows", [1, 64, 65, 1090])        # partial and whole tiles, a second tile group
 def test_lone_gemv_slices(torch_dev, oracle, rows, cols):
     """Lone GEMVs on raw and on staged activations around the K-slice boundary, twice each (the atomic sums and tickets of
@@ -445,8 +445,9 @@ def test_lone_gemv_slices(torch_dev, oracle, rows, cols):
     layer.close()
 
 
-@pytest.mark.parametrize("rows,cols", [(32768, 64), (32769, 64), (33000, 1003), (17000, 5121), (12289, 10241)])
+@pytest.mark.parametrize("rows,cols", [(8192, 5121), (32768, 64), (32769, 64), (33000, 1003), (17000, 5121), (12289, 10241)])
 def test_lone_gemv_many_tiles(torch_dev, oracle, rows, cols):
-    """The same around the 512 workgroups (tiles times K slices, on 256 CUs) from which a lone GEMV takes 16 tiles per
-    workgroup: 512 and 513 tiles of one chunk, 516 of 13, and 266 and 193 tiles of rows in two and three slices."""
+    """The same with 128 tiles in two slices of more than half the longest, and around the 512 workgroups (tiles times K
+    slices, on 256 CUs) from which a lone GEMV takes 16 tiles per workgroup: 512 and 513 tiles of one chunk, 516 of 13, and
+    266 and 193 tiles of rows that would be in two and three slices."""
     test_lone_gemv_slices(torch_dev, oracle, rows, cols)
