@@ -1122,9 +1122,10 @@ __device__ __forceinline__ void r16_all(float (&y)[N]) {
 // 4 j + e, so the running maximum and the exponentials are computed in registers (the quarters of a wave exchange the
 // maxima of their 4 positions) and only the factors go to LDS.
 //
-// What bounds it: the vector unit (65 % busy), 1.5 instructions per coordinate and position for the accumulators (a
-// fused multiply-add and half a packed conversion; at head_dim 128 3.3 of the 6.6 per score and wave), the sums of the
-// chains and the exponentials.
+// What bounds it: the vector unit (counters: 57 to 68 % busy, the matrix cores 8 to 13 %), 1.5 instructions per coordinate
+// and position for the accumulators (a fused multiply-add and half a packed conversion; at head_dim 128 3.3 of the 6.6 per
+// score and wave), the sums of the chains and the exponentials. At head_dim 256 the form of whole heads spills 13 of its
+// 168 registers (three waves per SIMD); at 128 it takes exactly the 128 of four.
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 struct PfAttnArgs {

@@ -168,8 +168,10 @@ struct GemmArgs {
 // are requested three K steps ahead, the activations of step k + 3 during step k and written to LDS as fragments a step
 // before their use (two buffers, one barrier per step, placed where the last reads of the step have been issued). With
 // 8-wave workgroups that decoded a whole K step behind the barrier before its products, the matrix pipe idled through
-// every decode. 2560 x 2560 x 512 tokens 30.4 -> 15.9 us per call, 23040 x 3072 x 128 38 -> 23.4, 6913 x 2563 x 100 35.8
-// -> 21.3, 23040 x 3072 x 512 56.9 -> 45.9 (1.58 POP/s; a plain int8 library product of 8192^3 reaches 2.1 on this card).
+// every decode. 2560 x 2560 x 512 tokens 30.4 -> 15.9 us per call, 23040 x 3072 x 128 38 -> 23.7, 6913 x 2563 x 100 35.8 ->
+// 15.4 (staging launch included), 23040 x 3072 x 512 56.9 -> 45.1 (1.61 POP/s; a plain int8 library product of 8192^3
+// reaches 2.1 on this card). 3072 x 23040 x 512, whose 31 MB of slice sums are written and read back, gained nothing (65 to
+// 69 us before and after).
 //
 // What bounds it: instruction issue. A wave issues an instruction about every 7 cycles, matrix products included, and a
 // K step of one wave is 5 R T products of 32 cycles beside 16 R lookups with their addresses, 36 R byte operations for
@@ -181,8 +183,8 @@ struct GemmArgs {
 // four 4 x 4 byte transposes, in the packed tail of the row, whose byte-columns hold five consecutive activations, byte
 // shifts). Pieces past the row read its last one: the weights there are zero trits; a chunk past the row, whose weights
 // repeat the last chunk's, gets zeros. Its scattered loads cost about 0.1 us per step more than those of fragments that
-// gemm_stage_kernel or the caller has written (xs), the staging launch 5 to 8 us per call (3072 x 3072 x 64 17 against
-// 12 us, 23040 x 3072 x 128 25.5 against 23.4).
+// gemm_stage_kernel or the caller has written (xs); the staging launch costs 4 us where calls follow one another (3072 x
+// 3072 x 64 17 against 12 us per call, 23040 x 3072 x 128 25.5 against 23.4).
 //
 // LDS: the trit table (row B: 32 copies of byte B's entry in the first 128 bytes of a 256-byte row; lane l reads copy
 // l % 32, conflict-free because LDS serves a wave in two 32-lane halves), and in the second halves of its rows the two
@@ -724,9 +726,9 @@ struct GemmPlan {
 // The tile (T token groups, R blocks per wave) and the K slices of least estimated time, in us: 7 for the call and, per
 // K step, 0.4 + 0.095 T R for a workgroup alone on a CU (0.068 T R of it matrix work at 2.4 GHz; a wave issues an
 // instruction every 7 cycles or so, which keeps the rest from running beside it), 0.7 of that for each of several on
-// one CU, plus for more than one slice the finish kernel, 3.5 and its traffic. Over 19 shapes of 512 x 512 to 46080 x 3072
-// and 64 to 512 tokens, timed with every tile and 1 to 12 slices, the choice was 2.7 % slower than the best on average
-// (14 % at worst). Slice sums are kept within the scratch of the no-allocation entry point.
+// one CU, plus for more than one slice the finish kernel, 3.5 and its traffic. Over 337 products of 64 x 4096 to 46080 x
+// 3072 and 33 to 1500 tokens, each timed with every tile and up to 19 numbers of slices, the choice was 1.8 % slower than
+// the best on average, more than 10 % in 12 of them. Slice sums are kept within the scratch of the no-allocation entry point.
 static GemmPlan gemm_plan(const Geometry& g, size_t M, int num_cus) {
     const uint32_t n_ksteps = static_cast<uint32_t>(gemm_ksteps(g.cols));
     const uint32_t n_tg = token_groups(M);
@@ -886,8 +888,8 @@ int launch_gemm(const uint8_t* w, const Geometry& g, int num_cus, const int8_t* 
 // are first loaded on that GPU and held until the process ends. Host code never passes `scratch` itself (in host code
 // the name is only a stand-in for the symbol); it passes the device address hipGetSymbolAddress returns for the
 // current device, looked up once per device. Every call on a GPU reuses that GPU's array, so calls that overlap on one
-// GPU race; the kernels write every word they later read (staged activations, plane-4 parts, K-slice partials), so
-// no clearing is needed between calls.
+// GPU race. The kernels write every word of the K-slice sums that they later read; stale fragments of tokens past M are
+// read too, but reach only outputs that are never stored. So no clearing is needed between calls.
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxScratchDevices = 64;
