@@ -1,7 +1,7 @@
 /*
  * decode_oracle.c - CPU restatement of the reference's decode step (TEST INFRASTRUCTURE ONLY).
  *
- * The token loop of BASELINE.json configs[3] (a BitNet-b1.58-2B-shaped model with random weights): RMSNorm, per-token
+ * The token loop (a BitNet-b1.58-2B-shaped model with random weights): RMSNorm, per-token
  * int8 quantization, ternary projections with the layer epilogue, NEOX RoPE, an F16 KV cache, the FP16-accumulator
  * flash attention of bitnet.cpp with its 4-chunk split, sub-norms, ReLU^2, a tied bf16 head and greedy argmax; and the
  * Falcon3 variant of the same loop (Normal RoPE, no sub-norms, SwiGLU with ggml's vector expf, an f16 embedding and

@@ -33,7 +33,7 @@ extern "C" {
 typedef struct vxo_model_config {
     uint32_t n_layers, hidden, n_heads, n_kv_heads, head_dim, ffn, vocab, max_ctx;
     float rms_eps, rope_theta;
-    /* The architecture switches of ModelConfig (config.rs:155-227); all zero is BASELINE.json configs[3]'s BitNet. */
+    /* The architecture switches of ModelConfig (config.rs:155-227); all zero is BitNet-2B's. */
     uint32_t act;       /* VXO_ACT_RELU2: relu2(gate) * up; VXO_ACT_SILU: swiglu(gate, up) (model.rs:155-170) */
     uint32_t rope_mode; /* VXO_ROPE_NEOX or VXO_ROPE_NORMAL (ops.rs:199-221) */
     uint32_t no_sub_norm; /* 1: no attention / FFN sub-norms (has_sub_norm = false, model.rs:172-190) */
@@ -63,7 +63,7 @@ void vxo_attend_head(const uint16_t* q_f16, const uint16_t* kbase, const uint16_
                      size_t head_dim, size_t seq_len, size_t max_ctx, float scale, float* out); /* attention.rs:436-542 */
 void vxo_projection(const uint8_t* planar, size_t rows, size_t cols, float ws, const int8_t* q, float as, float* out);
 
-/* The model of BASELINE.json configs[3] with weights generated from `seed` (projections: kind 0..6 = q, k, v, o, gate,
+/* The BitNet-2B-shaped model with weights generated from `seed` (projections: kind 0..6 = q, k, v, o, gate,
  * up, down; norms: kind 0..3 = attn, attn_sub, ffn, ffn_sub, layer n_layers kind 0 = output norm). */
 void vxo_projection_shape(const vxo_model_config* c, int kind, size_t* rows, size_t* cols);
 vxo_model* vxo_model_create(const vxo_model_config* cfg, uint64_t seed);

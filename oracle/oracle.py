@@ -326,8 +326,8 @@ ROPE_NEOX, ROPE_NORMAL = 0, 1
 
 
 class ModelConfig(ctypes.Structure):
-    """vxo_model_config: the decoder shape and its architecture switches (all zero: the BitNet of BASELINE.json
-    configs[3], bitnet_2b(); falcon3() sets SiLU, Normal RoPE, no sub-norms, an f16 embedding and an untied f16 head)."""
+    """vxo_model_config: the decoder shape and its architecture switches (all zero: the BitNet of
+    bitnet_2b(); falcon3() sets SiLU, Normal RoPE, no sub-norms, an f16 embedding and an untied f16 head)."""
     _fields_ = [("n_layers", ctypes.c_uint32), ("hidden", ctypes.c_uint32), ("n_heads", ctypes.c_uint32),
                 ("n_kv_heads", ctypes.c_uint32), ("head_dim", ctypes.c_uint32), ("ffn", ctypes.c_uint32),
                 ("vocab", ctypes.c_uint32), ("max_ctx", ctypes.c_uint32), ("rms_eps", ctypes.c_float),
@@ -353,7 +353,7 @@ def falcon3(n_layers, hidden, n_heads, n_kv_heads, head_dim, ffn, vocab, max_ctx
 
 
 def falcon3_10b(max_ctx: int = 4096, n_layers: int = 40) -> ModelConfig:
-    """BASELINE.json configs[1]'s Falcon3-10B shapes (40 layers, hidden 3072, 12 / 4 heads of 256, FFN 23040) with the
+    """The Falcon3-10B shapes (40 layers, hidden 3072, 12 / 4 heads of 256, FFN 23040) with the
     Falcon3 vocabulary (131072) and the other constants of falcon3_7b_default (config.rs:205-227)."""
     return falcon3(n_layers, 3072, 12, 4, 256, 23040, 131072, max_ctx)
 

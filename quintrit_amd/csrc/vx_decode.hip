@@ -1,4 +1,4 @@
-// Decode step of a ternary decoder on gfx950: the token loop around the velurex GEMV (BASELINE.json configs[3]).
+// Decode step of a ternary decoder on gfx950: the token loop around the velurex GEMV.
 //
 // One step follows the reference's CPU runtime operation by operation (quintrit-runtime/src/model.rs:64-377,
 // attention.rs:115-542, ops.rs), so that logits and greedy tokens are bit-identical to it:

@@ -68,7 +68,7 @@ class DecoderConfig:
 
     @classmethod
     def falcon3_10b(cls, max_ctx: int = 4096, n_layers: int = 40) -> "DecoderConfig":
-        """BASELINE.json configs[1]'s Falcon3-10B shapes (40 layers, hidden 3072, 12 / 4 heads of 256, FFN 23040,
+        """The Falcon3-10B shapes (40 layers, hidden 3072, 12 / 4 heads of 256, FFN 23040,
         vocabulary 131072) with the constants of falcon3_7b_default (config.rs:205-227)."""
         return cls.falcon3(n_layers, 3072, 12, 4, 256, 23040, 131072, max_ctx)
 

@@ -1,4 +1,4 @@
-"""GPU parity of the decode token loop (and the Falcon3 architecture of configs[1]) through
+"""GPU parity of the decode token loop (BitNet-2B shapes, and the Falcon3 architecture) through
 the C ABI (vx_decoder_*).
 
 The reference's loop (QuintritModel::forward_token_with_scratchpad, quintrit-runtime/src/model.rs:282-377, with
@@ -350,7 +350,7 @@ def test_decoder_argument_errors(torch_dev, oracle):
 
 
 def test_bitnet2b_greedy_golden(torch_dev, oracle):
-    """64 prompt tokens, 256 greedy tokens identical to the CPU reference's."""
+    """BitNet-2B shapes: 64 prompt tokens, 256 greedy tokens identical to the CPU reference's."""
     with open(os.path.join(HERE, "golden", "bitnet2b_greedy.json")) as f:
         gold = json.load(f)
     model = oracle.Model(oracle.bitnet_2b(gold["max_ctx"]), gold["seed"])
@@ -378,7 +378,7 @@ def test_bitnet2b_greedy_golden(torch_dev, oracle):
 
 
 def test_falcon3_10b_golden_logits_every_position(torch_dev, oracle):
-    """A random-init Falcon3-10B-shaped model (BASELINE.json configs[1] shapes, Falcon3 architecture) against the
+    """A random-init Falcon3-10B-shaped model (40 layers of hidden 3072, Falcon3 architecture) against the
     committed oracle run (tests/golden/falcon3_10b_greedy.json, written by tests/golden/make_falcon3_golden.py): at each
     of the 319 positions the sum of the bit patterns of all 131072 logits equals the oracle's (teacher forced with the
     oracle's tokens), and greedy generation reproduces its 256 tokens."""

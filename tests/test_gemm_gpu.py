@@ -2,7 +2,7 @@
 
 The reference has no multi-token kernel; its prefill calls the GEMV once per token (quintrit-runtime/src/engine.rs:
 625-631), so the GEMM must equal M independent GEMVs bit for bit. Small shapes are checked against brute force; the
-BASELINE.json configs[2] shapes (W 23040 x 3072 and 3072 x 23040, M in {8, 32, 128, 512}) against a float64 brute
+Falcon3-10B FFN shapes (W 23040 x 3072 and 3072 x 23040, M in {8, 32, 128, 512}) against a float64 brute
 force of every output.
 """
 import ctypes
@@ -75,7 +75,7 @@ def test_gemm_extreme_values(torch_dev, oracle):
 
 @pytest.mark.parametrize("rows,cols", [(23040, 3072), (3072, 23040)])
 def test_gemm_config2_equals_bruteforce(torch_dev, oracle, rows, cols):
-    """i.i.d. trits (P(-1)=P(+1)=0.35), X quantized per token from N(0,1). Every output of
+    """The Falcon3-10B FFN shapes: i.i.d. trits (P(-1)=P(+1)=0.35), X quantized per token from N(0,1). Every output of
     every M is compared with a float64 BLAS product of the unpacked trits, which is exact here: the operands are
     integers and every partial sum is at most 128 * 23040 < 2^53 in magnitude."""
     from quintrit_amd import VelurexHipLayer

@@ -2,7 +2,7 @@
 
 The integer results must be bit-exact; the fp32 epilogue must equal the oracle's bit for bit (it is one fp32 division
 and one fp32 multiplication per row, layer.rs:246-253). Shapes and patterns follow the reference's GPU tests
-(quintrit-cuda/tests/gemv.rs:46-64,77-125) and BASELINE.json configs 0-2.
+(quintrit-cuda/tests/gemv.rs:46-64,77-125) and the benchmark's shapes.
 """
 import ctypes
 
@@ -81,7 +81,7 @@ def test_awkward_and_model_shapes(torch_dev, oracle, rows, cols):
 
 
 def test_config0_exact_and_epilogue(torch_dev, oracle):
-    """BASELINE.json config 0: W 2560x2560, P(-1)=P(+1)=0.35, x uniform in [-127, 127], y = float(acc) * 0.02."""
+    """W 2560x2560, P(-1)=P(+1)=0.35, x uniform in [-127, 127], y = float(acc) * 0.02."""
     from quintrit_amd import VelurexHipLayer
     t = oracle.gen_trits(0xC0FFEE, (2560, 2560))
     a = oracle.gen_i8(0xBEEF, 2560, -127, 127)

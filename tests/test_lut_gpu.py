@@ -106,7 +106,7 @@ def test_shapes_repeat_and_match_the_digit_gemv(torch_dev, oracle, rows, cols):
 
 
 def test_config0_exact(torch_dev, oracle):
-    """BASELINE.json config 0 through the tables: W 2560x2560, P(-1)=P(+1)=0.35, x uniform in [-127, 127]."""
+    """The tables at W 2560x2560, P(-1)=P(+1)=0.35, x uniform in [-127, 127]."""
     from quintrit_amd import VelurexHipLayer
     torch = torch_dev
     t = oracle.gen_trits(0xC0FFEE, (2560, 2560))

@@ -1,4 +1,4 @@
-"""GPU parity of the block-scaled (Q2_0 x Q8_0) GEMV through the C ABI (BASELINE.json configs[4]).
+"""GPU parity of the block-scaled (Q2_0 x Q8_0) GEMV through the C ABI.
 
 The reference's definition is dot_row_scalar (quintrit-core/src/block_scaled.rs:175-202), restated by the oracle
 (vxo_q2_0_dot_row). The GPU keeps its fp32 order, so outputs are compared bit for bit; the config's own bounds (int32
@@ -88,7 +88,7 @@ def test_q2_lone_rounds(torch_dev, oracle, rows, cols):
 
 
 def test_q2_config4_shapes_and_plan(torch_dev, oracle):
-    """The Qwen3-8B-like projections of configs[4] (hidden 4096, FFN 12288, q/o 4096x4096, k/v 1024x4096), one plan."""
+    """The Qwen3-8B-like projections (hidden 4096, FFN 12288, q/o 4096x4096, k/v 1024x4096), one plan."""
     from quintrit_amd import _lib
     torch = torch_dev
     rng = np.random.default_rng(4)
