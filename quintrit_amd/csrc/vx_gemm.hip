@@ -196,7 +196,9 @@ struct GemmArgs {
 // groups there are. (With whole row groups per XCD, row group mod 8, most of the card idled below 8 of them and parts of
 // it at 9 to 15: 300 x 23040 x 512 36.1 -> 20.2 us, 3072 x 23040 x 64 26.4 -> 21.1, 40 x 3072 x 512 20.6 -> 9.8.) Row
 // groups in whole eights keep that assignment within the list: neighbouring row groups on one XCD instead took 14.5 us
-// against 11.8 at 8192 x 3072 x 33.
+// against 11.8 at 8192 x 3072 x 33 in calls repeated with one workspace. (Only there: 8192 x 3072 x 64 takes 15.6 us with
+// one workspace, 12.9 with another for each call, in either order, and the L2 misses are alike. Probably this kernel's
+// stores wait for lines that the finish kernel of the call before read on another XCD; not observed directly.)
 template <int T, int R, bool RAW>
 __global__ __launch_bounds__(256, T * R >= 8 ? 1 : 2) void gemm_kernel(GemmArgs a) {
     constexpr uint32_t kFrags = 5u * T;                 // B fragments of a K step
